@@ -179,7 +179,14 @@ int srt_create(int device, size_t hbm_budget_bytes, srt_ctx** out) {
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return SRT_E_HIP; }
     if (dev_alloc(c, c->counters, kCountersBytes)) { (void)hipStreamDestroy(c->stream); delete c; return SRT_E_OOM; }
     (void)hipMemset(c->counters.p, 0, kCountersBytes);
+    if (hipHostMalloc((void**)&c->live, 64, hipHostMallocDefault) != hipSuccess) {
+        dev_free(c, c->counters);
+        (void)hipStreamDestroy(c->stream);
+        delete c;
+        return SRT_E_OOM;
+    }
     if (int r = noalloc_init(c)) {
+        (void)hipHostFree(c->live);
         dev_free(c, c->counters);
         (void)hipStreamDestroy(c->stream);
         delete c;
@@ -208,6 +215,7 @@ void srt_destroy(srt_ctx* c) {
     dev_free(c, c->scan_tmp); dev_free(c, c->train_in9); dev_free(c, c->train_t); dev_free(c, c->segbuf);
     release_build_scratch(c);
     for (auto e : c->event_pool) (void)hipEventDestroy(e);
+    (void)hipHostFree(c->live);
     (void)hipStreamDestroy(c->stream);
     delete c;
 }

@@ -220,7 +220,8 @@ enum {
     CNT_FETCH_Q = CNT_FETCH_S + kParts * kCntLine,     // kParts lines: next standalone ray query
     CNT_MLPQ_PARTS = CNT_FETCH_Q + kParts * kCntLine,  // kParts lines: MLP query appends per partition
     CNT_MLPQ = CNT_MLPQ_PARTS + kParts * kCntLine,     // one line: MLP queries after compaction (dense)
-    CNT_WORDS = CNT_MLPQ + kCntLine
+    CNT_PATHS = CNT_MLPQ + kCntLine,                   // kParts lines: k_paths' segments and shadow rays (two 64-bit words)
+    CNT_WORDS = CNT_PATHS + kParts * kCntLine
 };
 // statistics (unsigned 64-bit) after the counters, then the end of the buffer
 constexpr size_t kTotalsOffset = (size_t)CNT_WORDS * 4;
@@ -321,6 +322,7 @@ struct srt_ctx {
     size_t gstack_entries = 0;            // int32 entries allocated in gstack
     int32_t trace_lds_depth = 16, trace_refill = 40, shadow_refill = 32, trace_blocks_per_cu = 0;   // 0: occupancy limit
     int32_t trace_bvh_width = 4;          // traversal over the 4-wide (4) or binary (2) tree
+    uint32_t* live = nullptr;             // pinned host word: live paths of the next bounce (report_live)
     int32_t trace_inner_exit = 18;        // stragglers resume after the leaf step
     int32_t trace_packet = 0;             // > 0: camera rays traversed as 64-ray packets (0: per ray)
     int64_t max_wide_nodes = srt::kMaxNodes4;   // 4-wide trees above this many nodes are traversed in binary form

@@ -469,6 +469,11 @@ SRT_D bool trav_leaf(const DevScene& S, TravState& st, uint32_t& nt) {
     return false;
 }
 
+// As trav_pend with the kind of ray known per lane (any: the first hit ends
+// the traversal, as trav_leaf<true>).
+template <bool INST>
+SRT_D bool trav_pend_any(const DevScene& S, TravState& st, const TravStack& k, bool any);
+
 // The postponed item of a lane: a triangle leaf (trav_leaf), or, in an
 // instanced scene, an instance to enter: the lane's current world-space
 // entry (if any) and kInstReturn are pushed, and the ray continues at the
@@ -491,6 +496,19 @@ SRT_D bool trav_pend(const DevScene& S, TravState& st, const TravStack& k, uint3
         return false;
     }
     return trav_leaf<ANY, COUNT, INST>(S, st, nt);
+}
+
+template <bool INST>
+SRT_D bool trav_pend_any(const DevScene& S, TravState& st, const TravStack& k, bool any) {
+    uint32_t nt = 0;
+    if (INST && is_inst_ref(st.pend)) return trav_pend<false, false, INST>(S, st, k, nt);
+    (void)trav_leaf<false, false, INST>(S, st, nt);
+    // a shadow ray's triangle hit in [tmin, tmax]: best_pos tells
+    if (any && st.best_pos >= 0) {
+        st.cur_ok = false;
+        return true;
+    }
+    return false;
 }
 
 // Persistent traversal with dynamic ray fetch.  Each lane holds one ray; when
@@ -839,6 +857,8 @@ SRT_D PathStart path_start(const Segment* segs, int nseg, uint32_t slot) {
 // slots [p cap, p cap + size)); clears the traversal fetch counters.
 __global__ void k_path_counts(uint32_t n, uint32_t cap, uint32_t* counts) {
     clear_parts(counts + CNT_FETCH_T);
+    clear_parts(counts + CNT_MLPQ_PARTS);
+    if (threadIdx.x < 4u * kParts) counts[CNT_PATHS + (threadIdx.x >> 2) * kCntLine + (threadIdx.x & 3u)] = 0u;
     if (threadIdx.x < (unsigned)kParts) counts[CNT_Q0 + threadIdx.x * kCntLine] = part_size(n, cap, threadIdx.x);
 }
 
@@ -1111,30 +1131,22 @@ SRT_D MatRec load_mat(const MatRec* mats, int32_t id) {
     return m;
 }
 
-// CAM: the first bounce, whose entries are the slots and whose path state is
-// path_start's; it also sets the path's radiance (no earlier stage does).
-template <bool CAM>
-SRT_D void shade_hit(const DevScene& S, const Segment* segs, int nseg, int depth, const PathQueue& qin, const HitBuf& h,
-                     const PathQueue& qout, const ShadowQueue& sq, float* Lr, float* Lg, float* Lb, uint32_t* counts,
-                     int qi, uint32_t part, uint32_t cap, const MlpIO& mio, uint32_t i) {
-    PathStart ps{};
-    if constexpr (CAM) ps = path_start(segs, nseg, i);
-    const uint32_t slot = CAM ? i : qin.slot[i];
-    const f3 rd = CAM ? ps.d : mk(qin.dx[i], qin.dy[i], qin.dz[i]);
-    f3 beta = CAM ? mk(1.0f) : mk(qin.br[i], qin.bg[i], qin.bb[i]);
-    if constexpr (CAM) {
-        Lr[slot] = 0.0f; Lg[slot] = 0.0f; Lb[slot] = 0.0f;
-    }
-    const int32_t tri = h.tri[i];
-    const uint32_t flags = CAM ? ps.flags : qin.flags[i];
-    const bool specular = (flags & 1u) != 0u;
-    const uint32_t segk = flags >> 8;
-    const SegHead P = load_seg_head(segs, segk);
-    const float u = h.u[i], v = h.v[i];
+// Shading of one hit, shared by the queue stage (k_shade) and the whole-path
+// kernel (k_paths).  Sink supplies what differs between them:
+//   f3 origin(), float scatter_pdf()   the ray's origin and the scatter pdf of the
+//                                      previous bounce (read only where an emitter is hit)
+//   void radiance(f3)                  adds to the path's radiance
+//   void shadow(emit, pos, dir, tmax, contribution)   the light sample's shadow ray
+//   void next(alive, pos, dir, beta, pdf, flags, rng) the path's continuation
+// shadow and next are reached by every lane that gets that far (emit / alive
+// say whether it has one); a path whose next is not reached ends here.
+template <class Sink>
+SRT_D void shade_path(const DevScene& S, const SegHead& P, uint32_t segk, int depth, uint32_t slot, f3 rd, f3 beta,
+                      bool specular, uint64_t rng_state, int32_t tri, float u, float v, int32_t inst, uint32_t* counts,
+                      uint32_t part, uint32_t cap, const MlpIO& mio, Sink& sink) {
     HitGeom hg = hit_geometry(S, tri, u, v);
     float4 X[3];               // instance transform (instanced scenes)
-    if (S.num_inst > 0) inst_hit(S, h.inst[i], hg, X);
-    const float w = hg.w;
+    if (S.num_inst > 0) inst_hit(S, inst, hg, X);
     const f3 pos = hg.pos, sn = hg.sn;
     f3 normal = hg.normal;
     const MatRec m = load_mat(S.mats, hg.matid);
@@ -1147,16 +1159,15 @@ SRT_D void shade_hit(const DevScene& S, const Segment* segs, int nseg, int depth
             if (P.use_nee && !specular) {
                 mis = 0.0f;
                 if (P.use_mis) {
-                    const f3 ro = CAM ? ps.o : mk(qin.ox[i], qin.oy[i], qin.oz[i]);
+                    const f3 ro = sink.origin();
                     const float t2 = dot(pos - ro, pos - ro);
                     const float lpdf = (m.intensity / S.light_wsum) * t2 / cos_i;
-                    const float scatter_pdf = CAM ? 1.0f : qin.pdf[i];
+                    const float scatter_pdf = sink.scatter_pdf();
                     mis = scatter_pdf / (lpdf + scatter_pdf);
                 }
             }
             const f3 Le = mk(m.emission_color[0], m.emission_color[1], m.emission_color[2]) * m.intensity;
-            const f3 add = beta * Le * mis;
-            add_rgb(Lr, Lg, Lb, slot, add.x, add.y, add.z);
+            sink.radiance(beta * Le * mis);
         }
         return;
     }
@@ -1168,9 +1179,9 @@ SRT_D void shade_hit(const DevScene& S, const Segment* segs, int nseg, int depth
     const bool last = (depth + 1 >= P.max_depth);
     const int64_t pid = P.path_begin + (int64_t)(slot - (uint32_t)P.slot_offset);
     const uint32_t sample = path_sample(pid, P.wh);
-    Pcg32 rng = rng_resume(CAM ? ps.rng : qin.rng[i], sample);
-    // next-event estimation (path_tracer.cu:113-142); the shadow ray and its
-    // would-be contribution go to the shadow queue
+    Pcg32 rng = rng_resume(rng_state, sample);
+    // next-event estimation (path_tracer.cu:113-142); the shadow ray carries
+    // its would-be contribution
     if (P.use_nee && !mat_is_specular(m)) {
         f2 lr;
         lr.x = rng.next_float();
@@ -1192,15 +1203,7 @@ SRT_D void shade_hit(const DevScene& S, const Segment* segs, int nseg, int depth
             const f3 f = sp_eval(m, spt, sdir, color);
             s_c = beta * f * fabsf(cos_o) * ls.emission * mis / lpdf;
         }
-        const int ja = wave_append(emit, counts + CNT_SHADOW + part * kCntLine);
-        if (ja >= 0) {
-            const uint32_t js = part * cap + (uint32_t)ja;
-            sq.ox[js] = pos.x; sq.oy[js] = pos.y; sq.oz[js] = pos.z;
-            sq.dx[js] = sdir.x; sq.dy[js] = sdir.y; sq.dz[js] = sdir.z;
-            sq.tmax[js] = t - 1e-3f;
-            sq.cr[js] = s_c.x; sq.cg[js] = s_c.y; sq.cb[js] = s_c.z;
-            sq.slot[js] = slot;
-        }
+        sink.shadow(emit, pos, sdir, t - 1e-3f, s_c);
     }
     if (P.mlp_mode != 0 && depth == 1 && !last) {
         // radiance-MLP hooks at vertex 2; features: position in the scene
@@ -1248,17 +1251,67 @@ SRT_D void shade_hit(const DevScene& S, const Segment* segs, int nseg, int depth
             else beta = beta / q;
         }
     }
-    const int ja = wave_append(alive, counts + cnt_q(qi ^ 1) + part * kCntLine);
-    if (ja >= 0) {
+    sink.next(alive, pos, ms.wi, beta, ms.pdf, (mat_is_specular(m) ? 1u : 0u) | (segk << 8), rng.state);
+}
+
+// k_shade's side of shade_path: queue entry i in, appends to the workgroup's
+// partition out (one atomic per wave, over the lanes active at the call).
+// CAM: the first bounce, whose entries are the slots and whose path state is
+// path_start's; it also sets the path's radiance (no earlier stage does).
+template <bool CAM>
+struct QueueSink {
+    const PathQueue &qin, &qout;
+    const ShadowQueue& sq;
+    float *Lr, *Lg, *Lb;
+    uint32_t* counts;
+    int qi;
+    uint32_t part, cap, i, slot;
+    f3 cam_o;
+    SRT_D f3 origin() const { return CAM ? cam_o : mk(qin.ox[i], qin.oy[i], qin.oz[i]); }
+    SRT_D float scatter_pdf() const { return CAM ? 1.0f : qin.pdf[i]; }
+    SRT_D void radiance(f3 c) const { add_rgb(Lr, Lg, Lb, slot, c.x, c.y, c.z); }
+    SRT_D void shadow(bool emit, f3 pos, f3 dir, float tmax, f3 c) const {
+        const int ja = wave_append(emit, counts + CNT_SHADOW + part * kCntLine);
+        if (ja < 0) return;
+        const uint32_t js = part * cap + (uint32_t)ja;
+        sq.ox[js] = pos.x; sq.oy[js] = pos.y; sq.oz[js] = pos.z;
+        sq.dx[js] = dir.x; sq.dy[js] = dir.y; sq.dz[js] = dir.z;
+        sq.tmax[js] = tmax;
+        sq.cr[js] = c.x; sq.cg[js] = c.y; sq.cb[js] = c.z;
+        sq.slot[js] = slot;
+    }
+    SRT_D void next(bool alive, f3 pos, f3 dir, f3 beta, float pdf, uint32_t flags, uint64_t rng) const {
+        const int ja = wave_append(alive, counts + cnt_q(qi ^ 1) + part * kCntLine);
+        if (ja < 0) return;
         const uint32_t jn = part * cap + (uint32_t)ja;
         qout.ox[jn] = pos.x; qout.oy[jn] = pos.y; qout.oz[jn] = pos.z;
-        qout.dx[jn] = ms.wi.x; qout.dy[jn] = ms.wi.y; qout.dz[jn] = ms.wi.z;
+        qout.dx[jn] = dir.x; qout.dy[jn] = dir.y; qout.dz[jn] = dir.z;
         qout.br[jn] = beta.x; qout.bg[jn] = beta.y; qout.bb[jn] = beta.z;
-        qout.pdf[jn] = ms.pdf;
-        qout.flags[jn] = (mat_is_specular(m) ? 1u : 0u) | (segk << 8);
-        qout.rng[jn] = rng.state;
+        qout.pdf[jn] = pdf;
+        qout.flags[jn] = flags;
+        qout.rng[jn] = rng;
         qout.slot[jn] = slot;
     }
+};
+template <bool CAM>
+SRT_D void shade_hit(const DevScene& S, const Segment* segs, int nseg, int depth, const PathQueue& qin, const HitBuf& h,
+                     const PathQueue& qout, const ShadowQueue& sq, float* Lr, float* Lg, float* Lb, uint32_t* counts,
+                     int qi, uint32_t part, uint32_t cap, const MlpIO& mio, uint32_t i) {
+    PathStart ps{};
+    if constexpr (CAM) ps = path_start(segs, nseg, i);
+    const uint32_t slot = CAM ? i : qin.slot[i];
+    const f3 rd = CAM ? ps.d : mk(qin.dx[i], qin.dy[i], qin.dz[i]);
+    const f3 beta = CAM ? mk(1.0f) : mk(qin.br[i], qin.bg[i], qin.bb[i]);
+    if constexpr (CAM) {
+        Lr[slot] = 0.0f; Lg[slot] = 0.0f; Lb[slot] = 0.0f;
+    }
+    const int32_t tri = h.tri[i];
+    const uint32_t flags = CAM ? ps.flags : qin.flags[i];
+    const uint32_t segk = flags >> 8;
+    const SegHead P = load_seg_head(segs, segk);
+    QueueSink<CAM> sink{qin, qout, sq, Lr, Lg, Lb, counts, qi, part, cap, i, slot, ps.o};
+    shade_path(S, P, segk, depth, slot, rd, beta, (flags & 1u) != 0u, CAM ? ps.rng : qin.rng[i], tri, h.u[i], h.v[i],
+               S.num_inst > 0 ? h.inst[i] : -1, counts, part, cap, mio, sink);
 }
 
 // Per entry of queue `qi`: a miss adds beta * env (path_tracer.cu:81-85) and
@@ -1332,13 +1385,26 @@ __global__ void __launch_bounds__(kShadeBlock, 4) k_shade(DevScene S, const Segm
     }
 }
 
-// Shadow rays of the bounce (fetch counter cleared by the trace stage).
+// Total of the kParts size counters at counts[cnt] into host memory, by the
+// first wave of one workgroup: the host reads it while later kernels run.
+SRT_D void report_live(const uint32_t* counts, int cnt, uint32_t* live) {
+    if (threadIdx.x >= 64u) return;
+    uint32_t v = threadIdx.x < (unsigned)kParts ? counts[cnt + threadIdx.x * kCntLine] : 0u;
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+    if (threadIdx.x == 0) __hip_atomic_store(live, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ void k_live(const uint32_t* counts, int cnt, uint32_t* live) { report_live(counts, cnt, live); }
+
+// Shadow rays of the bounce (fetch counter cleared by the trace stage); also
+// reports the size of the next bounce's queue (counts[next]) to the host.
 template <bool COUNT, bool WIDE, bool INST = false>
 __global__ void __launch_bounds__(kTraceBlock) k_shadow(DevScene S, ShadowQueue sq, float* Lr, float* Lg, float* Lb,
                                                        uint32_t* counts, uint32_t cap, int32_t* gstack,
-                                                       unsigned long long* totals, TraceCfg cfg) {
+                                                       unsigned long long* totals, TraceCfg cfg, int next,
+                                                       uint32_t* live) {
     __shared__ uint32_t prefix[kParts + 1];
     uint32_t lo, hi;
+    if (blockIdx.x == 0) report_live(counts, next, live);
     const QueueView view = queue_piece(counts, CNT_SHADOW, cap, prefix, lo, hi);
     uint32_t* fetch = counts + CNT_FETCH_S + my_part() * kCntLine;
     if (blockIdx.x < (unsigned)kParts && threadIdx.x == 0) atomicAdd(&totals[1], (unsigned long long)(hi - lo));
@@ -1349,6 +1415,218 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(DevScene S, ShadowQueue 
     if (COUNT) {
         atomicAdd(&totals[4], (unsigned long long)nv);
         atomicAdd(&totals[5], (unsigned long long)nt);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Whole paths in one launch: each lane takes a path and follows it to its end
+// (closest hit, shading, shadow ray, next bounce), with its state in registers
+// instead of queues.  A bounce of the queue stages costs three launches, each
+// of which lasts as long as its slowest ray (60 to 150 us on the 1M-triangle
+// scene however few rays are left, 6 us with an empty queue); here a lane that
+// is done goes on with its own next ray, so a launch lasts as long as its
+// slowest path.  The price is registers (156 VGPRs, 3 waves per SIMD, against 6
+// of the traversal kernels), which loses once there are rays enough to fill the
+// queue stages: run_chunk switches to it at kWholePathMax live paths.
+// A wave traces until `refill` of its lanes wait for shading or a new path (or
+// none is tracing), then shades those together; a lane starts its path's next
+// ray right after the shadow ray, without waiting for the others.  The shadow
+// ray uses the closest-hit traversal (its answer does not depend on the order).
+// Radiance is added in the order of the queue stages (bounce by bounce, emitter
+// or environment, then light sample), so images are the same bit for bit.
+// ---------------------------------------------------------------------------
+struct PathSink {      // shade_path's results for a path held in registers
+    f3 ro;                   // origin of the ray that hit
+    f3 &beta, &ndir, &L, &sc, &pos, &sdir;
+    float &pdf, &stmax;
+    uint32_t& flags;
+    uint64_t& rng;
+    bool &has_shadow, &alive;
+    SRT_D f3 origin() const { return ro; }
+    SRT_D float scatter_pdf() const { return pdf; }
+    SRT_D void radiance(f3 c) const { L = L + c; }
+    SRT_D void shadow(bool emit, f3 p, f3 dir, float tmax, f3 c) const {
+        has_shadow = emit;
+        pos = p;
+        sdir = dir;
+        stmax = tmax;
+        sc = c;
+    }
+    SRT_D void next(bool go, f3 p, f3 dir, f3 b, float q, uint32_t f, uint64_t state) const {
+        alive = go;
+        pos = p;
+        ndir = dir;
+        beta = b;
+        pdf = q;
+        flags = f;
+        rng = state;
+    }
+};
+
+template <bool CAM, bool INST>
+__global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segment* segs, int nseg, PathQueue q, int depth0,
+                                                      int qi, uint32_t cap, uint32_t* counts, float* Lr, float* Lg,
+                                                      float* Lb, int32_t* gstack, MlpIO mio, float* snap, TraceCfg cfg) {
+    __shared__ uint32_t prefix[kParts + 1];
+    uint32_t lo, hi;
+    const QueueView view = queue_piece(counts, cnt_q(qi), cap, prefix, lo, hi);
+    const uint32_t part = my_part();
+    uint32_t* fetch = counts + CNT_FETCH_T + part * kCntLine;
+    const TravStack k = make_stack<INST>(gstack, cfg);
+    const f3 env = mk(S.env[0], S.env[1], S.env[2]);
+    const int lane = __lane_id();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    // a launch with fewer paths than resident lanes spreads them over its waves
+    const uint32_t waves = gridDim.x / (unsigned)kParts * (kTraceBlock / 64);
+    const uint32_t quota = min(64u, max(1u, (hi - lo + waves - 1u) / waves));
+    const int refill = max(1, (int)(cfg.refill * quota / 64u)), inner_exit = (int)(k.inner_exit * quota / 64u);
+    bool exhausted = (uint32_t)lane >= quota;
+    uint32_t nseg_traced = 0, nshadow = 0, nv = 0;
+    // the path
+    uint32_t slot = 0, flags = 0;
+    uint64_t rng = 0;
+    f3 beta = mk(0.0f), L = mk(0.0f), ndir = mk(0.0f), sc = mk(0.0f);   // ndir: the current or next closest-hit ray's direction
+    float pdf = 1.0f;
+    int depth = 0;
+    bool ready = false;      // a closest-hit result waits for shading
+    bool shadow = false;     // the ray in flight is the shadow ray
+    bool alive = false;      // shadow ray in flight: the path goes on after it
+    bool has = false;        // a ray in flight
+    TravState st;
+    st.cur_ok = false;
+    st.has_pend = false;
+    for (;;) {
+        const unsigned long long act = __ballot(has);
+        const unsigned long long idle = __ballot(!has && !exhausted);
+        if (idle != 0ull && (act == 0ull || __popcll(idle) >= refill)) {
+            f3 o = mk(0.0f), d = mk(0.0f);
+            float tmax = 1e16f;
+            bool start = false;
+            if (ready) {
+                ready = false;
+                const int32_t tri = st.best_pos;
+                f3 ro = st.o;
+                if (INST) {
+                    f3 wd;
+                    unstash_ray(ro, wd);
+                }
+                alive = false;
+                bool has_shadow = false;
+                if (tri < 0) {
+                    L = L + beta * env;
+                } else {
+                    const uint32_t segk = flags >> 8;
+                    const SegHead P = load_seg_head(segs, segk);
+                    const f3 rd = ndir;
+                    PathSink sink{ro, beta, ndir, L, sc, o, d, pdf, tmax, flags, rng, has_shadow, alive};
+                    shade_path(S, P, segk, depth, slot, rd, beta, (flags & 1u) != 0u, rng, tri, st.bu, st.bv, st.best_inst,
+                               counts, part, cap, mio, sink);
+                }
+                if (snap && depth == 1 && !has_shadow) {
+                    snap[3 * (size_t)slot] = L.x; snap[3 * (size_t)slot + 1] = L.y; snap[3 * (size_t)slot + 2] = L.z;
+                }
+                shadow = has_shadow;
+                start = has_shadow || alive;
+                if (has_shadow) {
+                    nshadow++;
+                } else if (alive) {
+                    d = ndir;
+                    tmax = 1e16f;
+                    depth++;
+                    nseg_traced++;
+                } else {
+                    Lr[slot] = L.x; Lg[slot] = L.y; Lb[slot] = L.z;
+                }
+            }
+            const bool want = !has && !exhausted && !start;
+            const unsigned long long m = __ballot(want);
+            if (m != 0ull) {
+                const int leader = __ffsll(m) - 1;
+                uint32_t base = 0;
+                if (lane == leader) base = atomicAdd(fetch, (uint32_t)__popcll(m));
+                base = __shfl(base, leader);
+                if (want) {
+                    const uint32_t idx = lo + base + (uint32_t)__popcll(m & below);
+                    if (idx < hi) {
+                        const uint32_t i = view.entry(idx);
+                        if (CAM) {
+                            const PathStart p = path_start(segs, nseg, i);
+                            slot = i;
+                            o = p.o; ndir = p.d;
+                            beta = mk(1.0f);
+                            L = mk(0.0f);
+                            pdf = 1.0f;
+                            flags = p.flags;
+                            rng = p.rng;
+                            depth = 0;
+                        } else {
+                            slot = q.slot[i];
+                            o = mk(q.ox[i], q.oy[i], q.oz[i]); ndir = mk(q.dx[i], q.dy[i], q.dz[i]);
+                            beta = mk(q.br[i], q.bg[i], q.bb[i]);
+                            L = mk(Lr[slot], Lg[slot], Lb[slot]);
+                            pdf = q.pdf[i];
+                            flags = q.flags[i];
+                            rng = q.rng[i];
+                            depth = depth0;
+                        }
+                        d = ndir;
+                        tmax = 1e16f;
+                        shadow = false;
+                        start = true;
+                        nseg_traced++;
+                    } else {
+                        exhausted = true;
+                    }
+                }
+            }
+            if (start) {
+                trav_begin<INST>(st, o, d, 1e-3f, tmax, S.root4, !shadow);
+                has = true;
+            }
+            if (__ballot(has) == 0ull) break;    // nothing in flight: every lane has run out of paths
+        } else if (act == 0ull) {
+            break;
+        }
+        if (has) {
+            trav_inner4<false, INST, false>(S, st, k, nv, inner_exit);
+            bool occl = false;
+            if (st.has_pend) occl = trav_pend_any<INST>(S, st, k, shadow);
+            if (occl || (!st.cur_ok && !st.has_pend)) {
+                if (!shadow) {
+                    has = false;
+                    ready = true;
+                } else {
+                    if (!occl) L = L + sc;
+                    if (snap && depth == 1) {
+                        snap[3 * (size_t)slot] = L.x; snap[3 * (size_t)slot + 1] = L.y; snap[3 * (size_t)slot + 2] = L.z;
+                    }
+                    shadow = false;
+                    if (alive) {
+                        f3 o = st.o;
+                        if (INST) {
+                            f3 wd;
+                            unstash_ray(o, wd);
+                        }
+                        depth++;
+                        nseg_traced++;
+                        trav_begin<INST>(st, o, ndir, 1e-3f, 1e16f, S.root4, true);
+                    } else {
+                        Lr[slot] = L.x; Lg[slot] = L.y; Lb[slot] = L.z;
+                        has = false;
+                    }
+                }
+            }
+        }
+    }
+    // the launch's segment and shadow-ray counts, per partition
+    for (int d = 32; d > 0; d >>= 1) {
+        nseg_traced += __shfl_xor(nseg_traced, d);
+        nshadow += __shfl_xor(nshadow, d);
+    }
+    if (lane == 0 && nseg_traced) {
+        unsigned long long* c = reinterpret_cast<unsigned long long*>(counts + CNT_PATHS + part * kCntLine);
+        atomicAdd(&c[0], (unsigned long long)nseg_traced);
+        if (nshadow) atomicAdd(&c[1], (unsigned long long)nshadow);
     }
 }
 
@@ -1407,7 +1685,14 @@ __global__ void __launch_bounds__(256) k_targets(int n, const float* Lr, const f
 // Per pixel: add this chunk's samples in sample order (path_tracer.cu:164-165),
 // dropping non-finite samples but keeping the 1/spp weight.  One grid row per
 // segment; a request's film is written when its last segment completes.
-__global__ void __launch_bounds__(256) k_finalize(const float* Lr, const float* Lg, const float* Lb, const Segment* segs) {
+__global__ void __launch_bounds__(256) k_finalize(const float* Lr, const float* Lg, const float* Lb, const Segment* segs,
+                                                  const uint32_t* counts, unsigned long long* totals) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2u) {     // k_paths' segments and shadow rays
+        unsigned long long t = 0;
+        for (int p = 0; p < kParts; p++)
+            t += reinterpret_cast<const unsigned long long*>(counts + CNT_PATHS + p * kCntLine)[threadIdx.x];
+        totals[threadIdx.x] += t;
+    }
     const Segment& sg = segs[blockIdx.y];
     int q = blockIdx.x * blockDim.x + threadIdx.x;     // tile rank of the pixel
     if (q >= sg.wh) return;
@@ -2039,6 +2324,37 @@ static int ensure_mlp_bufs(srt_ctx* c, int64_t slots) {
     return SRT_OK;
 }
 
+// Live paths at which run_chunk finishes a chunk's paths with k_paths (4-wide
+// trees; visit counts come from the queue stages).  Measured with the switch
+// at 0 / 2^20 / 2^21 / 2^22 live paths: 1M-triangle frame 1280x720x1 depth 16
+// 2.89 / 1.61 / 1.63 / 1.62 ms, instanced 1280x720x8 8.12 / 7.14 / 7.11 / 7.62,
+// tube 1280x720x16 4.01 / 3.32 / 3.21 / 3.28, Cornell 256x256x16 0.476 / 0.404 /
+// 0.403 / 0.407, 256x256x64 with the MLP 0.740 / 0.717 / 0.770 / 0.817,
+// 512x512x16 (4.2M paths, all of them at once) 0.87 against 1.04.
+constexpr int64_t kWholePathMax = 1 << 20;
+
+// Waits for the size of the next bounce's queue (report_live), which arrives
+// once the bounce's shading is done, while its shadow rays are still traced:
+// the next launches are queued before the device runs dry.
+constexpr uint32_t kNotYet = 0xffffffffu;
+static int wait_live(srt_ctx* c, int64_t* n) {
+    for (;;) {
+        for (int spin = 0; spin < 4096; spin++) {
+            const uint32_t v = __atomic_load_n(c->live, __ATOMIC_RELAXED);
+            if (v != kNotYet) {
+                *n = v;
+                return SRT_OK;
+            }
+            __builtin_ia32_pause();
+        }
+        const hipError_t e = hipStreamQuery(c->stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return hip_check(c, e, "bounce");
+        if (__atomic_load_n(c->live, __ATOMIC_SEQ_CST) == kNotYet)
+            return set_err(c, SRT_E_HIP, "the bounce's path count did not arrive");
+    }
+}
+
 // Runs one chunk: segments (in slot order) of one scene share the path queues.
 int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, TrainOut* train) {
     if (nseg <= 0 || nseg > kMaxSegments) return set_err(c, SRT_E_LIMIT, "bad segment count %d", nseg);
@@ -2059,8 +2375,14 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     const int tgrid = part_grid(trace_grid(c, n));
     const int pgrid = part_grid(trace_grid(c, n, reinterpret_cast<const void*>(k_trace_packet)));
     const uint32_t cap = part_cap((uint32_t)n);
-    if (int r = ensure_gstack(c, s, (int64_t)tgrid * kTraceBlock)) return r;
+    const bool inst = s->ninst > 0;
+    const int wgrid = part_grid(trace_grid(c, n, inst ? reinterpret_cast<const void*>(k_paths<true, true>)
+                                                      : reinterpret_cast<const void*>(k_paths<true, false>)));
+    if (int r = ensure_gstack(c, s, (int64_t)std::max(tgrid, wgrid) * kTraceBlock)) return r;
     const TraceCfg tcfg = trace_cfg(c, s);
+    const int64_t whole = tcfg.wide && !c->count_visits ? kWholePathMax : 0;
+    int64_t npaths = n;                   // live paths of the bounce
+    uint32_t* live = c->live;
     TraceCfg scfg = tcfg;
     scfg.refill = c->shadow_refill;
     const size_t tlds = trace_lds_bytes(tcfg);
@@ -2092,7 +2414,6 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     uint32_t* counts = (uint32_t*)c->counters.p;
     unsigned long long* totals = (unsigned long long*)((char*)c->counters.p + kTotalsOffset);
     PathQueue Q[2] = {make_queue(c, 0), make_queue(c, 1)};
-    const bool inst = s->ninst > 0;
     HitBuf H;
     H.u = (float*)c->hits[1].p; H.v = (float*)c->hits[2].p; H.tri = (int32_t*)c->hits[3].p;
     H.inst = inst ? (int32_t*)c->hits[4].p : nullptr;
@@ -2110,14 +2431,34 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     hipEvent_t ev;
     // the first bounce's queue is the slots (its trace and shade stages compute
     // each path's camera ray and state); only its partition sizes are set here
-    k_path_counts<<<1, 64, 0, st>>>((uint32_t)n, cap, counts);
+    k_path_counts<<<1, 4 * kParts, 0, st>>>((uint32_t)n, cap, counts);
     if (max_depth == 0)                   // no shade stage sets the radiance
         for (float* L : {Lr, Lg, Lb}) k_zero<<<nblk, 256, 0, st>>>(L, (size_t)n);
     if (mlp_mode == 2) k_zero<<<nblk, 256, 0, st>>>((float*)mio.rec_valid, (size_t)n);
-    for (int depth = 0; depth < max_depth; depth++) {
+    for (int depth = 0; depth < max_depth && npaths > 0; depth++) {
         int qi = depth & 1;
         const bool cam = depth == 0;
         const bool cnt = c->count_visits;
+        const int packet = cam && !cnt ? trace_packet_ok(c, s, tcfg) : 0;
+        if (npaths <= whole && !packet) {      // the rest of every path in one launch
+            prof_begin(c, "paths", &ev);
+            float* snap = mlp_mode == 2 && depth <= 1 ? (float*)c->mlpbuf[7].p : nullptr;
+            if (inst) {
+                if (cam) k_paths<true, true><<<wgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
+                else k_paths<false, true><<<wgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
+            } else {
+                if (cam) k_paths<true, false><<<wgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
+                else k_paths<false, false><<<wgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
+            }
+            prof_end(c, "paths", ev, 0);
+            if (depth <= 1 && mlp_mode == 1) {
+                float* pred = (float*)c->mlpbuf[3].p;
+                k_mlp_compact<<<shade_grid, 256, 0, st>>>(counts, cap, mio);
+                if (int r = mlp_query_dev(c, mio.q_in9, counts + CNT_MLPQ, (int)n, pred)) return r;
+                k_mlp_apply<<<shade_grid, 256, 0, st>>>(counts, pred, mio.q_beta, mio.q_slot, Lr, Lg, Lb);
+            }
+            break;
+        }
         prof_begin(c, "trace", &ev);
         if (inst) {
             if (cam && cnt) k_trace_cam<true, true, true><<<tgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, H, counts, cap, gst, totals, tcfg);
@@ -2126,7 +2467,7 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
             else k_trace<false, true, true><<<tgrid, kTraceBlock, ilds, st>>>(S, Q[qi], H, counts, qi, cap, gst, totals, tcfg);
         } else if (tcfg.wide) {
             TraceCfg pcfg = tcfg;
-            pcfg.packet = cam && !cnt ? trace_packet_ok(c, s, tcfg) : 0;
+            pcfg.packet = packet;
             if (cam && cnt) k_trace_cam<true, true><<<tgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, H, counts, cap, gst, totals, tcfg);
             else if (pcfg.packet) k_trace_packet<<<pgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, H, counts, cap, totals, pcfg);
             else if (cam) k_trace_cam<false, true><<<tgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, H, counts, cap, gst, totals, tcfg);
@@ -2145,20 +2486,23 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
         else
             k_shade<false><<<shade_grid, 256, 0, st>>>(S, segs, nseg, depth, Q[qi], H, Q[qi ^ 1], SQ, Lr, Lg, Lb, counts, qi, cap, mio);
         prof_end(c, "shade", ev, 0);
-        if (any_nee) {
+        __atomic_store_n(live, kNotYet, __ATOMIC_SEQ_CST);
+        if (!any_nee) {
+            k_live<<<1, 64, 0, st>>>(counts, cnt_q(qi ^ 1), live);
+        } else {
             prof_begin(c, "shadow", &ev);
             if (inst) {
                 if (c->count_visits)
-                    k_shadow<true, true, true><<<tgrid, kTraceBlock, ilds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg);
-                else k_shadow<false, true, true><<<tgrid, kTraceBlock, ilds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg);
+                    k_shadow<true, true, true><<<tgrid, kTraceBlock, ilds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg, cnt_q(qi ^ 1), live);
+                else k_shadow<false, true, true><<<tgrid, kTraceBlock, ilds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg, cnt_q(qi ^ 1), live);
             } else if (tcfg.wide) {
                 if (c->count_visits)
-                    k_shadow<true, true><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg);
-                else k_shadow<false, true><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg);
+                    k_shadow<true, true><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg, cnt_q(qi ^ 1), live);
+                else k_shadow<false, true><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg, cnt_q(qi ^ 1), live);
             } else {
                 if (c->count_visits)
-                    k_shadow<true, false><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg);
-                else k_shadow<false, false><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg);
+                    k_shadow<true, false><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg, cnt_q(qi ^ 1), live);
+                else k_shadow<false, false><<<tgrid, kTraceBlock, tlds, st>>>(S, SQ, Lr, Lg, Lb, counts, cap, gst, totals, scfg, cnt_q(qi ^ 1), live);
             }
             prof_end(c, "shadow", ev, 0);
         }
@@ -2170,6 +2514,9 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
             k_mlp_apply<<<shade_grid, 256, 0, st>>>(counts, pred, mio.q_beta, mio.q_slot, Lr, Lg, Lb);
         }
         if (depth == 1 && mlp_mode == 2) k_snapshot<<<nblk, 256, 0, st>>>((int)n, Lr, Lg, Lb, (float*)c->mlpbuf[7].p);
+        if (depth + 1 < max_depth) {
+            if (int r = wait_live(c, &npaths)) return r;
+        }
     }
     if (mlp_mode == 2 && train && train->count < train->cap) {
         float* snap_t = (float*)c->mlpbuf[7].p;     // snapshot, then overwritten by the targets
@@ -2195,7 +2542,7 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     int maxwh = 0;
     for (int k = 0; k < nseg; k++) maxwh = std::max(maxwh, (int)segs_host[k].wh);
     prof_begin(c, "finalize", &ev);
-    k_finalize<<<dim3((unsigned)((maxwh + 255) / 256), (unsigned)nseg), 256, 0, st>>>(Lr, Lg, Lb, segs);
+    k_finalize<<<dim3((unsigned)((maxwh + 255) / 256), (unsigned)nseg), 256, 0, st>>>(Lr, Lg, Lb, segs, counts, totals);
     prof_end(c, "finalize", ev, maxwh);
     // the host segment array may be reused by the caller after this returns
     return hip_check(c, hipStreamSynchronize(st), "chunk");

@@ -145,3 +145,24 @@ def test_query_paths_independent_of_chunking(ctx):
     ctx.release(h)
     assert np.isfinite(a).all()
     assert np.array_equal(a, b)
+
+
+def test_hooks_equal_in_whole_path_kernel_and_queue_stages(ctx):
+    """Training frames (vertex-2 records and snapshots) and query frames give
+    the same bits whether the paths are finished by the whole-path kernel or
+    run as queue stages (visit counting on)."""
+    from srt_amd import scenes
+    s = scenes.cornell()
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    out = []
+    for count in (0, 1):
+        ctx.set_option("count_visits", count)
+        ctx.mlp_create(seed=3, lr=1e-3)
+        loss, n = ctx.mlp_train_frame(h, s.camera, 77, 53, 4, 5, 4, seed=9, max_samples=1 << 14, steps=3)
+        out.append((loss, n, ctx.mlp_params(), ctx.render(h, s.camera, 77, 53, 3, 5, 4, 1, 1, 2, mlp_mode=1)))
+    ctx.set_option("count_visits", 0)
+    ctx.release(h)
+    assert out[0][:2] == out[1][:2] and out[0][1] > 1000
+    assert np.array_equal(out[0][2], out[1][2])
+    assert np.array_equal(out[0][3], out[1][3])

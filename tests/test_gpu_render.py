@@ -236,3 +236,26 @@ def test_skinned_tube_posed_frame(ctx, frame):
     # the pose moved the tube: the image differs from the rest pose's
     rest, _ = O.render(O.Scene(s), s.camera, W, H, 2, 6, 4, 1, 1, 100 + frame)
     assert np.mean(np.any(np.abs(rest[:, :3] - ref[:, :3]) > 1e-3, axis=1)) > 0.02
+
+
+@pytest.mark.parametrize("name,W,H,spp,depth", [
+    ("cornell", 1, 1, 1, 5), ("cornell", 65, 33, 3, 1), ("cornell", 97, 61, 5, 16),
+    ("spheres", 129, 71, 2, 8), ("tube", 250, 131, 3, 6), ("cornell_instanced", 67, 45, 4, 5),
+    ("cornell", 1031, 1021, 1, 5),          # above the switch: its first bounces run as queue stages
+    ("cornell_instanced", 1031, 1021, 1, 4)])
+def test_whole_path_kernel_equals_queue_stages(ctx, name, W, H, spp, depth):
+    """Chunks of few live paths are finished by one kernel that keeps each
+    path in registers; with visit counting on, every bounce runs as queue
+    stages.  Both add the same terms in the same order: equal bits, and equal
+    segment and shadow-ray counts."""
+    s = getattr(scenes, name)()
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    out = []
+    for count in (0, 1):
+        ctx.set_option("count_visits", count)
+        out.append((ctx.render(h, s.camera, W, H, spp, depth, 4, 1, 1, 7), ctx.last_counts()))
+    ctx.set_option("count_visits", 0)
+    ctx.release(h)
+    assert np.array_equal(out[0][0], out[1][0])
+    assert out[0][1] == out[1][1]
