@@ -125,9 +125,10 @@ const char* srt_last_error(const srt_ctx* ctx);
  * results are identical; packets gain 1 % of the closest-hit time on a scene
  * that fills the frame with deep traversals and lose 10 % where camera rays
  * visit few nodes), "keep_build_scratch" (1, the
- * default: the device scratch of a BVH build stays allocated for the next build
- * and counts in srt_hbm_used; it is freed when an allocation would exceed the
- * budget or fail; 0: freed now and at the end of every build).  Limits: 2^28 - 1 triangles per scene; "path_pool" and the pool
+ * default: the device scratch of a BVH build, and of a denoise pass up to 512 MiB,
+ * stays allocated for the next one and counts in srt_hbm_used; it is freed when
+ * an allocation would exceed the budget or fail; 0: freed now and at the end of
+ * every build and pass).  Limits: 2^28 - 1 triangles per scene; "path_pool" and the pool
  * of srt_serve_start in [64, 2^31 - 1]. */
 int srt_set_option(srt_ctx* ctx, const char* key, int64_t value);
 size_t srt_hbm_used(const srt_ctx* ctx);

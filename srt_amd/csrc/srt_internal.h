@@ -316,6 +316,7 @@ struct srt_ctx {
     // allocates and frees nothing); released when an allocation would exceed
     // the budget or fail, and at srt_destroy
     std::vector<srt::DevBuf> build_scratch;
+    srt::DevBuf post_scratch;             // the last denoise's scratch, kept and released in the same way
     std::mutex scratch_mu;
     bool keep_build_scratch = true;
     int64_t film_pixels = 0;
@@ -363,7 +364,7 @@ int dev_alloc(srt_ctx* c, DevBuf& b, size_t bytes);
 void dev_free(srt_ctx* c, DevBuf& b);
 // keeps b when it already holds exactly `bytes`, else frees and allocates
 int dev_realloc(srt_ctx* c, DevBuf& b, size_t bytes);
-// frees the kept build-scratch chunks; returns whether there were any
+// frees the kept scratch of builds and denoise passes; returns whether there was any
 bool release_build_scratch(srt_ctx* c);
 int set_err(srt_ctx* c, int code, const char* fmt, ...);
 int hip_check(srt_ctx* c, hipError_t e, const char* what);
@@ -419,7 +420,7 @@ int trace_rays_noalloc(srt_ctx* c, SceneRec* s, int n, const float* o_dev, const
                        const float* tmax_dev, int any, float* t, float* u, float* v, int32_t* prim);
 int tonemap_dev(srt_ctx* c, float* rgba, int n, int type, float exposure, int use_gamma);
 int accumulate_dev(srt_ctx* c, float* acc, float* rgba, int n, int frame_count);
-int denoise_dev(srt_ctx* c, float* rgba, float* tmp, int W, int H);
+int denoise_dev(srt_ctx* c, float* rgba, float* tmp, int images, int W, int H);
 DevScene dev_scene(const SceneRec* s);
 DevCamera make_camera(const float pos[3], const float target[3], const float up[3], float fov, int W, int H);
 }  // namespace srt

@@ -64,3 +64,33 @@ def test_odd_sizes_and_device_film(ctx):
     finally:
         ctx.device_free(ptr)
     assert np.array_equal(back, ref)
+
+
+@pytest.mark.parametrize("W,H", [(1, 1), (3, 70), (64, 16), (65, 129), (200, 67)])
+@pytest.mark.parametrize("short", [False, True])
+def test_row_groups_and_scratch_sizes(ctx, W, H, short):
+    """Four rows a thread at every spacing: images below, at and above one
+    group of rows and one wave of columns, with weights from 1 to 0, an
+    infinite and a NaN pixel; with the scratch of three images and, under a
+    tight budget, of two (a guide kernel per pass).  Equal to the oracle's plain
+    loop bit for bit (NaN where it is NaN)."""
+    rng = np.random.default_rng(W * 1000 + H)
+    a = np.ones((W * H, 4), np.float32)
+    a[:, :3] = np.exp(rng.normal(0.0, 1.0 + 2.0 * (rng.uniform(size=(W * H, 1)) < 0.1), size=(W * H, 3)))
+    a[rng.uniform(size=W * H) < 0.1, :3] = 0.0
+    a[:, 3] = rng.uniform(size=W * H)
+    if W * H > 5000:
+        a[1234, 0] = np.inf
+        a[4321, 1] = np.nan
+    ref = O.denoise(a, W, H)
+    if short:
+        ctx.set_option("keep_build_scratch", 0)
+        ctx.set_option("hbm_budget", ctx.hbm_used() + a.nbytes * 3 + 64)
+    try:
+        out = ctx.denoise(a, W, H)
+    finally:
+        if short:
+            ctx.set_option("hbm_budget", 64 << 30)
+            ctx.set_option("keep_build_scratch", 1)
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    assert np.array_equal(np.nan_to_num(out), np.nan_to_num(ref))
