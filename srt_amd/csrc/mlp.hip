@@ -522,12 +522,25 @@ __global__ void __launch_bounds__(MLP_BLOCK, 1) k_mlp_train(const float* in9, co
 constexpr int ADAM_PARAMS = 64;
 constexpr int ADAM_GROUPS = 16;
 constexpr int ADAM_BLOCK = ADAM_PARAMS * ADAM_GROUPS;
+constexpr int ADAM_BLOCKS = (W_TOTAL + B_TOTAL + ADAM_PARAMS - 1) / ADAM_PARAMS;
 __global__ void __launch_bounds__(ADAM_BLOCK) k_mlp_adam(int nchunks, const float* wpart, const float* bpart, float* W, float* B,
                                                   float* mW, float* vW, float* mB, float* vB, float lr, float b1, float b2,
                                                   float eps, float c1, float c2, int apply, float* grad_out, uint16_t* wf,
-                                                  uint16_t* wt) {
+                                                  uint16_t* wt, const float* loss_part, float* loss) {
     __shared__ float sg[ADAM_BLOCK];
     const int t = threadIdx.x, grp = t >> 6;
+    if (blockIdx.x == ADAM_BLOCKS) {       // the extra block: the step's loss, its partials added in order
+        float s = 0.0f;
+        for (int base = 0; base < nchunks; base += ADAM_BLOCK) {
+            if (base + t < nchunks) sg[t] = loss_part[base + t];
+            __syncthreads();
+            if (t == 0)
+                for (int i = 0; i < min(ADAM_BLOCK, nchunks - base); i++) s += sg[i];
+            __syncthreads();
+        }
+        if (t == 0) loss[0] = s;
+        return;
+    }
     const int p = blockIdx.x * ADAM_PARAMS + (t & 63);
     float part = 0.0f;
     if (p < W_TOTAL) {
@@ -577,14 +590,6 @@ __global__ void __launch_bounds__(ADAM_BLOCK) k_mlp_adam(int nchunks, const floa
             float mh = m / c1, vh = v / c2;
             B[q] = B[q] - lr * mh / (__builtin_sqrtf(vh) + eps);
         }
-    }
-}
-
-__global__ void k_loss_sum(const float* part, int nparts, float* out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        float s = 0.0f;
-        for (int i = 0; i < nparts; i++) s += part[i];
-        out[0] = s;
     }
 }
 
@@ -646,10 +651,9 @@ static MlpDev mlp_dev(MlpState* m) {
 
 // refresh BF16 copies without an update (apply = 0)
 static int refresh_copies(srt_ctx* c, MlpState* m) {
-    const int tot = W_TOTAL + B_TOTAL;
-    k_mlp_adam<<<(tot + ADAM_PARAMS - 1) / ADAM_PARAMS, ADAM_BLOCK, 0, c->stream>>>(0, nullptr, nullptr, (float*)m->W.p, (float*)m->B.p, nullptr,
+    k_mlp_adam<<<ADAM_BLOCKS, ADAM_BLOCK, 0, c->stream>>>(0, nullptr, nullptr, (float*)m->W.p, (float*)m->B.p, nullptr,
                                                          nullptr, nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f, 0,
-                                                         nullptr, (uint16_t*)m->wf.p, (uint16_t*)m->wt.p);
+                                                         nullptr, (uint16_t*)m->wf.p, (uint16_t*)m->wt.p, nullptr, nullptr);
     return hip_check(c, hipGetLastError(), "mlp refresh");
 }
 
@@ -683,43 +687,42 @@ static int ensure_in(srt_ctx* c, MlpState* m, int64_t n) {
 static int infer_grid(srt_ctx* c, int64_t n) {
     int64_t tiles = (n + T_TILE - 1) / T_TILE;
     int64_t blocks = (tiles + MLP_BLOCK / 64 - 1) / (MLP_BLOCK / 64);
-    hipDeviceProp_t prop;
-    int cus = 256;
-    if (hipGetDeviceProperties(&prop, c->device) == hipSuccess) cus = prop.multiProcessorCount;
-    int64_t cap = (int64_t)cus * 2;
+    int64_t cap = (int64_t)num_cus(c) * 2;
     return (int)std::max<int64_t>(1, std::min(blocks, cap));
 }
 
 // one training step on device arrays (in9 [n][9], target [n][3]); apply = 0
-// computes gradients only (grad_out host pointer optional)
-static int train_step_dev(srt_ctx* c, MlpState* m, const float* in9, const float* target, int n, int apply, float* loss_host,
-                          float* grad_host) {
+// computes gradients only (grad_out host pointer optional); the loss sum stays
+// in the given slot of the loss buffer (loss_host: and is read back)
+static int train_step_dev(srt_ctx* c, MlpState* m, const float* in9, const float* target, int n, int apply, int slot,
+                          float* loss_host, float* grad_host) {
     if (int r = ensure_train(c, m, n)) return r;
     hipStream_t st = c->stream;
     MlpDev d = mlp_dev(m);
     const int chunk = train_chunk(n), chunks = (n + chunk - 1) / chunk;
-    if (!m->loss.p) if (int r = dev_alloc(c, m->loss, 16)) return r;
+    if (!m->loss.p) if (int r = dev_alloc(c, m->loss, kLossSlots * 4)) return r;
     if (!m->grad.p) if (int r = dev_alloc(c, m->grad, (size_t)(W_TOTAL + B_TOTAL) * 4)) return r;
     hipEvent_t ev;
     prof_begin(c, "mlp_train", &ev);
     k_mlp_train<<<chunks, MLP_BLOCK, 0, st>>>(in9, target, n, chunk, 1.0f / (3.0f * (float)n), d, (float*)m->wpart.p,
                                               (float*)m->bpart.p, (float*)m->loss_part.p);
     prof_end(c, "mlp_train", ev, n);
-    k_loss_sum<<<1, 64, 0, st>>>((const float*)m->loss_part.p, chunks, (float*)m->loss.p);
+    float* loss = (float*)m->loss.p + slot;
     if (apply) m->step++;
     const float c1 = 1.0f - std::pow(m->b1, (float)std::max(m->step, 1));
     const float c2 = 1.0f - std::pow(m->b2, (float)std::max(m->step, 1));
     const int tot = W_TOTAL + B_TOTAL;
     prof_begin(c, "mlp_adam", &ev);
-    k_mlp_adam<<<(tot + ADAM_PARAMS - 1) / ADAM_PARAMS, ADAM_BLOCK, 0, st>>>(chunks, (const float*)m->wpart.p, (const float*)m->bpart.p, (float*)m->W.p,
+    k_mlp_adam<<<ADAM_BLOCKS + 1, ADAM_BLOCK, 0, st>>>(chunks, (const float*)m->wpart.p, (const float*)m->bpart.p, (float*)m->W.p,
                                                   (float*)m->B.p, (float*)m->mW.p, (float*)m->vW.p, (float*)m->mB.p,
                                                   (float*)m->vB.p, m->lr, m->b1, m->b2, m->eps, c1, c2, apply,
-                                                  (float*)m->grad.p, (uint16_t*)m->wf.p, (uint16_t*)m->wt.p);
+                                                  (float*)m->grad.p, (uint16_t*)m->wf.p, (uint16_t*)m->wt.p,
+                                                  (const float*)m->loss_part.p, loss);
     prof_end(c, "mlp_adam", ev, tot);
     if (int r = hip_check(c, hipGetLastError(), "mlp train launch")) return r;
     if (loss_host) {
         float l = 0.0f;
-        if (int r = hip_check(c, hipMemcpyAsync(&l, m->loss.p, 4, hipMemcpyDeviceToHost, st), "loss")) return r;
+        if (int r = hip_check(c, hipMemcpyAsync(&l, loss, 4, hipMemcpyDeviceToHost, st), "loss")) return r;
         if (int r = hip_check(c, hipStreamSynchronize(st), "mlp train")) return r;
         *loss_host = l / (3.0f * (float)n);
     }
@@ -760,10 +763,19 @@ int mlp_query_dev(srt_ctx* c, const float* in9, const uint32_t* count_dev, int m
 
 bool mlp_ready(srt_ctx* c) { return mlp_of(c) != nullptr; }
 
-int mlp_train_dev(srt_ctx* c, const float* in9, const float* target, int n, float* loss_host) {
+int mlp_train_dev(srt_ctx* c, const float* in9, const float* target, int n, int slot) {
     MlpState* m = mlp_of(c);
     if (!m) return set_err(c, SRT_E_STATE, "no MLP: call srt_mlp_create first");
-    return train_step_dev(c, m, in9, target, n, 1, loss_host, nullptr);
+    return train_step_dev(c, m, in9, target, n, 1, slot, nullptr, nullptr);
+}
+
+int mlp_losses(srt_ctx* c, int n, int count, float* mean) {
+    MlpState* m = mlp_of(c);
+    if (!m || !m->loss.p) return set_err(c, SRT_E_STATE, "no MLP: call srt_mlp_create first");
+    if (int r = hip_check(c, hipMemcpyAsync(mean, m->loss.p, 4 * (size_t)count, hipMemcpyDeviceToHost, c->stream), "loss")) return r;
+    if (int r = hip_check(c, hipStreamSynchronize(c->stream), "mlp train")) return r;
+    for (int k = 0; k < count; k++) mean[k] = mean[k] / (3.0f * (float)n);
+    return SRT_OK;
 }
 
 void mlp_bounds(srt_ctx* c, const float lo[3], const float hi[3]) {
@@ -961,7 +973,7 @@ int srt_mlp_train_step(srt_ctx* c, int32_t n, const float* in9, const float* tar
     if (int r = hip_check(c, hipMemcpy(m->in_buf.p, in9, (size_t)n * 36, hipMemcpyHostToDevice), "upload")) return r;
     if (int r = hip_check(c, hipMemcpy(m->tgt_buf.p, target3, (size_t)n * 12, hipMemcpyHostToDevice), "upload")) return r;
     std::vector<float> g(grads ? (size_t)(W_TOTAL + B_TOTAL) : 0);
-    int r = train_step_dev(c, m, (const float*)m->in_buf.p, (const float*)m->tgt_buf.p, n, apply, loss,
+    int r = train_step_dev(c, m, (const float*)m->in_buf.p, (const float*)m->tgt_buf.p, n, apply, 0, loss,
                            grads ? g.data() : nullptr);
     if (r) return r;
     prof_collect(c);

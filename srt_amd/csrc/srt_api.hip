@@ -183,12 +183,14 @@ int srt_create(int device, size_t hbm_budget_bytes, srt_ctx** out) {
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return SRT_E_HIP; }
     if (dev_alloc(c, c->counters, kCountersBytes)) { (void)hipStreamDestroy(c->stream); delete c; return SRT_E_OOM; }
     (void)hipMemset(c->counters.p, 0, kCountersBytes);
-    if (hipHostMalloc((void**)&c->live, 64, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void**)&c->live, 128, hipHostMallocDefault) != hipSuccess) {
         dev_free(c, c->counters);
         (void)hipStreamDestroy(c->stream);
         delete c;
         return SRT_E_OOM;
     }
+    memset(c->live, 0, 128);
+    c->host_totals = reinterpret_cast<unsigned long long*>(c->live + 16);
     if (int r = noalloc_init(c)) {
         (void)hipHostFree(c->live);
         dev_free(c, c->counters);
@@ -817,13 +819,16 @@ int srt_mlp_train_frame(srt_ctx* c, srt_scene h, const srt_camera* cam, const sr
     const int64_t batch = tr.count / steps;
     double lsum = 0.0;
     int done = 0;
+    float mean[kLossSlots];
     for (int k = 0; k < steps && batch > 0; k++) {
-        float l = 0.0f;
-        if (int r = mlp_train_dev(c, tr.in9 + (size_t)k * batch * 9, tr.target + (size_t)k * batch * 3, (int)batch,
-                                  loss_out ? &l : nullptr))
-            return r;
-        lsum += l;
+        const int slot = k % kLossSlots;
+        if (int r = mlp_train_dev(c, tr.in9 + (size_t)k * batch * 9, tr.target + (size_t)k * batch * 3, (int)batch, slot)) return r;
         done++;
+        // the losses are read together, once the steps are queued
+        if (loss_out && (slot == kLossSlots - 1 || k == steps - 1)) {
+            if (int r = mlp_losses(c, (int)batch, slot + 1, mean)) return r;
+            for (int j = 0; j <= slot; j++) lsum += mean[j];
+        }
     }
     if (loss_out) *loss_out = done ? (float)(lsum / done) : 0.0f;
     if (int r = hip_check(c, hipStreamSynchronize(c->stream), "train frame")) return r;

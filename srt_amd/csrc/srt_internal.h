@@ -224,6 +224,7 @@ enum {
     CNT_WORDS = CNT_PATHS + kParts * kCntLine
 };
 // statistics (unsigned 64-bit) after the counters, then the end of the buffer
+constexpr int kTotals = 6;             // segments, shadow rays, node visits and triangle tests of both
 constexpr size_t kTotalsOffset = (size_t)CNT_WORDS * 4;
 constexpr size_t kCountersBytes = kTotalsOffset + 256;
 // first size counter of path queue qi (0 or 1)
@@ -323,7 +324,12 @@ struct srt_ctx {
     size_t gstack_entries = 0;            // int32 entries allocated in gstack
     int32_t trace_lds_depth = 16, trace_refill = 40, shadow_refill = 32, trace_blocks_per_cu = 0;   // 0: occupancy limit
     int32_t trace_bvh_width = 4;          // traversal over the 4-wide (4) or binary (2) tree
-    uint32_t* live = nullptr;             // pinned host word: live paths of the next bounce (report_live)
+    // pinned host memory that kernels write: live[0] the live paths of the next
+    // bounce (report_live), live[1] a training chunk's samples; host_totals
+    // (kTotals words) the render's totals (k_finalize)
+    uint32_t* live = nullptr;
+    unsigned long long* host_totals = nullptr;
+    std::map<std::pair<const void*, size_t>, int> occupancy;   // resident workgroups per CU by kernel and LDS bytes
     int32_t trace_inner_exit = 18;        // stragglers resume after the leaf step
     int32_t trace_packet = 0;             // > 0: camera rays traversed as 64-ray packets (0: per ray)
     int64_t max_wide_nodes = srt::kMaxNodes4;   // 4-wide trees above this many nodes are traversed in binary form
@@ -359,6 +365,7 @@ struct srt_ctx {
     } while (0)
 
 namespace srt {
+int num_cus(srt_ctx* c);
 // allocation helpers (budget-checked)
 int dev_alloc(srt_ctx* c, DevBuf& b, size_t bytes);
 void dev_free(srt_ctx* c, DevBuf& b);
@@ -401,7 +408,11 @@ int render_light(srt_ctx* c, SceneRec* s, const DevCamera& cam, int spp, int max
 // MLP (mlp.hip)
 int mlp_infer_dev(srt_ctx* c, const float* in9, int n, float* out3);
 int mlp_query_dev(srt_ctx* c, const float* in9, const uint32_t* count_dev, int max_n, float* out3);
-int mlp_train_dev(srt_ctx* c, const float* in9, const float* target, int n, float* loss_host);
+// one Adam step whose loss sum stays in slot k of the MLP's loss buffer, and
+// the means of the steps in slots [0, count) (waits for them)
+constexpr int kLossSlots = 256;
+int mlp_train_dev(srt_ctx* c, const float* in9, const float* target, int n, int slot);
+int mlp_losses(srt_ctx* c, int n, int count, float* mean);
 bool mlp_ready(srt_ctx* c);
 // the MLP that renders of scene h query: h's own, else the context's own (or null)
 void* mlp_for_scene(srt_ctx* c, uint64_t h);

@@ -854,13 +854,18 @@ SRT_D PathStart path_start(const Segment* segs, int nseg, uint32_t slot) {
     p.rng = rng.state;
     return p;
 }
-// Sizes of the first bounce's queue partitions (n slots, partition p holds
-// slots [p cap, p cap + size)); clears the traversal fetch counters.
-__global__ void k_path_counts(uint32_t n, uint32_t cap, uint32_t* counts) {
+// Start of a chunk: sizes of the first bounce's queue partitions (n slots,
+// partition p holds slots [p cap, p cap + size)), cleared fetch counters and
+// whole-path counts; a lone segment comes as an argument (put) instead of a
+// copy of its own, and a frame's first chunk clears the totals (first).
+__global__ void k_chunk_begin(uint32_t n, uint32_t cap, uint32_t* counts, Segment seg, Segment* segs, int put,
+                              unsigned long long* totals, int first) {
     clear_parts(counts + CNT_FETCH_T);
     clear_parts(counts + CNT_MLPQ_PARTS);
     if (threadIdx.x < 4u * kParts) counts[CNT_PATHS + (threadIdx.x >> 2) * kCntLine + (threadIdx.x & 3u)] = 0u;
     if (threadIdx.x < (unsigned)kParts) counts[CNT_Q0 + threadIdx.x * kCntLine] = part_size(n, cap, threadIdx.x);
+    if (put && threadIdx.x == 0) segs[0] = seg;
+    if (first && threadIdx.x < (unsigned)kTotals) totals[threadIdx.x] = 0ull;
 }
 
 // Ray sources/sinks of the persistent traversal loop.
@@ -1553,6 +1558,7 @@ __global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segm
                         if (CAM) {
                             const PathStart p = path_start(segs, nseg, i);
                             slot = i;
+                            if (snap) mio.rec_valid[slot] = 0u;
                             o = p.o; ndir = p.d;
                             beta = mk(1.0f);
                             L = mk(0.0f);
@@ -1687,12 +1693,16 @@ __global__ void __launch_bounds__(256) k_targets(int n, const float* Lr, const f
 // dropping non-finite samples but keeping the 1/spp weight.  One grid row per
 // segment; a request's film is written when its last segment completes.
 __global__ void __launch_bounds__(256) k_finalize(const float* Lr, const float* Lg, const float* Lb, const Segment* segs,
-                                                  const uint32_t* counts, unsigned long long* totals) {
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2u) {     // k_paths' segments and shadow rays
-        unsigned long long t = 0;
-        for (int p = 0; p < kParts; p++)
-            t += reinterpret_cast<const unsigned long long*>(counts + CNT_PATHS + p * kCntLine)[threadIdx.x];
-        totals[threadIdx.x] += t;
+                                                  const uint32_t* counts, unsigned long long* totals,
+                                                  unsigned long long* host_totals) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < (unsigned)kTotals) {
+        // the totals, with k_paths' segments and shadow rays, into host memory
+        unsigned long long t = totals[threadIdx.x];
+        if (threadIdx.x < 2u)
+            for (int p = 0; p < kParts; p++)
+                t += reinterpret_cast<const unsigned long long*>(counts + CNT_PATHS + p * kCntLine)[threadIdx.x];
+        totals[threadIdx.x] = t;
+        __hip_atomic_store(&host_totals[threadIdx.x], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     const Segment& sg = segs[blockIdx.y];
     int q = blockIdx.x * blockDim.x + threadIdx.x;     // tile rank of the pixel
@@ -1702,7 +1712,9 @@ __global__ void __launch_bounds__(256) k_finalize(const float* Lr, const float* 
     int64_t s0 = (sg.path_begin - q + sg.wh - 1) / sg.wh;
     if (s0 < 0) s0 = 0;
     float* acc = sg.film_acc;
-    float ax = acc[3 * (size_t)px], ay = acc[3 * (size_t)px + 1], az = acc[3 * (size_t)px + 2];
+    // the sums of the request's earlier chunks (none before its first path)
+    float ax = 0.0f, ay = 0.0f, az = 0.0f;
+    if (sg.path_begin != 0) { ax = acc[3 * (size_t)px]; ay = acc[3 * (size_t)px + 1]; az = acc[3 * (size_t)px + 2]; }
     const float fspp = (float)sg.spp;
     for (int64_t s = s0;; s++) {
         int64_t pid = s * sg.wh + q;
@@ -1715,8 +1727,8 @@ __global__ void __launch_bounds__(256) k_finalize(const float* Lr, const float* 
             az = az + L.z / fspp;
         }
     }
-    acc[3 * (size_t)px] = ax; acc[3 * (size_t)px + 1] = ay; acc[3 * (size_t)px + 2] = az;
-    if (sg.last && sg.film_out) sg.film_out[px] = make_float4(ax, ay, az, 1.0f);
+    if (!sg.last) { acc[3 * (size_t)px] = ax; acc[3 * (size_t)px + 1] = ay; acc[3 * (size_t)px + 2] = az; }
+    else if (sg.film_out) sg.film_out[px] = make_float4(ax, ay, az, 1.0f);
 }
 
 __global__ void k_zero(float* p, size_t n) {
@@ -2244,7 +2256,7 @@ __global__ void __launch_bounds__(256) k_atrous(const float4* in, const float4* 
 // ---------------------------------------------------------------------------
 // host drivers
 // ---------------------------------------------------------------------------
-static int num_cus(srt_ctx* c) {
+int num_cus(srt_ctx* c) {
     static int cached = -1;
     if (cached < 0) {
         hipDeviceProp_t prop;
@@ -2290,10 +2302,11 @@ static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr) {
     const TraceCfg cfg = trace_cfg(c, nullptr);
     int per_cu = c->trace_blocks_per_cu;
     if (per_cu <= 0) {
-        int nb = 0;
         if (!kernel) kernel = reinterpret_cast<const void*>(k_trace<false, true>);
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kTraceBlock, trace_lds_bytes(cfg)) != hipSuccess ||
-            nb <= 0)
+        int& nb = c->occupancy[{kernel, trace_lds_bytes(cfg)}];      // asked once per kernel and LDS size
+        if (nb <= 0 &&
+            (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kTraceBlock, trace_lds_bytes(cfg)) != hipSuccess ||
+             nb <= 0))
             nb = 8;
         per_cu = nb;
     }
@@ -2387,8 +2400,9 @@ DevCamera make_camera(const float pos[3], const float target[3], const float up[
 
 __global__ void __launch_bounds__(256) k_scatter_train(int n, const uint32_t* flag, const uint32_t* pos, int64_t base,
                                                        int64_t cap, const float* rec_in9, const float* tgt, float* out_in9,
-                                                       float* out_t) {
+                                                       float* out_t, uint32_t* host_count) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == n - 1) __hip_atomic_store(host_count, pos[i] + flag[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (i >= n || !flag[i]) return;
     int64_t j = base + pos[i];
     if (j >= cap) return;
@@ -2476,9 +2490,9 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     const size_t tlds = trace_lds_bytes(tcfg);
     if (!c->segbuf.p) if (int r = dev_alloc(c, c->segbuf, sizeof(Segment) * kMaxSegments)) return r;
     hipStream_t st = c->stream;
-    // the segment table is small; a synchronous copy keeps the host array free
-    if (int r = hip_check(c, hipMemcpyAsync(c->segbuf.p, segs_host, sizeof(Segment) * nseg, hipMemcpyHostToDevice, st), "segments"))
-        return r;
+    if (nseg > 1)       // (a lone segment travels as a kernel argument)
+        if (int r = hip_check(c, hipMemcpyAsync(c->segbuf.p, segs_host, sizeof(Segment) * nseg, hipMemcpyHostToDevice, st), "segments"))
+            return r;
     const Segment* segs = (const Segment*)c->segbuf.p;
     MlpIO mio{};
     if (mlp_mode != 0) {
@@ -2519,15 +2533,18 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     hipEvent_t ev;
     // the first bounce's queue is the slots (its trace and shade stages compute
     // each path's camera ray and state); only its partition sizes are set here
-    k_path_counts<<<1, 4 * kParts, 0, st>>>((uint32_t)n, cap, counts);
+    k_chunk_begin<<<1, 4 * kParts, 0, st>>>((uint32_t)n, cap, counts, segs_host[0], (Segment*)c->segbuf.p, nseg == 1, totals,
+                                            nseg == 1 && segs_host[0].path_begin == 0);
     if (max_depth == 0)                   // no shade stage sets the radiance
         for (float* L : {Lr, Lg, Lb}) k_zero<<<nblk, 256, 0, st>>>(L, (size_t)n);
-    if (mlp_mode == 2) k_zero<<<nblk, 256, 0, st>>>((float*)mio.rec_valid, (size_t)n);
+    const int packet0 = c->count_visits ? 0 : trace_packet_ok(c, s, tcfg);     // camera rays as packets
+    if (mlp_mode == 2 && (n > whole || packet0))                               // (whole paths clear their own)
+        k_zero<<<nblk, 256, 0, st>>>((float*)mio.rec_valid, (size_t)n);
     for (int depth = 0; depth < max_depth && npaths > 0; depth++) {
         int qi = depth & 1;
         const bool cam = depth == 0;
         const bool cnt = c->count_visits;
-        const int packet = cam && !cnt ? trace_packet_ok(c, s, tcfg) : 0;
+        const int packet = cam ? packet0 : 0;
         if (npaths <= whole && !packet) {      // the rest of every path in one launch
             prof_begin(c, "paths", &ev);
             float* snap = mlp_mode == 2 && depth <= 1 ? (float*)c->mlpbuf[7].p : nullptr;
@@ -2620,20 +2637,19 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
         if (int r = hip_check(c, hipcub::DeviceScan::ExclusiveSum(c->scan_tmp.p, tbytes, flag, pos, (int)n, st), "scan"))
             return r;
         k_scatter_train<<<nblk, 256, 0, st>>>((int)n, flag, pos, train->count, train->cap, mio.rec_in9, snap_t, train->in9,
-                                              train->target);
-        uint32_t lastpos = 0, lastflag = 0;
-        if (int r = hip_check(c, hipMemcpyAsync(&lastpos, pos + n - 1, 4, hipMemcpyDeviceToHost, st), "count")) return r;
-        if (int r = hip_check(c, hipMemcpyAsync(&lastflag, flag + n - 1, 4, hipMemcpyDeviceToHost, st), "count")) return r;
-        if (int r = hip_check(c, hipStreamSynchronize(st), "train samples")) return r;
-        train->count = std::min<int64_t>(train->cap, train->count + lastpos + lastflag);
+                                              train->target, c->live + 1);
     }
     int maxwh = 0;
     for (int k = 0; k < nseg; k++) maxwh = std::max(maxwh, (int)segs_host[k].wh);
     prof_begin(c, "finalize", &ev);
-    k_finalize<<<dim3((unsigned)((maxwh + 255) / 256), (unsigned)nseg), 256, 0, st>>>(Lr, Lg, Lb, segs, counts, totals);
+    k_finalize<<<dim3((unsigned)((maxwh + 255) / 256), (unsigned)nseg), 256, 0, st>>>(Lr, Lg, Lb, segs, counts, totals,
+                                                                                             c->host_totals);
     prof_end(c, "finalize", ev, maxwh);
     // the host segment array may be reused by the caller after this returns
-    return hip_check(c, hipStreamSynchronize(st), "chunk");
+    if (int r = hip_check(c, hipStreamSynchronize(st), "chunk")) return r;
+    if (mlp_mode == 2 && train && train->count < train->cap)
+        train->count = std::min<int64_t>(train->cap, train->count + __atomic_load_n(c->live + 1, __ATOMIC_SEQ_CST));
+    return SRT_OK;
 }
 
 int render_wavefront(srt_ctx* c, SceneRec* s, const DevCamera& cam, const DevParams& p, float* film_dev, TrainOut* train) {
@@ -2646,13 +2662,6 @@ int render_wavefront(srt_ctx* c, SceneRec* s, const DevCamera& cam, const DevPar
         dev_free(c, c->film_acc);
         if (dev_alloc(c, c->film_acc, (size_t)wh * 3 * sizeof(float))) return SRT_E_OOM;
         c->film_pixels = wh;
-    }
-    hipStream_t st = c->stream;
-    unsigned long long* totals = (unsigned long long*)((char*)c->counters.p + kTotalsOffset);
-    {
-        size_t n3 = (size_t)wh * 3;
-        k_zero<<<(unsigned)((n3 + 255) / 256), 256, 0, st>>>((float*)c->film_acc.p, n3);
-        k_zero<<<1, 64, 0, st>>>((float*)totals, 16);
     }
     if (train) train->count = 0;
     Segment sg;
@@ -2670,9 +2679,8 @@ int render_wavefront(srt_ctx* c, SceneRec* s, const DevCamera& cam, const DevPar
         if (int r = run_chunk(c, s, &sg, 1, train)) return r;
     }
     if (int r = hip_check(c, hipGetLastError(), "render launch")) return r;
-    unsigned long long tot[6] = {0, 0, 0, 0, 0, 0};
-    if (int r = hip_check(c, hipMemcpyAsync(tot, totals, sizeof(tot), hipMemcpyDeviceToHost, st), "counters")) return r;
-    if (int r = hip_check(c, hipStreamSynchronize(st), "render")) return r;
+    // (run_chunk waited for the stream: the last chunk's finalize has written the totals)
+    const unsigned long long* tot = c->host_totals;
     c->last_segments = (int64_t)tot[0];
     c->last_shadow_rays = (int64_t)tot[1];
     for (int k = 0; k < 4; k++) c->last_visits[k] = (int64_t)tot[2 + k];
