@@ -63,6 +63,7 @@ struct TraceCfg {
     int32_t inner_exit;  // leave the inner-node loop once at most this many lanes still search a leaf
     int32_t packet;      // > 0: each wave traverses its 64 rays as one packet (coherent camera rays),
                          // testing postponed leaves once this many lanes hold one
+    int32_t deal;        // first bounce: the slots are dealt to the pieces (CamView)
 };
 
 // ---------------------------------------------------------------------------
@@ -202,8 +203,8 @@ struct ShadowQueue {
 // partitions with a size counter each: partition p holds entries
 // [p cap, p cap + size_p), cap = part_cap(chunk paths).  A stage reads its
 // input queue as the concatenation of the partitions, cut into kParts
-// contiguous pieces of equal length (QueueView): workgroup b works on piece
-// b mod kParts and appends what it produces to partition b mod kParts of the
+// contiguous pieces of equal length (QueueView): a workgroup works on piece
+// my_part() and appends what it produces to the partition of that number of the
 // next queue.  The appends of a stage thus spread over kParts counters, the
 // pieces keep the work balanced and spatially coherent (camera paths fill the
 // partitions in slot order), and no partition can outgrow cap: a piece holds

@@ -120,8 +120,19 @@ SRT_D int wave_append(bool pred, uint32_t* counter) {
 SRT_D void clear_parts(uint32_t* first) {
     if (threadIdx.x < (unsigned)kParts) first[threadIdx.x * kCntLine] = 0u;
 }
-// Partition of this workgroup in a partitioned queue (grid: a multiple of kParts)
-SRT_D uint32_t my_part() { return blockIdx.x % (uint32_t)kParts; }
+// Partition of this workgroup in a partitioned queue, and its index among the
+// partition's workgroups (grid: a multiple of kParts).  Consecutive workgroups
+// run on the 8 XCDs in turn: where the grid allows, each partition gets
+// workgroups of every XCD (kXcds consecutive ones), so that a partition with more
+// work than the others is not left to one XCD.  With partition = workgroup
+// mod kParts, the lower half of an image whose upper half is sky (alternate
+// pieces at 16 samples) kept four XCDs busy and four idle.
+constexpr uint32_t kXcds = 8;
+SRT_D bool xcd_spread() { return gridDim.x % (kXcds * (unsigned)kParts) == 0u; }
+SRT_D uint32_t my_part() { return (xcd_spread() ? blockIdx.x / kXcds : blockIdx.x) % (uint32_t)kParts; }
+SRT_D uint32_t my_index() {
+    return xcd_spread() ? blockIdx.x / (kXcds * (unsigned)kParts) * kXcds + blockIdx.x % kXcds : blockIdx.x / (unsigned)kParts;
+}
 
 // One ray's traversal state, kept in registers while its lane walks the BVH.
 struct TravState {
@@ -512,27 +523,139 @@ SRT_D bool trav_pend_any(const DevScene& S, TravState& st, const TravStack& k, b
     return false;
 }
 
+// A partitioned queue read as the concatenation of its partitions: prefix[p]
+// entries come before partition p, prefix[kParts] is the total (in LDS).
+struct QueueView {
+    const uint32_t* prefix;
+    uint32_t cap;
+    uint32_t p0;        // partition of the first entry of this workgroup's piece
+    SRT_D void seek(uint32_t lo) {
+        p0 = 0u;
+        while (p0 + 1u < (unsigned)kParts && lo >= prefix[p0 + 1]) ++p0;
+    }
+    // queue entry of concatenated index j (prefix[p0] <= j < total)
+    SRT_D uint32_t entry(uint32_t j) const {
+        uint32_t p = p0;
+        while (j >= prefix[p + 1]) ++p;
+        return p * cap + (j - prefix[p]);
+    }
+};
+// Workgroup prologue, run by all its threads: the prefix sums of the kParts
+// size counters at counts[cnt] into lds[0..kParts], and this workgroup's piece
+// [lo, hi) of the concatenation (piece blockIdx mod kParts of kParts equal ones).
+SRT_D QueueView queue_piece(const uint32_t* counts, int cnt, uint32_t cap, uint32_t* lds, uint32_t& lo, uint32_t& hi) {
+    if (threadIdx.x < 64u) {
+        uint32_t v = threadIdx.x < (unsigned)kParts ? counts[cnt + threadIdx.x * kCntLine] : 0u;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t t = __shfl_up(v, d);
+            if ((int)threadIdx.x >= d) v += t;
+        }
+        if (threadIdx.x < (unsigned)kParts) lds[threadIdx.x + 1] = v;
+        if (threadIdx.x == 0) lds[0] = 0u;
+    }
+    __syncthreads();
+    const uint32_t total = lds[kParts];
+    const uint32_t piece = my_part();
+    lo = (uint32_t)((uint64_t)total * piece / kParts);
+    hi = (uint32_t)((uint64_t)total * (piece + 1u) / kParts);
+    QueueView v{lds, cap, 0u};
+    v.seek(lo);
+    return v;
+}
+struct IdentityEntry {
+    SRT_D uint32_t entry(uint32_t j) const { return j; }
+};
+// The first bounce's queue (entry = slot).  A piece of fewer paths than the
+// image has pixels is a band of the image, and the workgroups of the bands that
+// hold the geometry run on alone when the others are done; such chunks are
+// dealt (TraceCfg.deal): runs of 2^shift slots go to the pieces in turn, piece p's
+// share holding run 32 r + (p + a mixed turn of r) mod 32 of every round r (the
+// turns keep a piece from meeting the same image columns in every round when
+// the width is a power of two: without them Cornell 256x256x16 took 0.56 ms
+// instead of 0.40).  What does not fill a round keeps its place.  Runs of 512
+// slots (8 tiles) keep neighbouring tiles together in this and the next queues;
+// frames too small for 16 runs a piece take shorter ones.
+// Dealt / in slot order: tube 1280x720x16 2.98 / 3.27 ms, 1M triangles
+// 1280x720x1 1.52 / 1.58, MLP training frame 256x256x8 0.575 / 0.625, Cornell
+// 256x256x16 0.40 / 0.38; chunks of 32 sample planes or more, whose pieces are
+// whole planes, lose their order for nothing: 1920x1080x64 60.9 / 59.3.
+struct CamView {
+    uint32_t per, shift;      // runs per piece
+    SRT_D uint32_t entry(uint32_t j) const {
+        const uint32_t run = j >> shift;
+        const uint32_t p = per ? run / per : (uint32_t)kParts;
+        if (p >= (uint32_t)kParts) return j;
+        const uint32_t r = run - p * per;
+        const uint32_t turn = (r * 0x9E3779B1u) >> 27;        // 0 .. kParts - 1, mixed
+        return ((r * (uint32_t)kParts + ((p + turn) % (uint32_t)kParts)) << shift) + (j & ((1u << shift) - 1u));
+    }
+};
+SRT_D CamView cam_view(uint32_t n, int deal) {
+    n = __builtin_amdgcn_readfirstlane(n);
+    CamView v;
+    v.shift = n >= (uint32_t)kParts * 16u * 512u ? 9u : (n >= (uint32_t)kParts * 16u * 64u ? 6u : 0u);
+    v.per = deal ? (n >> v.shift) / (uint32_t)kParts : 0u;
+    return v;
+}
+// Hands a wave the entries of its workgroup's piece: piece `p` of np equal
+// pieces of `total` positions, each with a fetch counter of its own (one line
+// apart at `counters`, so the atomics of the pieces do not wait for each other).
+// Waves stay with their piece: moving on to other pieces' entries once it was
+// used up cost 5 % of the 1M-triangle frame (with looks at all the counters
+// 8 %: reads of a line that the whole GPU changes are serialised as its atomics
+// are, 50 us per launch for 6144 waves), since the pieces hold like shares of
+// the image (CamView) and the extra rays start a launch's tail anew.
+template <class View>
+struct Feeder {
+    View view;
+    uint32_t* counter;
+    uint32_t lo, hi;
+    SRT_D Feeder(const View& v, uint32_t* counters, uint32_t total, uint32_t np, uint32_t p)
+        : view(v), counter(counters + p * kCntLine), lo((uint32_t)((uint64_t)total * p / np)),
+          hi((uint32_t)((uint64_t)total * (p + 1u) / np)) {}
+    // For the whole wave at once: an entry for every lane that wants one; false
+    // where the piece has none left.
+    SRT_D bool take(bool want, uint32_t& entry) {
+        const unsigned long long m = __ballot(want);
+        if (m == 0ull) return false;
+        const int lane = __lane_id();
+        const int leader = __ffsll(m) - 1;
+        uint32_t base = 0;
+        if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
+        base = __shfl(base, leader);
+        const uint32_t idx = lo + base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        if (!want || idx >= hi) return false;
+        entry = view.entry(idx);
+        return true;
+    }
+};
+// over a partitioned queue's concatenation (or the first bounce's slots), the
+// counters at counts[cnt]
+template <class View>
+SRT_D Feeder<View> queue_feeder(const View& view, const uint32_t* prefix, uint32_t* counts, int cnt) {
+    return Feeder<View>(view, counts + cnt, prefix[kParts], (uint32_t)kParts, my_part());
+}
+// over a dense array [0, n): min(kParts, grid size) pieces
+SRT_D Feeder<IdentityEntry> dense_feeder(uint32_t n, uint32_t* fetch) {
+    const uint32_t np = gridDim.x < (unsigned)kParts ? gridDim.x : (uint32_t)kParts;
+    return Feeder<IdentityEntry>(IdentityEntry{}, fetch, n, np, blockIdx.x % np);
+}
+
 // Persistent traversal with dynamic ray fetch.  Each lane holds one ray; when
 // at least `refill` lanes of the wave (or all of them) are idle, the wave
-// stores the finished lanes' results and takes that many new ray indices from
-// `fetch` with one atomic, so lanes do not idle while the wave's slowest ray
+// stores the finished lanes' results and takes that many new rays from the
+// feeder with one atomic, so lanes do not idle while the wave's slowest ray
 // finishes, and the stores' appends and memory traffic happen once per refill.
-// The wave works on indices [lo, hi), taken from `fetch` (lo + fetch), of
-// entries view.entry(index); the workgroups of a grid work on separate ranges
-// with separate counters (queue_piece, dense_range), so the fetch atomics
-// spread over lines.
 // IO supplies
 //   void load(uint32_t i, TravState&, int32_t root)
 //   void store(uint32_t i, const TravState&, bool occluded)   (on the storing lanes)
-// Every wave leaves the loop once `fetch` has passed hi - lo and its lanes
-// have finished and stored.
+// Every wave leaves the loop once its piece is used up and its lanes have
+// finished and stored.
 template <bool ANY, bool COUNT, bool WIDE, class IO, class View, bool INST = false>
-SRT_D void trace_persistent(const DevScene& S, const View& view, uint32_t lo, uint32_t hi, uint32_t* fetch, int refill,
-                            const TravStack& k, IO& io, uint32_t& nv, uint32_t& nt) {
+SRT_D void trace_persistent(const DevScene& S, Feeder<View> feed, int refill, const TravStack& k, IO& io, uint32_t& nv,
+                            uint32_t& nt) {
     static_assert(!INST || WIDE, "instanced scenes are traversed in the 4-wide form");
     const int32_t root = WIDE ? S.root4 : S.root;
-    const int lane = __lane_id();
-    const unsigned long long below = (1ull << lane) - 1ull;
     TravState st;
     st.cur_ok = false;
     st.has_pend = false;
@@ -547,20 +670,12 @@ SRT_D void trace_persistent(const DevScene& S, const View& view, uint32_t lo, ui
                 io.store(ri, st, occl);
                 done = false;
             }
-            const int leader = __ffsll(m) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(fetch, (uint32_t)__popcll(m));
-            base = __shfl(base, leader);
-            if (idle) {
-                const uint32_t idx = lo + base + (uint32_t)__popcll(m & below);
-                if (idx < hi) {
-                    ri = view.entry(idx);
-                    has = true;
-                    occl = false;
-                    io.template load<INST>(ri, st, root);
-                } else {
-                    exhausted = true;
-                }
+            if (feed.take(idle, ri)) {
+                has = true;
+                occl = false;
+                io.template load<INST>(ri, st, root);
+            } else if (idle) {
+                exhausted = true;
             }
             act = __ballot(has);
         }
@@ -701,54 +816,6 @@ SRT_D void trace_packet(const DevScene& S, const View& view, uint32_t lo, uint32
         if (valid) io.store(ri, st, false);
         __builtin_amdgcn_wave_barrier();
     }
-}
-
-// A partitioned queue read as the concatenation of its partitions: prefix[p]
-// entries come before partition p, prefix[kParts] is the total (in LDS).
-struct QueueView {
-    const uint32_t* prefix;
-    uint32_t cap;
-    uint32_t p0;        // partition of the first entry of this workgroup's piece
-    // queue entry of concatenated index j (prefix[p0] <= j < total)
-    SRT_D uint32_t entry(uint32_t j) const {
-        uint32_t p = p0;
-        while (j >= prefix[p + 1]) ++p;
-        return p * cap + (j - prefix[p]);
-    }
-};
-// Workgroup prologue, run by all its threads: the prefix sums of the kParts
-// size counters at counts[cnt] into lds[0..kParts], and this workgroup's piece
-// [lo, hi) of the concatenation (piece blockIdx mod kParts of kParts equal ones).
-SRT_D QueueView queue_piece(const uint32_t* counts, int cnt, uint32_t cap, uint32_t* lds, uint32_t& lo, uint32_t& hi) {
-    if (threadIdx.x < 64u) {
-        uint32_t v = threadIdx.x < (unsigned)kParts ? counts[cnt + threadIdx.x * kCntLine] : 0u;
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t t = __shfl_up(v, d);
-            if ((int)threadIdx.x >= d) v += t;
-        }
-        if (threadIdx.x < (unsigned)kParts) lds[threadIdx.x + 1] = v;
-        if (threadIdx.x == 0) lds[0] = 0u;
-    }
-    __syncthreads();
-    const uint32_t total = lds[kParts];
-    const uint32_t piece = my_part();
-    lo = (uint32_t)((uint64_t)total * piece / kParts);
-    hi = (uint32_t)((uint64_t)total * (piece + 1u) / kParts);
-    QueueView v{lds, cap, 0u};
-    while (v.p0 + 1u < (unsigned)kParts && lo >= lds[v.p0 + 1]) ++v.p0;
-    return v;
-}
-struct IdentityEntry {
-    SRT_D uint32_t entry(uint32_t j) const { return j; }
-};
-// A dense array [0, n): workgroup b works on piece b mod P of P = min(kParts,
-// grid size) contiguous pieces, with the piece's counter at fetch + piece lines.
-SRT_D uint32_t* dense_range(uint32_t n, uint32_t* fetch, uint32_t& lo, uint32_t& hi) {
-    const uint32_t np = gridDim.x < (unsigned)kParts ? gridDim.x : (uint32_t)kParts;
-    const uint32_t piece = blockIdx.x % np;
-    lo = (uint32_t)((uint64_t)n * piece / np);
-    hi = (uint32_t)((uint64_t)n * (piece + 1u) / np);
-    return fetch + piece * kCntLine;
 }
 
 // ---------------------------------------------------------------------------
@@ -938,13 +1005,12 @@ SRT_D TravStack make_stack(int32_t* gstack, TraceCfg cfg) {
 // following shade and shadow stages append to or fetch from.  COUNT: also
 // total node visits and triangle tests (an untimed pass used for the
 // algorithmic byte count).
-template <bool COUNT, bool WIDE, bool INST, class IO>
+template <bool COUNT, bool WIDE, bool INST, bool CAM, class IO>
 SRT_D void trace_stage(const DevScene& S, IO& io, uint32_t* counts, int qi, uint32_t cap, int32_t* gstack,
                        unsigned long long* totals, TraceCfg cfg) {
     __shared__ uint32_t prefix[kParts + 1];
     uint32_t lo, hi;
     const QueueView view = queue_piece(counts, cnt_q(qi), cap, prefix, lo, hi);
-    uint32_t* fetch = counts + CNT_FETCH_T + my_part() * kCntLine;
     if (blockIdx.x == 0) {
         clear_parts(counts + CNT_FETCH_S);
         clear_parts(counts + cnt_q(qi ^ 1));
@@ -952,10 +1018,15 @@ SRT_D void trace_stage(const DevScene& S, IO& io, uint32_t* counts, int qi, uint
         clear_parts(counts + CNT_MLPQ_PARTS);
         if (threadIdx.x == 0) counts[CNT_MLPQ] = 0u;
     }
-    if (blockIdx.x < (unsigned)kParts && threadIdx.x == 0) atomicAdd(&totals[0], (unsigned long long)(hi - lo));
+    if (my_index() == 0u && threadIdx.x == 0) atomicAdd(&totals[0], (unsigned long long)(hi - lo));
     const TravStack k = make_stack<INST>(gstack, cfg);
     uint32_t nv = 0, nt = 0;
-    trace_persistent<false, COUNT, WIDE, IO, QueueView, INST>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
+    if constexpr (CAM)
+        trace_persistent<false, COUNT, WIDE, IO, CamView, INST>(
+            S, queue_feeder(cam_view(prefix[kParts], cfg.deal), prefix, counts, CNT_FETCH_T), cfg.refill, k, io, nv, nt);
+    else
+        trace_persistent<false, COUNT, WIDE, IO, QueueView, INST>(S, queue_feeder(view, prefix, counts, CNT_FETCH_T),
+                                                                  cfg.refill, k, io, nv, nt);
     if (COUNT) {
         atomicAdd(&totals[2], (unsigned long long)nv);
         atomicAdd(&totals[3], (unsigned long long)nt);
@@ -966,7 +1037,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace(DevScene S, PathQueue q, 
                                                       uint32_t cap, int32_t* gstack, unsigned long long* totals,
                                                       TraceCfg cfg) {
     QueueIO io{q, h};
-    trace_stage<COUNT, WIDE, INST, QueueIO>(S, io, counts, qi, cap, gstack, totals, cfg);
+    trace_stage<COUNT, WIDE, INST, false, QueueIO>(S, io, counts, qi, cap, gstack, totals, cfg);
 }
 // The first bounce (queue 0): the same, with each camera ray computed from
 // its slot (path_start) instead of read from the queue.
@@ -975,7 +1046,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_cam(DevScene S, const Seg
                                                           uint32_t* counts, uint32_t cap, int32_t* gstack,
                                                           unsigned long long* totals, TraceCfg cfg) {
     CamIO io{segs, nseg, h};
-    trace_stage<COUNT, WIDE, INST, CamIO>(S, io, counts, 0, cap, gstack, totals, cfg);
+    trace_stage<COUNT, WIDE, INST, true, CamIO>(S, io, counts, 0, cap, gstack, totals, cfg);
 }
 
 // Closest hit of the first bounce's camera rays as 64-ray packets
@@ -995,9 +1066,9 @@ __global__ void __launch_bounds__(kTraceBlock) k_trace_packet(DevScene S, const 
         clear_parts(counts + CNT_MLPQ_PARTS);
         if (threadIdx.x == 0) counts[CNT_MLPQ] = 0u;
     }
-    if (blockIdx.x < (unsigned)kParts && threadIdx.x == 0) atomicAdd(&totals[0], (unsigned long long)(hi - lo));
+    if (my_index() == 0u && threadIdx.x == 0) atomicAdd(&totals[0], (unsigned long long)(hi - lo));
     CamIO io{segs, nseg, h};
-    trace_packet<CamIO, QueueView>(S, view, lo, hi, fetch, cfg.lds_depth, cfg.packet, io);
+    trace_packet<CamIO, CamView>(S, cam_view(prefix[kParts], cfg.deal), lo, hi, fetch, cfg.lds_depth, cfg.packet, io);
 }
 
 struct LightSample { f3 pos, normal, emission; float pdf; };
@@ -1336,7 +1407,7 @@ template <bool CAM>
 __global__ void __launch_bounds__(kShadeBlock, 4) k_shade(DevScene S, const Segment* segs, int nseg, int depth,
                                                          PathQueue qin, HitBuf h, PathQueue qout, ShadowQueue sq,
                                                          float* Lr, float* Lg, float* Lb, uint32_t* counts, int qi,
-                                                         uint32_t cap, MlpIO mio) {
+                                                         uint32_t cap, MlpIO mio, int deal) {
     __shared__ uint32_t gather[kShadeBlock / 64][128];
     const int lane = threadIdx.x & 63;
     uint32_t* buf = gather[threadIdx.x >> 6];
@@ -1346,9 +1417,10 @@ __global__ void __launch_bounds__(kShadeBlock, 4) k_shade(DevScene S, const Segm
     __shared__ uint32_t prefix[kParts + 1];
     uint32_t lo, hi;
     const QueueView view = queue_piece(counts, cnt_q(qi), cap, prefix, lo, hi);
+    const CamView cview = cam_view(prefix[kParts], deal);
     const uint32_t part = my_part();
     const uint32_t count = hi - lo;
-    const int wave = (int)((blockIdx.x / (unsigned)kParts) * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    const int wave = (int)(my_index() * (blockDim.x >> 6) + (threadIdx.x >> 6));
     const int nwaves = (int)((gridDim.x / (unsigned)kParts) * (blockDim.x >> 6));
     if (blockIdx.x == 0) clear_parts(counts + CNT_FETCH_T);   // the next trace stage fetches from 0
     const f3 env = mk(S.env[0], S.env[1], S.env[2]);
@@ -1359,7 +1431,7 @@ __global__ void __launch_bounds__(kShadeBlock, 4) k_shade(DevScene S, const Segm
         while (nbuf < 64u && base < count) {
             const uint32_t r = base + (uint32_t)lane;
             const bool valid = r < count;
-            const uint32_t i = valid ? view.entry(lo + r) : 0u;
+            const uint32_t i = !valid ? 0u : (CAM ? cview.entry(lo + r) : view.entry(lo + r));
             const int32_t tri = valid ? h.tri[i] : -1;
             if (valid && tri < 0) {
                 if constexpr (CAM) {
@@ -1412,12 +1484,12 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(DevScene S, ShadowQueue 
     uint32_t lo, hi;
     if (blockIdx.x == 0) report_live(counts, next, live);
     const QueueView view = queue_piece(counts, CNT_SHADOW, cap, prefix, lo, hi);
-    uint32_t* fetch = counts + CNT_FETCH_S + my_part() * kCntLine;
-    if (blockIdx.x < (unsigned)kParts && threadIdx.x == 0) atomicAdd(&totals[1], (unsigned long long)(hi - lo));
+    if (my_index() == 0u && threadIdx.x == 0) atomicAdd(&totals[1], (unsigned long long)(hi - lo));
     const TravStack k = make_stack<INST>(gstack, cfg);
     ShadowIO io{sq, Lr, Lg, Lb};
     uint32_t nv = 0, nt = 0;
-    trace_persistent<true, COUNT, WIDE, ShadowIO, QueueView, INST>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
+    trace_persistent<true, COUNT, WIDE, ShadowIO, QueueView, INST>(S, queue_feeder(view, prefix, counts, CNT_FETCH_S), cfg.refill,
+                                                                   k, io, nv, nt);
     if (COUNT) {
         atomicAdd(&totals[4], (unsigned long long)nv);
         atomicAdd(&totals[5], (unsigned long long)nt);
@@ -1477,11 +1549,13 @@ __global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segm
     uint32_t lo, hi;
     const QueueView view = queue_piece(counts, cnt_q(qi), cap, prefix, lo, hi);
     const uint32_t part = my_part();
-    uint32_t* fetch = counts + CNT_FETCH_T + part * kCntLine;
+    std::conditional_t<CAM, CamView, QueueView> pview;
+    if constexpr (CAM) pview = cam_view(prefix[kParts], cfg.deal);
+    else pview = view;
+    auto feed = queue_feeder(pview, prefix, counts, CNT_FETCH_T);
     const TravStack k = make_stack<INST>(gstack, cfg);
     const f3 env = mk(S.env[0], S.env[1], S.env[2]);
     const int lane = __lane_id();
-    const unsigned long long below = (1ull << lane) - 1ull;
     // a launch with fewer paths than resident lanes spreads them over its waves
     const uint32_t waves = gridDim.x / (unsigned)kParts * (kTraceBlock / 64);
     const uint32_t quota = min(64u, max(1u, (hi - lo + waves - 1u) / waves));
@@ -1545,46 +1619,36 @@ __global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segm
                 }
             }
             const bool want = !has && !exhausted && !start;
-            const unsigned long long m = __ballot(want);
-            if (m != 0ull) {
-                const int leader = __ffsll(m) - 1;
-                uint32_t base = 0;
-                if (lane == leader) base = atomicAdd(fetch, (uint32_t)__popcll(m));
-                base = __shfl(base, leader);
-                if (want) {
-                    const uint32_t idx = lo + base + (uint32_t)__popcll(m & below);
-                    if (idx < hi) {
-                        const uint32_t i = view.entry(idx);
-                        if (CAM) {
-                            const PathStart p = path_start(segs, nseg, i);
-                            slot = i;
-                            if (snap) mio.rec_valid[slot] = 0u;
-                            o = p.o; ndir = p.d;
-                            beta = mk(1.0f);
-                            L = mk(0.0f);
-                            pdf = 1.0f;
-                            flags = p.flags;
-                            rng = p.rng;
-                            depth = 0;
-                        } else {
-                            slot = q.slot[i];
-                            o = mk(q.ox[i], q.oy[i], q.oz[i]); ndir = mk(q.dx[i], q.dy[i], q.dz[i]);
-                            beta = mk(q.br[i], q.bg[i], q.bb[i]);
-                            L = mk(Lr[slot], Lg[slot], Lb[slot]);
-                            pdf = q.pdf[i];
-                            flags = q.flags[i];
-                            rng = q.rng[i];
-                            depth = depth0;
-                        }
-                        d = ndir;
-                        tmax = 1e16f;
-                        shadow = false;
-                        start = true;
-                        nseg_traced++;
-                    } else {
-                        exhausted = true;
-                    }
+            uint32_t i = 0;
+            if (feed.take(want, i)) {
+                if (CAM) {
+                    const PathStart p = path_start(segs, nseg, i);
+                    slot = i;
+                    if (snap) mio.rec_valid[slot] = 0u;
+                    o = p.o; ndir = p.d;
+                    beta = mk(1.0f);
+                    L = mk(0.0f);
+                    pdf = 1.0f;
+                    flags = p.flags;
+                    rng = p.rng;
+                    depth = 0;
+                } else {
+                    slot = q.slot[i];
+                    o = mk(q.ox[i], q.oy[i], q.oz[i]); ndir = mk(q.dx[i], q.dy[i], q.dz[i]);
+                    beta = mk(q.br[i], q.bg[i], q.bb[i]);
+                    L = mk(Lr[slot], Lg[slot], Lb[slot]);
+                    pdf = q.pdf[i];
+                    flags = q.flags[i];
+                    rng = q.rng[i];
+                    depth = depth0;
                 }
+                d = ndir;
+                tmax = 1e16f;
+                shadow = false;
+                start = true;
+                nseg_traced++;
+            } else if (want) {
+                exhausted = true;
             }
             if (start) {
                 trav_begin<INST>(st, o, d, 1e-3f, tmax, S.root4, !shadow);
@@ -1645,7 +1709,7 @@ __global__ void __launch_bounds__(256) k_mlp_compact(uint32_t* counts, uint32_t 
     const QueueView view = queue_piece(counts, CNT_MLPQ_PARTS, cap, prefix, lo, hi);
     if (blockIdx.x == 0 && threadIdx.x == 0) counts[CNT_MLPQ] = prefix[kParts];
     const uint32_t step = (gridDim.x / (unsigned)kParts) * blockDim.x;
-    for (uint32_t r = (blockIdx.x / (unsigned)kParts) * blockDim.x + threadIdx.x; r < hi - lo; r += step) {
+    for (uint32_t r = my_index() * blockDim.x + threadIdx.x; r < hi - lo; r += step) {
         const size_t j = lo + r, e = view.entry(lo + r);
         for (int k = 0; k < 9; k++) mio.q_in9[j * 9 + k] = mio.qs_in9[e * 9 + k];
         for (int k = 0; k < 3; k++) mio.q_beta[j * 3 + k] = mio.qs_beta[e * 3 + k];
@@ -1769,18 +1833,17 @@ template <bool INST = false>
 __global__ void __launch_bounds__(kTraceBlock) k_trace_rays(DevScene S, uint32_t n, RaysIO io, uint32_t* fetch,
                                                            int32_t* gstack, TraceCfg cfg) {
     const TravStack k = make_stack<INST>(gstack, cfg);
-    uint32_t nv = 0, nt = 0, lo, hi;
-    fetch = dense_range(n, fetch, lo, hi);
-    const IdentityEntry view;
+    uint32_t nv = 0, nt = 0;
+    const Feeder<IdentityEntry> feed = dense_feeder(n, fetch);
     if (INST) {
-        if (io.any) trace_persistent<true, false, true, RaysIO, IdentityEntry, true>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
-        else trace_persistent<false, false, true, RaysIO, IdentityEntry, true>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
+        if (io.any) trace_persistent<true, false, true, RaysIO, IdentityEntry, true>(S, feed, cfg.refill, k, io, nv, nt);
+        else trace_persistent<false, false, true, RaysIO, IdentityEntry, true>(S, feed, cfg.refill, k, io, nv, nt);
     } else if (cfg.wide) {
-        if (io.any) trace_persistent<true, false, true>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
-        else trace_persistent<false, false, true>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
+        if (io.any) trace_persistent<true, false, true>(S, feed, cfg.refill, k, io, nv, nt);
+        else trace_persistent<false, false, true>(S, feed, cfg.refill, k, io, nv, nt);
     } else {
-        if (io.any) trace_persistent<true, false, false>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
-        else trace_persistent<false, false, false>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
+        if (io.any) trace_persistent<true, false, false>(S, feed, cfg.refill, k, io, nv, nt);
+        else trace_persistent<false, false, false>(S, feed, cfg.refill, k, io, nv, nt);
     }
 }
 
@@ -1810,10 +1873,8 @@ template <bool WIDE, bool INST>
 __global__ void __launch_bounds__(kTraceBlock) k_simple_trace(DevScene S, uint32_t n, SimpleIO io, uint32_t* fetch,
                                                              int32_t* gstack, TraceCfg cfg) {
     const TravStack k = make_stack<INST>(gstack, cfg);
-    uint32_t nv = 0, nt = 0, lo, hi;
-    fetch = dense_range(n, fetch, lo, hi);
-    trace_persistent<false, false, WIDE, SimpleIO, IdentityEntry, INST>(S, IdentityEntry{}, lo, hi, fetch, cfg.refill, k,
-                                                                        io, nv, nt);
+    uint32_t nv = 0, nt = 0;
+    trace_persistent<false, false, WIDE, SimpleIO, IdentityEntry, INST>(S, dense_feeder(n, fetch), cfg.refill, k, io, nv, nt);
 }
 
 // the Simple pass types (SimpleParams::Type, params/npr_params.h)
@@ -1944,7 +2005,7 @@ __global__ void __launch_bounds__(256) k_lt_shade(DevScene S, LtParams P, int de
     const f3 cam_pos = ld3(P.cam.pos);
     const int64_t wh = (int64_t)P.width * P.height;
     const uint32_t step = (gridDim.x / (unsigned)kParts) * blockDim.x;
-    for (uint32_t r = (blockIdx.x / (unsigned)kParts) * blockDim.x + threadIdx.x; r < hi - lo; r += step) {
+    for (uint32_t r = my_index() * blockDim.x + threadIdx.x; r < hi - lo; r += step) {
         const uint32_t i = view.entry(lo + r);
         const f3 ro = mk(qin.ox[i], qin.oy[i], qin.oz[i]), rd = mk(qin.dx[i], qin.dy[i], qin.dz[i]);
         f3 beta = mk(qin.br[i], qin.bg[i], qin.bb[i]);
@@ -2055,11 +2116,11 @@ __global__ void __launch_bounds__(kTraceBlock) k_lt_shadow(DevScene S, ShadowQue
     __shared__ uint32_t prefix[kParts + 1];
     uint32_t lo, hi;
     const QueueView view = queue_piece(counts, CNT_SHADOW, cap, prefix, lo, hi);
-    uint32_t* fetch = counts + CNT_FETCH_S + my_part() * kCntLine;
     const TravStack k = make_stack<INST>(gstack, cfg);
     LtShadowIO io{sq, film};
     uint32_t nv = 0, nt = 0;
-    trace_persistent<true, false, WIDE, LtShadowIO, QueueView, INST>(S, view, lo, hi, fetch, cfg.refill, k, io, nv, nt);
+    trace_persistent<true, false, WIDE, LtShadowIO, QueueView, INST>(S, queue_feeder(view, prefix, counts, CNT_FETCH_S),
+                                                                     cfg.refill, k, io, nv, nt);
 }
 
 __global__ void __launch_bounds__(256) k_film_clear(float4* film, int64_t n) {
@@ -2280,6 +2341,7 @@ static TraceCfg trace_cfg(srt_ctx* c, const SceneRec* s) {
     cfg.wide = use_wide(c, s) ? 1 : 0;
     cfg.inner_exit = c->trace_inner_exit;
     cfg.packet = 0;
+    cfg.deal = 0;
     return cfg;
 }
 // Packet traversal of a launch's camera rays (TraceCfg.packet: the number of
@@ -2297,7 +2359,11 @@ static size_t trace_lds_bytes(const TraceCfg& cfg, bool inst = false) {
 }
 
 // Persistent traversal grid: as many workgroups as are resident at once
-// (occupancy of the traversal kernel with its LDS stack), capped by the work.
+// (occupancy of the traversal kernel with its LDS stack), at most 6 waves per
+// SIMD, capped by the work.  A seventh wave (a kernel of 72 VGPRs or fewer)
+// costs more in the caches than it hides: 37.6 against 35.9 ms of closest
+// hits on the 1M-triangle frame.
+constexpr int kTraceBlocksPerCu = 6 * 4 * 64 / kTraceBlock;
 static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr) {
     const TraceCfg cfg = trace_cfg(c, nullptr);
     int per_cu = c->trace_blocks_per_cu;
@@ -2308,7 +2374,7 @@ static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr) {
             (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kTraceBlock, trace_lds_bytes(cfg)) != hipSuccess ||
              nb <= 0))
             nb = 8;
-        per_cu = nb;
+        per_cu = std::min(nb, kTraceBlocksPerCu);
     }
     int64_t want = (n + kTraceBlock - 1) / kTraceBlock;
     int64_t cap = (int64_t)num_cus(c) * per_cu;
@@ -2434,6 +2500,7 @@ static int ensure_mlp_bufs(srt_ctx* c, int64_t slots) {
 // 0.403 / 0.407, 256x256x64 with the MLP 0.740 / 0.717 / 0.770 / 0.817,
 // 512x512x16 (4.2M paths, all of them at once) 0.87 against 1.04.
 constexpr int64_t kWholePathMax = 1 << 20;
+constexpr int64_t kPathSpread = 32;      // workgroups per 128 paths that k_paths may use
 
 // Waits for the size of the next bounce's queue (report_live), which arrives
 // once the bounce's shading is done, while its shadow rays are still traced:
@@ -2478,10 +2545,15 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     const int pgrid = part_grid(trace_grid(c, n, reinterpret_cast<const void*>(k_trace_packet)));
     const uint32_t cap = part_cap((uint32_t)n);
     const bool inst = s->ninst > 0;
-    const int wgrid = part_grid(trace_grid(c, n, inst ? reinterpret_cast<const void*>(k_paths<true, true>)
-                                                      : reinterpret_cast<const void*>(k_paths<true, false>)));
+    // few paths are spread over more waves (k_paths' quota): the lanes of a wave
+    // wait for each other at every branch, and the chip has waves to spare.  1M
+    // triangles 64x64x1 depth 8: 0.84 ms with 64 paths per wave, 0.40 with 2 or
+    // less; Cornell 64x64x4 0.196 -> 0.171
+    const int wgrid = part_grid(trace_grid(c, n * kPathSpread, inst ? reinterpret_cast<const void*>(k_paths<true, true>)
+                                                                    : reinterpret_cast<const void*>(k_paths<true, false>)));
     if (int r = ensure_gstack(c, s, (int64_t)std::max(tgrid, wgrid) * kTraceBlock)) return r;
-    const TraceCfg tcfg = trace_cfg(c, s);
+    TraceCfg tcfg = trace_cfg(c, s);
+    for (int k = 0; k < nseg; k++) tcfg.deal |= n < (int64_t)kParts * segs_host[k].wh ? 1 : 0;
     const int64_t whole = tcfg.wide && !c->count_visits ? kWholePathMax : 0;
     int64_t npaths = n;                   // live paths of the bounce
     uint32_t* live = c->live;
@@ -2587,9 +2659,9 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
         prof_end(c, "trace", ev, 0);
         prof_begin(c, "shade", &ev);
         if (cam)
-            k_shade<true><<<shade_grid, 256, 0, st>>>(S, segs, nseg, depth, Q[qi], H, Q[qi ^ 1], SQ, Lr, Lg, Lb, counts, qi, cap, mio);
+            k_shade<true><<<shade_grid, 256, 0, st>>>(S, segs, nseg, depth, Q[qi], H, Q[qi ^ 1], SQ, Lr, Lg, Lb, counts, qi, cap, mio, tcfg.deal);
         else
-            k_shade<false><<<shade_grid, 256, 0, st>>>(S, segs, nseg, depth, Q[qi], H, Q[qi ^ 1], SQ, Lr, Lg, Lb, counts, qi, cap, mio);
+            k_shade<false><<<shade_grid, 256, 0, st>>>(S, segs, nseg, depth, Q[qi], H, Q[qi ^ 1], SQ, Lr, Lg, Lb, counts, qi, cap, mio, 0);
         prof_end(c, "shade", ev, 0);
         __atomic_store_n(live, kNotYet, __ATOMIC_SEQ_CST);
         if (!any_nee) {

@@ -259,3 +259,27 @@ def test_whole_path_kernel_equals_queue_stages(ctx, name, W, H, spp, depth):
     ctx.release(h)
     assert np.array_equal(out[0][0], out[1][0])
     assert out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("W,H,spp", [(8, 8, 1), (61, 37, 1), (160, 57, 1), (311, 170, 5), (640, 411, 2), (97, 61, 40)])
+def test_dealt_slots_cover_every_path(ctx, W, H, spp):
+    """Chunks of fewer than 32 sample planes deal their slots to the queue's
+    pieces in runs of 1, 64 or 512: every path is traced once whatever the
+    remainder (queue stages by visit counting), and the image is the whole-path
+    kernel's and, for small frames, the oracle's."""
+    s = scenes.cornell()
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    ctx.set_option("count_visits", 1)
+    a = ctx.render(h, s.camera, W, H, spp, 3, 4, 1, 1, 13)
+    na = ctx.last_counts()
+    ctx.set_option("count_visits", 0)
+    b = ctx.render(h, s.camera, W, H, spp, 3, 4, 1, 1, 13)
+    nb = ctx.last_counts()
+    ctx.release(h)
+    assert na == nb and na[0] >= W * H * spp
+    assert np.array_equal(a, b)
+    if W * H * spp < 20000:
+        osc = O.Scene(s)
+        ref, _ = O.render(osc, s.camera, W, H, spp, 3, 4, 1, 1, 13, bvh=O.Bvh(osc))
+        assert _rel(a[:, :3], ref[:, :3]).max() <= TOL
