@@ -43,6 +43,28 @@ def test_small_soups(ctx, n):
     _compare(ctx, _soup(n, seed=n))
 
 
+@pytest.mark.parametrize("n", [255, 257, 4096, 4097, 4098, 8193, 12290])
+def test_pieces_of_the_level_order(ctx, n):
+    """Radix trees and binary trees whose node counts lie around a multiple of
+    the level order's pieces (4096 nodes, 256 threads): the tree equals the
+    oracle's, and the closest hits found through its 4-wide form equal those of
+    the oracle's tree."""
+    s = _soup(n, seed=n)
+    _compare(ctx, s)
+    rng = np.random.default_rng(n)
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    o = rng.uniform(-12, 12, size=(512, 3))
+    d = rng.normal(size=(512, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    got = ctx.trace(h, o, d)
+    ctx.release(h)
+    osc = O.Scene(s)
+    want = O.trace(osc, o, d, bvh=O.Bvh(osc))
+    assert np.array_equal(got[3], want[3])
+    assert np.array_equal(got[0], want[0])
+
+
 @pytest.mark.parametrize("cluster", [8, 16, 100])
 def test_top_level_sah(ctx, cluster):
     info = _compare(ctx, _soup(5000, seed=9), cluster_size=cluster)
