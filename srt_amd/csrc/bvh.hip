@@ -252,9 +252,10 @@ __global__ void __launch_bounds__(256) k_level_scan(int pieces, int32_t* hist, i
     }
     if (tid == 0) size[blockIdx.x] = run;
 }
+// `ids`: node at each position; `number`: position of each node (or null);
 // `first`: first position of every level, kLevels + 1 entries
 __global__ void __launch_bounds__(256) k_level_rank(int n, const uint8_t* key, int pieces, const int32_t* hist,
-                                                    const int32_t* size, uint32_t* ids, int32_t* first) {
+                                                    const int32_t* size, uint32_t* ids, int32_t* number, int32_t* first) {
     __shared__ int32_t s_w[4];
     __shared__ int32_t s_next[4][kLevels];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -294,7 +295,10 @@ __global__ void __launch_bounds__(256) k_level_rank(int n, const uint8_t* key, i
             __builtin_amdgcn_wave_barrier();      // the next match may be of the same level
             todo &= ~same;
         }
-        if (k >= 0) ids[at] = (uint32_t)i;
+        if (k >= 0) {
+            ids[at] = (uint32_t)i;
+            if (number) number[i] = at;
+        }
     }
 }
 // Depth of radix-tree node i below the root (node 0)
@@ -394,10 +398,47 @@ SRT_D void set_child(BvhNode* nd, int side, const DBox& b, int32_t ref) {
 }
 
 // ---------------------------------------------------------------------------
-// 6. top-level binned SAH, one workgroup, breadth-first
+// 6. top-level binned SAH over the clusters, breadth-first
 // ---------------------------------------------------------------------------
-constexpr int kTopThreads = 1024;
+// A split of a node's item range [b, e) at `mid` is the only one with this
+// boundary in the whole tree, so the node's record is kept under its boundary
+// and needs no number until the end: nodes are numbered breadth-first, left
+// before right, which is the order of (level, boundary), one counting sort.
+// No level therefore waits for the number of nodes of the one before it, and
+// the host reads nothing until all are split.  A node's split depends only on
+// its own items, so the tree is the one a sequential build produces.
+//   wide levels  (the first ones, where every node has thousands of items):
+//                chunks of kWideChunk items bin into their node's accumulators,
+//                one wave per node chooses the split, the chunks partition
+//   middle levels: one launch per level; a node of more than kBlockItems items
+//                is split by a workgroup, one of more than kSmallItems by a wave
+//   small nodes  (two to kSmallItems items): one wave builds the whole subtree
+//                in LDS
+// Items are read from it[level & 1] and written, partitioned, to the other.
+// Lane 16 a + k of a wave holds bin k of axis a when a split is chosen; the
+// boxes and centroid bounds of a node's children are unions of bins, so a level
+// reads its items once to bin and once to partition them.
+// Before, per level: bounds, bins by LDS atomics, partition, child boxes, a
+// scan that numbered the children and a wait for their count, with one wave
+// per node down to two items: 3.0 ms of the 4.7 ms of a rebuild of the
+// 1M-triangle field (347 thousand clusters, 26 levels); now 1.1 ms.
 constexpr int kBins = 16;
+constexpr int kTopWaves = 4;           // waves of a workgroup
+// 3 axes x 21 items are one wave's split candidates
+constexpr int kSmallItems = 21;
+// four waves share a node that one would work on for more than four rounds of 64
+// items: a rebuild of the 1M-triangle field takes 3.00 ms, 3.04 ms with a line at 128 or at 512
+constexpr int kBlockItems = 256;
+// A wide level of the 1M-triangle field takes 35 us whatever its nodes' sizes, a
+// level of middle nodes as long as its largest node: with seven wide levels
+// instead of nine (1300 items per node on average) the rebuild takes 3.09 ms.
+constexpr int kWideLevels = 9;
+constexpr int kWideMin = 1024;         // items per node on average down to which levels are wide
+constexpr int kWideChunk = 512;        // two rounds of a wave's 64 items
+constexpr int kWideCopies = 8;         // accumulators of a node: chunks of a node share an address eight times less
+constexpr int kRegions = 64;           // small nodes are listed by region of the items, each with its own counter
+constexpr int kRegionBlocks = 32;       // two workgroups a SIMD
+constexpr int kAccWords = 14;          // box lo xyz, hi xyz, centroid lo xyz, hi xyz (keys), triangles, items
 
 SRT_D int bin_of(float c, float lo, float scale) {
     int bi = (int)((c - lo) * scale);
@@ -412,738 +453,705 @@ SRT_D void copy_item(const Items& s, int i, const Items& d, int j) {
     d.cx[j] = s.cx[i]; d.cy[j] = s.cy[i]; d.cz[j] = s.cz[i];
     d.count[j] = s.count[i]; d.ref[j] = s.ref[i];
 }
-
-// Level-parallel form: one workgroup per node of a level finds its split and
-// partitions its item range in place (stable: left items, then right items,
-// each in their previous order); k_top_link then numbers the inner children of
-// the level in order (breadth-first numbering, left before right) and writes
-// the parents' child boxes and refs.  Each node's split depends only on its own
-// items, so the tree is the one a sequential breadth-first build produces.
-struct TopSplit {
-    int32_t mid;
-    float box[2][6];        // child boxes: lo xyz, hi xyz
-};
-constexpr int kSplitThreads = 256;
-static_assert(kSplitThreads == 256, "k_top_split ranks items four waves at a time");
-// min / max of ordered float keys over the 64 lanes of a wave (every lane gets them)
+SRT_D void wave_sync() {      // LDS of one wave: its accesses stay in order, the compiler must keep them so
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// word q of an accumulator: identity, union
+SRT_D uint32_t acc_empty(int q) {
+    return q >= 12 ? 0u : (q % 6 < 3 ? fkey(__builtin_huge_valf()) : fkey(-__builtin_huge_valf()));
+}
+SRT_D uint32_t acc_union(int q, uint32_t x, uint32_t y) { return q >= 12 ? x + y : (q % 6 < 3 ? min(x, y) : max(x, y)); }
+// the value of the lane CTRL names within a row of 16 lanes, `old` where there is none
+template <int CTRL> SRT_D uint32_t row_get(uint32_t old, uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, 0xf, 0xf, false);
+}
+constexpr int kRowShl = 0x100, kRowShr = 0x110;       // + lanes
+// a value that is the same in all lanes, held in a scalar register: loops over it need no per-lane exit
+SRT_D int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+SRT_D uint32_t read_lane(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
+// minimum over the wave, in every lane
 SRT_D uint32_t wave_min_u32(uint32_t v) {
-    for (int off = 32; off > 0; off >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, off));
+    v = min(v, row_get<kRowShr + 1>(~0u, v));
+    v = min(v, row_get<kRowShr + 2>(~0u, v));
+    v = min(v, row_get<kRowShr + 4>(~0u, v));
+    v = min(v, row_get<kRowShr + 8>(~0u, v));
+    return min(min(read_lane(v, 15), read_lane(v, 31)), min(read_lane(v, 47), read_lane(v, 63)));
+}
+
+struct alignas(16) TopTask {
+    int32_t b, e;           // items; e == b: none
+    int32_t up;             // 2 * parent's boundary + side, 0 for the root
+    uint32_t cb[6];         // centroid bounds (keys): lo xyz, hi xyz
+};
+struct SmallTask {
+    int32_t b, e, up, level;
+};
+// A child is another node (its boundary, written when that node is split), a
+// given ref, or the item at a position of it[0] or it[1].
+constexpr int kChildNode = 0, kChildRef = 1, kChildItem = 2;
+struct alignas(64) TopRec {
+    float box[2][6];        // child boxes: lo xyz, hi xyz
+    int32_t child[2];
+    int32_t kind[2];
+};
+struct WideSplit {
+    int32_t axis, split, mid;
+    float lo, scale;
+};
+struct TopBuild {
+    int m;                  // items
+    int wide_levels;
+    Items it[2];
+    TopRec* rec;            // by boundary, 1 .. m - 1
+    uint8_t* level;         // of boundary p at p - 1
+    TopTask* wide[2];       // 2^L slots: the children of slot t are 2 t and 2 t + 1
+    TopTask* mid[2];        // slot of a node: the multiple of kSmallItems + 1 in its range, see mid_slot
+    SmallTask* small;       // by regions
+    int32_t* nsmall;        // per region, 256 bytes apart
+    int32_t* any;           // [L]: level L has middle nodes
+    uint32_t* cb;           // centroid bounds of all items (keys)
+    uint32_t* acc;          // wide nodes' accumulators [slot][copy][word][lane 0 .. 47]
+    int32_t* chunk_items;   // items per chunk and lane (bin) of a wide level
+    WideSplit* wsplit;
+};
+// Nodes of a level are disjoint ranges of more than kSmallItems items, so each
+// holds a multiple of kSmallItems + 1 that no other one holds: a slot without a
+// counter.
+__host__ __device__ inline int mid_slot(int b) { return (b + kSmallItems) / (kSmallItems + 1); }
+__host__ __device__ inline int mid_slots(int m) { return m / (kSmallItems + 1) + 1; }
+// first item and first list entry of a region: nodes start at least two items apart
+__host__ __device__ inline int region_first(int m, int r) { return (int)(((int64_t)r * m + kRegions - 1) / kRegions); }
+__host__ __device__ inline int region_base(int m, int r) { return region_first(m, r) / 2 + r; }
+SRT_D int region_of(int m, int b) { return (int)((int64_t)b * kRegions / m); }
+
+// one child of the node split at `mid` on level L (one lane)
+SRT_D void top_child(const TopBuild& B, int L, int mid, int side, int b, int e, const uint32_t* cb, int wide_slot) {
+    TopRec* r = B.rec + mid;
+    if (e - b == 1) {
+        r->child[side] = b;
+        r->kind[side] = kChildItem + ((L + 1) & 1);
+        return;
+    }
+    r->kind[side] = kChildNode;
+    const int32_t up = 2 * mid + side;
+    if (e - b <= kSmallItems) {
+        const int reg = region_of(B.m, b);
+        const int q = atomicAdd(B.nsmall + reg * 64, 1);
+        B.small[region_base(B.m, reg) + q] = {b, e, up, L + 1};
+        return;
+    }
+    TopTask t;
+    t.b = b; t.e = e; t.up = up;
+    for (int q = 0; q < 6; q++) t.cb[q] = cb[q];
+    if (wide_slot >= 0) {
+        B.wide[(L + 1) & 1][wide_slot] = t;
+    } else {
+        B.mid[(L + 1) & 1][mid_slot(b)] = t;
+        B.any[L + 1] = 1;
+    }
+}
+// the node of task t split at `mid`: `side` holds the children's boxes and
+// centroid bounds (one lane)
+SRT_D void top_node(const TopBuild& B, int L, const TopTask& t, int mid, const uint32_t side[2][12], int wide_slot) {
+    TopRec* r = B.rec + mid;
+    for (int s = 0; s < 2; s++)
+        for (int q = 0; q < 6; q++) r->box[s][q] = fromkey(side[s][q]);
+    B.level[mid - 1] = level_key(L);
+    if (t.up) B.rec[t.up >> 1].child[t.up & 1] = mid;
+    top_child(B, L, mid, 0, t.b, mid, side[0] + 6, wide_slot);
+    top_child(B, L, mid, 1, mid, t.e, side[1] + 6, wide_slot < 0 ? -1 : wide_slot + 1);
+}
+
+// Bins in LDS, R copies of each word next to each other: neighbouring items
+// mostly share a bin, and the lanes of a wave that do add to R different banks
+// (one copy per wave, as before, took a wide level of the 1M-triangle field
+// 35 us, lanes that own a bin and look at every item 24 to 43 us, 16 copies
+// 13 us).  A workgroup shares 16 copies, a wave on its own has 4 of the same
+// memory.
+constexpr int kAccTotal = kAccWords * 48;
+constexpr int kBlockCopies = 16, kWaveCopies = kBlockCopies / kTopWaves;
+template <int R> SRT_D void bins_clear(uint32_t* s, int tid, int threads) {
+    for (int i = 4 * tid; i < kAccTotal * R; i += 4 * threads) {
+        const uint32_t v = acc_empty(i / (48 * R));
+        *(uint4*)(s + i) = make_uint4(v, v, v, v);
+    }
+}
+// the wave's items [b, e)
+template <int R> SRT_D void bins_add(const Items& it, int b, int e, const uint32_t* cb, uint32_t* s) {
+    const int lane = __lane_id();
+    float lo[3], ext[3], scale[3];
+    for (int a = 0; a < 3; a++) {
+        lo[a] = fromkey(cb[a]);
+        ext[a] = fromkey(cb[3 + a]) - lo[a];
+        scale[a] = ext[a] > 0.0f ? (float)kBins / ext[a] : 0.0f;
+    }
+    for (int i = b + lane; i < e; i += 64) {
+        const DBox ib = ldbox(it.box, i);
+        const float c[3] = {it.cx[i], it.cy[i], it.cz[i]};
+        const uint32_t tris = (uint32_t)it.count[i];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            if (!(ext[a] > 0.0f)) continue;
+            uint32_t* p = s + (16 * a + bin_of(c[a], lo[a], scale[a])) * R + lane % R;
+            for (int q = 0; q < 3; q++) {
+                atomicMin(p + q * (48 * R), fkey(ib.lo[q]));
+                atomicMax(p + (3 + q) * (48 * R), fkey(ib.hi[q]));
+                atomicMin(p + (6 + q) * (48 * R), fkey(c[q]));
+                atomicMax(p + (9 + q) * (48 * R), fkey(c[q]));
+            }
+            atomicAdd(p + 12 * (48 * R), tris);
+            atomicAdd(p + 13 * (48 * R), 1u);
+        }
+    }
+}
+// word q of bin l (0 .. 47); the copies in an order that spreads the lanes over the banks
+template <int R> SRT_D uint32_t bins_word(const uint32_t* s, int q, int l) {
+    uint32_t v = acc_empty(q);
+    for (int c = 0; c < R; c++) v = acc_union(q, v, s[(q * 48 + l) * R + (c + l) % R]);
     return v;
 }
-SRT_D uint32_t wave_max_u32(uint32_t v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
-    return v;
-}
-constexpr int kSplitWaves = 4;     // kSplitThreads / 64
-// SAH over the 15 bin boundaries of each axis (cost = area x count per side of
-// the boundary) from the bins' key boxes and counts: the first minimum in
-// (axis, boundary) order; axis -1 when no boundary separates items (every
-// extent zero or every item in one bin).
-// The same choice by all 64 lanes of a wave (every lane gets the result):
-// lane 16a + k holds bin k of axis a; inclusive prefix and suffix unions of
-// the bins' key boxes and counts come from shuffles within each group of 16
-// lanes (unions of keys are exact, so each prefix box equals the sequential
-// one); the cost of boundary k uses the suffix of lane k + 1; the minimum over
-// (cost, 16a + k) picks the first minimum in (axis, boundary) order, as the
-// sequential loop does with its strict comparison.
-SRT_D void sah_choose_wave(const uint32_t (*bin)[kBins][6], const int32_t (*cnt)[kBins], const float* ext, int32_t* axis,
-                           int32_t* split) {
-    static_assert(kBins == 16, "one group of 16 lanes per axis");
+// SAH over the 15 bin boundaries of each axis (cost = area x triangles per side
+// of the boundary) from the lanes' bins: the first minimum in (axis, boundary)
+// order.  Returns its lane, -1 when no boundary separates items (every extent
+// zero or every item in one bin); `side` gets the children's words.
+SRT_D int sah_choose_wave(const uint32_t* acc, const uint32_t* cb, uint32_t side[2][kAccWords]) {
+    static_assert(kBins == 16, "a row of 16 lanes per axis");
     const int lane = __lane_id();
     const int a = lane >> 4, k = lane & 15;
-    const bool on = a < 3;
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    uint32_t pl[6], sl[6];
-    int32_t pc = 0, sc = 0;
-    for (int q = 0; q < 6; q++) pl[q] = on ? bin[a][k][q] : (q < 3 ? kinf : kninf);
-    if (on) pc = cnt[a][k];
-    for (int q = 0; q < 6; q++) sl[q] = pl[q];
-    sc = pc;
-    for (int d = 1; d < 16; d <<= 1) {
-        int32_t u = __shfl_up(pc, d, 16), w = __shfl_down(sc, d, 16);
-        if (k >= d) pc += u;
-        if (k + d < 16) sc += w;
-        for (int q = 0; q < 6; q++) {
-            const uint32_t x = (uint32_t)__shfl_up((int)pl[q], d, 16), y = (uint32_t)__shfl_down((int)sl[q], d, 16);
-            if (k >= d) pl[q] = (q < 3) ? min(pl[q], x) : max(pl[q], x);
-            if (k + d < 16) sl[q] = (q < 3) ? min(sl[q], y) : max(sl[q], y);
-        }
+    uint32_t pre[kAccWords], suf[kAccWords];
+    for (int q = 0; q < kAccWords; q++) {
+        const uint32_t none = acc_empty(q);
+        uint32_t p = acc[q], s = acc[q];
+        p = acc_union(q, p, row_get<kRowShr + 1>(none, p));
+        s = acc_union(q, s, row_get<kRowShl + 1>(none, s));
+        p = acc_union(q, p, row_get<kRowShr + 2>(none, p));
+        s = acc_union(q, s, row_get<kRowShl + 2>(none, s));
+        p = acc_union(q, p, row_get<kRowShr + 4>(none, p));
+        s = acc_union(q, s, row_get<kRowShl + 4>(none, s));
+        p = acc_union(q, p, row_get<kRowShr + 8>(none, p));
+        s = acc_union(q, s, row_get<kRowShl + 8>(none, s));
+        pre[q] = p;
+        suf[q] = row_get<kRowShl + 1>(none, s);         // the right side of boundary k starts at bin k + 1
     }
     DBox lb, rb;
     for (int q = 0; q < 3; q++) {
-        lb.lo[q] = fromkey(pl[q]); lb.hi[q] = fromkey(pl[3 + q]);
-        rb.lo[q] = fromkey(sl[q]); rb.hi[q] = fromkey(sl[3 + q]);
+        lb.lo[q] = fromkey(pre[q]); lb.hi[q] = fromkey(pre[3 + q]);
+        rb.lo[q] = fromkey(suf[q]); rb.hi[q] = fromkey(suf[3 + q]);
     }
-    const float la = box_area(lb), ra = box_area(rb);
-    // the right side of boundary k: suffix of bin k + 1
-    const float ra1 = __shfl_down(ra, 1, 16);
-    const int32_t rc1 = __shfl_down(sc, 1, 16);
-    unsigned long long key = ~0ull;
-    if (on && k < kBins - 1 && ext[a] > 0.0f && pc != 0 && rc1 != 0) {
-        const float cost = la * (float)pc + ra1 * (float)rc1;
-        if (cost < __builtin_huge_valf()) key = ((unsigned long long)__float_as_uint(cost) << 32) | (unsigned)lane;
+    const int axis = min(a, 2);
+    const uint32_t klo = axis == 0 ? cb[0] : (axis == 1 ? cb[1] : cb[2]);
+    const uint32_t khi = axis == 0 ? cb[3] : (axis == 1 ? cb[4] : cb[5]);
+    uint32_t key = ~0u;
+    if (a < 3 && k < kBins - 1 && fromkey(khi) - fromkey(klo) > 0.0f && pre[12] != 0 && suf[12] != 0) {
+        const float cost = box_area(lb) * (float)(int32_t)pre[12] + box_area(rb) * (float)(int32_t)suf[12];
+        if (cost < __builtin_huge_valf()) key = __float_as_uint(cost);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned long long o = __shfl_xor(key, off);
-        key = o < key ? o : key;
+    const uint32_t best = wave_min_u32(key);
+    if (best == ~0u) return -1;
+    const int w = uniform(__ffsll(__ballot(key == best)) - 1);
+    for (int q = 0; q < kAccWords; q++) {
+        side[0][q] = read_lane(pre[q], w);
+        side[1][q] = read_lane(suf[q], w);
     }
-    if (key == ~0ull) {
-        *axis = -1;
-        *split = -1;
-    } else {
-        *axis = (int32_t)((key & 0xffffffffu) >> 4);
-        *split = (int32_t)(key & 15u);
+    return w;
+}
+// the words of the items [b, e) by one wave, for a node without a boundary
+SRT_D void union_items(const Items& it, int b, int e, uint32_t* out) {
+    uint32_t v[12];
+    for (int q = 0; q < 12; q++) v[q] = acc_empty(q);
+    for (int i = b + __lane_id(); i < e; i += 64) {
+        const DBox ib = ldbox(it.box, i);
+        for (int a = 0; a < 3; a++) {
+            const uint32_t c = fkey(item_c(it, a, i));
+            v[a] = min(v[a], fkey(ib.lo[a]));
+            v[3 + a] = max(v[3 + a], fkey(ib.hi[a]));
+            v[6 + a] = min(v[6 + a], c);
+            v[9 + a] = max(v[9 + a], c);
+        }
+    }
+    for (int q = 0; q < 12; q++) {
+        for (int d = 32; d > 0; d >>= 1) v[q] = acc_union(q, v[q], (uint32_t)__shfl_xor((int)v[q], d));
+        out[q] = read_lane(v[q], 0);
     }
 }
-__global__ void __launch_bounds__(kSplitThreads) k_top_split(Items it, Items tmp, const int32_t* task_b, const int32_t* task_e,
-                                                             TopSplit* out) {
-    __shared__ uint32_t s_cb[6];
-    // bins per wave (fewer lanes contend for one LDS word), merged after binning
-    __shared__ uint32_t s_bin[kSplitWaves][3][kBins][6];
-    __shared__ int32_t s_cnt[kSplitWaves][3][kBins];
-    __shared__ int32_t s_scan[kSplitThreads];
-    __shared__ uint32_t s_box[2][6];
-    __shared__ int32_t s_axis, s_split, s_run;
-    __shared__ float s_lo[3], s_ext[3];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wv = tid >> 6;
-    const int b = task_b[blockIdx.x], e = task_e[blockIdx.x];
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    if (tid < 6) s_cb[tid] = (tid < 3) ? kinf : kninf;
-    for (int j = tid; j < kSplitWaves * 3 * kBins * 6; j += kSplitThreads)
-        (&s_bin[0][0][0][0])[j] = ((j % 6) < 3) ? kinf : kninf;
-    for (int j = tid; j < kSplitWaves * 3 * kBins; j += kSplitThreads) (&s_cnt[0][0][0])[j] = 0;
-    if (tid < 12) (&s_box[0][0])[tid] = ((tid % 6) < 3) ? kinf : kninf;
-    __syncthreads();
-    // centroid bounds: per-lane keys, a wave reduction, one LDS atomic per wave
-    {
-        uint32_t mn[3] = {kinf, kinf, kinf}, mx[3] = {kninf, kninf, kninf};
-        for (int i = b + tid; i < e; i += kSplitThreads)
-            for (int a = 0; a < 3; a++) {
-                const uint32_t k = fkey(item_c(it, a, i));
-                mn[a] = min(mn[a], k);
-                mx[a] = max(mx[a], k);
-            }
-        for (int a = 0; a < 3; a++) {
-            const uint32_t wmn = wave_min_u32(mn[a]), wmx = wave_max_u32(mx[a]);
-            if (lane == 0) {
-                atomicMin(&s_cb[a], wmn);
-                atomicMax(&s_cb[3 + a], wmx);
-            }
+// the wave's items [b, e), stable: left ones from `l`, right ones from `r`
+SRT_D void partition_items(const Items& src, const Items& dst, int b, int e, int axis, float lo, float scale, int split,
+                           int l, int r) {
+    const int lane = __lane_id();
+    b = uniform(b);
+    e = uniform(e);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (int start = b; start < e; start += 64) {
+        const int i = start + lane;
+        const bool has = i < e;
+        const bool left = has && bin_of(item_c(src, axis, i), lo, scale) <= split;
+        const unsigned long long ml = __ballot(left), mr = __ballot(has && !left);
+        if (has) copy_item(src, i, dst, left ? l + __popcll(ml & below) : r + __popcll(mr & below));
+        l += __popcll(ml);
+        r += __popcll(mr);
+    }
+}
+// One node of a middle level by W waves (each takes a consecutive part of the
+// items); with W > 1 every wave of the workgroup calls it with the same task.
+template <int W>
+SRT_D void split_task(const TopBuild& B, int L, const TopTask& t, int wv, uint32_t* s_bins, int32_t* s_left) {
+    constexpr int R = W == 1 ? kWaveCopies : kBlockCopies;
+    const int lane = __lane_id();
+    const Items &src = B.it[L & 1], &dst = B.it[(L + 1) & 1];
+    const int per = (t.e - t.b + W * 64 - 1) / (W * 64) * 64;
+    const int b = uniform(W == 1 ? t.b : min(t.b + wv * per, t.e)), e = uniform(W == 1 ? t.e : min(b + per, t.e));
+    uint32_t* bins = W == 1 ? s_bins + wv * (kAccTotal * kWaveCopies) : s_bins;
+    bins_clear<R>(bins, W == 1 ? lane : (int)threadIdx.x, 64 * W);
+    if (W > 1) __syncthreads();
+    else wave_sync();
+    bins_add<R>(src, b, e, t.cb, bins);
+    if (W > 1) __syncthreads();
+    else wave_sync();
+    uint32_t acc[kAccWords];
+    for (int q = 0; q < kAccWords; q++) acc[q] = lane < 48 ? bins_word<R>(bins, q, lane) : acc_empty(q);
+    uint32_t side[2][kAccWords];
+    const int w = uniform(sah_choose_wave(acc, t.cb, side));
+    int mid = (t.b + t.e) / 2;
+    if (w >= 0) {
+        mid = t.b + (int)side[0][13];
+        const int axis = w >> 4;
+        const float lo = fromkey(axis == 0 ? t.cb[0] : (axis == 1 ? t.cb[1] : t.cb[2]));
+        const float ext = fromkey(axis == 0 ? t.cb[3] : (axis == 1 ? t.cb[4] : t.cb[5])) - lo;
+        int before = 0;
+        if (W > 1) {
+            int32_t left = 0;
+            for (int i = b + lane; i < e; i += 64)
+                left += bin_of(item_c(src, axis, i), lo, (float)kBins / ext) <= (w & 15) ? 1 : 0;
+            for (int d = 32; d > 0; d >>= 1) left += __shfl_xor(left, d);
+            if (lane == 0) s_left[wv] = left;
+            __syncthreads();
+            for (int v = 0; v < wv; v++) before += s_left[v];
         }
-    }
-    __syncthreads();
-    if (tid < 3) {
-        float lo = fromkey(s_cb[tid]), hi = fromkey(s_cb[3 + tid]);
-        s_lo[tid] = lo;
-        s_ext[tid] = hi - lo;
-    }
-    __syncthreads();
-    // bins for the three axes
-    for (int i = b + tid; i < e; i += kSplitThreads) {
-        DBox ib = ldbox(it.box, i);
-        int cnt = it.count[i];
-        for (int a = 0; a < 3; a++) {
-            float ex = s_ext[a];
-            if (!(ex > 0.0f)) continue;
-            float scale = (float)kBins / ex;
-            int bi = bin_of(item_c(it, a, i), s_lo[a], scale);
-            for (int q = 0; q < 3; q++) {
-                atomicMin(&s_bin[wv][a][bi][q], fkey(ib.lo[q]));
-                atomicMax(&s_bin[wv][a][bi][3 + q], fkey(ib.hi[q]));
-            }
-            atomicAdd(&s_cnt[wv][a][bi], cnt);
-        }
-    }
-    __syncthreads();
-    // merge the waves' bins into copy 0 (min / max of keys and integer sums: order-free)
-    for (int j = tid; j < 3 * kBins * 7; j += kSplitThreads) {
-        const int w = j % 7, ab = j / 7;
-        const int a = ab / kBins, k = ab % kBins;
-        if (w < 6) {
-            uint32_t v = s_bin[0][a][k][w];
-            for (int q = 1; q < kSplitWaves; q++) v = (w < 3) ? min(v, s_bin[q][a][k][w]) : max(v, s_bin[q][a][k][w]);
-            s_bin[0][a][k][w] = v;
-        } else {
-            int32_t v = s_cnt[0][a][k];
-            for (int q = 1; q < kSplitWaves; q++) v += s_cnt[q][a][k];
-            s_cnt[0][a][k] = v;
-        }
-    }
-    __syncthreads();
-    if (tid < 64) {
-        int32_t ax, sp;
-        sah_choose_wave(s_bin[0], s_cnt[0], s_ext, &ax, &sp);
-        if (tid == 0) {
-            s_axis = ax;
-            s_split = sp;
-            s_run = 0;
-        }
-    }
-    __syncthreads();
-    const int axis = s_axis, split = s_split;
-    int mid;
-    if (axis < 0) {
-        mid = (b + e) / 2;
+        partition_items(src, dst, b, e, axis, lo, (float)kBins / ext, w & 15, t.b + before, mid + (b - t.b) - before);
     } else {
-        const float scale = (float)kBins / s_ext[axis];
-        const float lo = s_lo[axis];
-        // stable partition, 256 items per step: each wave ranks its items with
-        // a ballot, the four wave counts go through LDS
-        const unsigned long long below = (1ull << lane) - 1ull;
-        for (int pass = 0; pass < 2; pass++) {
-            const int base = (pass == 0) ? b : b + s_run;   // s_run holds nleft after pass 0
-            __syncthreads();
-            int run = 0;
-            for (int start = b; start < e; start += kSplitThreads) {
-                int i = start + tid;
-                bool flag = false;
-                if (i < e) {
-                    bool left = bin_of(item_c(it, axis, i), lo, scale) <= split;
-                    flag = (pass == 0) ? left : !left;
-                }
-                const unsigned long long m = __ballot(flag);
-                if (lane == 0) s_scan[wv] = __popcll(m);
-                __syncthreads();
-                int wbase = 0, total = 0;
-                for (int q = 0; q < kSplitWaves; q++) {
-                    const int c = s_scan[q];
-                    wbase += (q < wv) ? c : 0;
-                    total += c;
-                }
-                if (flag) copy_item(it, i, tmp, base + run + wbase + __popcll(m & below));
-                run += total;
-                __syncthreads();
+        for (int i = b + lane; i < e; i += 64) copy_item(src, i, dst, i);
+        union_items(src, t.b, mid, side[0]);
+        union_items(src, mid, t.e, side[1]);
+    }
+    if (wv == 0 || W == 1) {
+        if (lane == 0) {
+            const uint32_t* s0 = side[0];
+            const uint32_t* s1 = side[1];
+            uint32_t sd[2][12];
+            for (int q = 0; q < 12; q++) {
+                sd[0][q] = s0[q];
+                sd[1][q] = s1[q];
             }
-            if (pass == 0 && tid == 0) s_run = run;
-            __syncthreads();
+            top_node(B, L, t, mid, sd, -1);
         }
-        mid = b + s_run;
-        __syncthreads();
-        for (int i = b + tid; i < e; i += kSplitThreads) copy_item(tmp, i, it, i);
+    }
+}
+// workgroup g: kMidSlots slots of the level, nodes of more than kBlockItems
+// items by all waves, then the others by one wave each.  Bound by the latency
+// of a node's chain (load, bin, scan, choose, partition); with one slot a wave
+// most workgroups of a level were empty and a level took at least 48 us.
+constexpr int kMidSlots = 16;
+__global__ void __launch_bounds__(64 * kTopWaves) k_top_mid(TopBuild B, int L, int slots) {
+    __shared__ alignas(16) uint32_t s_bins[kAccTotal * kBlockCopies];
+    __shared__ TopTask s_task[kMidSlots];
+    __shared__ int32_t s_left[kTopWaves];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // every wave knows the slots in use; wave 0 takes the tasks out of them
+    const int slot = blockIdx.x * kMidSlots + lane;
+    TopTask* p = B.mid[L & 1] + slot;
+    TopTask mine;
+    mine.b = mine.e = 0;
+    if (wv == 0 && lane < kMidSlots) {
+        if (slot < slots) {
+            mine = *p;
+            if (mine.e > mine.b) p->b = p->e = 0;    // the list of level L + 2
+        }
+        s_task[lane] = mine;
+    }
+    __syncthreads();
+    int n = 0;
+    if (lane < kMidSlots) n = s_task[lane].e - s_task[lane].b;
+    for (unsigned long long big = __ballot(n > kBlockItems); big; big &= big - 1) {
+        split_task<kTopWaves>(B, L, s_task[__ffsll(big) - 1], wv, s_bins, s_left);
         __syncthreads();
     }
-    // child boxes: per-lane keys of each side, wave reductions, one LDS atomic per wave
-    {
-        uint32_t mn[2][3], mx[2][3];
-        for (int sd = 0; sd < 2; sd++)
-            for (int q = 0; q < 3; q++) { mn[sd][q] = kinf; mx[sd][q] = kninf; }
-        for (int i = b + tid; i < e; i += kSplitThreads) {
-            const int side = (i < mid) ? 0 : 1;
+    int k = 0;
+    for (unsigned long long some = __ballot(n > 0 && n <= kBlockItems); some; some &= some - 1)
+        if (k++ % kTopWaves == wv) split_task<1>(B, L, s_task[__ffsll(some) - 1], wv, s_bins, s_left);
+}
+// Subtrees of two to kSmallItems items, one wave each.  With so few items the
+// candidates are the items themselves: lane 21 a + i is the boundary after item
+// i's bin of axis a (an empty bin's boundary costs the same as the one before
+// it), it looks at every item once and has both sides' boxes and counts, with
+// no bins and no scan.  Nodes of two items, a third of all, are left to the
+// end and split by a lane each.  Bound by instructions, about 300 for a node.
+__global__ void __launch_bounds__(64 * kTopWaves) k_top_small(TopBuild B) {
+    static_assert(3 * kSmallItems <= 64, "one lane per axis and item");
+    struct alignas(16) Item {
+        uint32_t w[12];     // box and centroid keys, triangles, ref
+    };
+    __shared__ Item s_item[kTopWaves][kSmallItems];
+    __shared__ int32_t s_bin[kTopWaves][64];
+    __shared__ int4 s_stack[kTopWaves][kSmallItems];
+    __shared__ int4 s_pair[kTopWaves][kSmallItems / 2];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int axis = lane / kSmallItems, li = lane % kSmallItems, ax = min(axis, 2);
+    const int reg = blockIdx.x / kRegionBlocks, first = blockIdx.x % kRegionBlocks * kTopWaves + wv;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    Item* item = s_item[wv];
+    const int count = B.nsmall[reg * 64], base = region_base(B.m, reg);
+    for (int k = first; k < count; k += kRegionBlocks * kTopWaves) {
+        const SmallTask t = B.small[base + k];
+        const Items& it = B.it[t.level & 1];
+        const int total = t.e - t.b;
+        wave_sync();
+        if (lane < total) {
+            const int i = t.b + lane;
+            Item v;
             const DBox ib = ldbox(it.box, i);
-            for (int q = 0; q < 3; q++) {
-                mn[side][q] = min(mn[side][q], fkey(ib.lo[q]));
-                mx[side][q] = max(mx[side][q], fkey(ib.hi[q]));
+            for (int a = 0; a < 3; a++) {
+                v.w[a] = fkey(ib.lo[a]);
+                v.w[3 + a] = fkey(ib.hi[a]);
+                v.w[6 + a] = fkey(item_c(it, a, i));
             }
+            v.w[9] = (uint32_t)it.count[i];
+            v.w[10] = (uint32_t)it.ref[i];
+            v.w[11] = 0;
+            item[lane] = v;
         }
-        for (int sd = 0; sd < 2; sd++)
-            for (int q = 0; q < 3; q++) {
-                const uint32_t wmn = wave_min_u32(mn[sd][q]), wmx = wave_max_u32(mx[sd][q]);
-                if (lane == 0) {
-                    atomicMin(&s_box[sd][q], wmn);
-                    atomicMax(&s_box[sd][3 + q], wmx);
+        if (lane == 0) {
+            s_stack[wv][0] = make_int4(0, total, t.up, t.level);
+            s_pair[wv][0] = make_int4(0, total, t.up, t.level);
+        }
+        wave_sync();
+        int sp = total > 2 ? 1 : 0, pairs = total > 2 ? 0 : 1;
+        while (sp > 0) {
+            sp--;
+            const int4 f = s_stack[wv][sp];
+            const int b = uniform(f.x), e = uniform(f.y);
+            const int n = e - b;
+            uint32_t mn = ~0u, mx = 0u;
+            for (int j = b; j < e; j++) {
+                const uint32_t c = item[j].w[6 + ax];
+                mn = min(mn, c);
+                mx = max(mx, c);
+            }
+            const float lo = fromkey(mn), ext = fromkey(mx) - lo;
+            const bool on = axis < 3 && li < n && ext > 0.0f;
+            int bin = kBins;
+            if (on) bin = bin_of(fromkey(item[b + li].w[6 + ax]), lo, (float)kBins / ext);
+            s_bin[wv][lane] = bin;
+            wave_sync();
+            // lane j < n: item j and its bins of the three axes
+            const Item v = item[min(b + lane, kSmallItems - 1)];
+            const int own = min(lane, kSmallItems - 1);
+            const uint32_t bins = (uint32_t)s_bin[wv][own] | (uint32_t)s_bin[wv][kSmallItems + own] << 8 |
+                                  (uint32_t)s_bin[wv][2 * kSmallItems + own] << 16;
+            uint32_t l[6], r[6];
+            int32_t lc = 0, rc = 0;
+            for (int q = 0; q < 6; q++) l[q] = r[q] = acc_empty(q);
+            for (int j = 0; j < n; j++) {
+                uint32_t x[6];
+                for (int q = 0; q < 6; q++) x[q] = read_lane(v.w[q], j);
+                const int32_t tris = (int32_t)read_lane(v.w[9], j);
+                if ((int)((read_lane(bins, j) >> (8 * ax)) & 0xffu) <= bin) {
+                    for (int q = 0; q < 6; q++) l[q] = acc_union(q, l[q], x[q]);
+                    lc += tris;
+                } else {
+                    for (int q = 0; q < 6; q++) r[q] = acc_union(q, r[q], x[q]);
+                    rc += tris;
                 }
             }
+            uint32_t key = ~0u;
+            if (on && bin < kBins - 1 && lc != 0 && rc != 0) {
+                DBox lb, rb;
+                for (int q = 0; q < 3; q++) {
+                    lb.lo[q] = fromkey(l[q]); lb.hi[q] = fromkey(l[3 + q]);
+                    rb.lo[q] = fromkey(r[q]); rb.hi[q] = fromkey(r[3 + q]);
+                }
+                const float cost = box_area(lb) * (float)lc + box_area(rb) * (float)rc;
+                if (cost < __builtin_huge_valf()) key = __float_as_uint(cost);
+            }
+            const uint32_t best = wave_min_u32(key);
+            int w = 0, nl = (t.b + b + t.b + e) / 2 - (t.b + b);
+            bool left = lane < nl;
+            if (best != ~0u) {
+                // the first minimum in (axis, boundary) order
+                const uint32_t code = key == best ? (uint32_t)(16 * axis + bin) : ~0u;
+                const uint32_t pick = wave_min_u32(code);
+                w = __ffsll(__ballot(code == pick)) - 1;
+                left = lane < n && s_bin[wv][(int)(pick >> 4) * kSmallItems + min(lane, kSmallItems - 1)] <= (int)(pick & 15u);
+                nl = __popcll(__ballot(left));
+            } else {
+                for (int q = 0; q < 6; q++) l[q] = r[q] = acc_empty(q);
+                for (int j = 0; j < n; j++)
+                    for (int q = 0; q < 6; q++) {
+                        const uint32_t x = read_lane(v.w[q], j);
+                        if (j < nl) l[q] = acc_union(q, l[q], x);
+                        else r[q] = acc_union(q, r[q], x);
+                    }
+            }
+            const unsigned long long ml = __ballot(left), mr = __ballot(lane < n && !left);
+            wave_sync();
+            if (lane < n) item[b + (left ? __popcll(ml & below) : nl + __popcll(mr & below))] = v;
+            wave_sync();
+            const int mid = t.b + b + nl;
+            TopRec* rec = B.rec + mid;
+            if (lane == w)
+                for (int q = 0; q < 6; q++) {
+                    rec->box[0][q] = fromkey(l[q]);
+                    rec->box[1][q] = fromkey(r[q]);
+                }
+            const bool li1 = nl == 1, ri1 = n - nl == 1;
+            if (lane == 0) {
+                B.level[mid - 1] = level_key(f.w);
+                if (f.z) B.rec[f.z >> 1].child[f.z & 1] = mid;
+                rec->kind[0] = li1 ? kChildRef : kChildNode;
+                rec->kind[1] = ri1 ? kChildRef : kChildNode;
+                if (li1) rec->child[0] = (int32_t)item[b].w[10];
+                if (ri1) rec->child[1] = (int32_t)item[e - 1].w[10];
+                const int4 lt = make_int4(b, b + nl, 2 * mid, f.w + 1), rt = make_int4(b + nl, e, 2 * mid + 1, f.w + 1);
+                int at = sp, pat = pairs;
+                if (n - nl == 2) s_pair[wv][pat++] = rt;
+                else if (!ri1) s_stack[wv][at++] = rt;
+                if (nl == 2) s_pair[wv][pat++] = lt;
+                else if (!li1) s_stack[wv][at++] = lt;
+            }
+            sp += (nl > 2 ? 1 : 0) + (n - nl > 2 ? 1 : 0);
+            pairs += (nl == 2 ? 1 : 0) + (n - nl == 2 ? 1 : 0);
+            wave_sync();
+        }
+        // The nodes of two items, one lane each: every boundary costs the same,
+        // so the first axis whose bins differ splits them, in bin order.
+        if (lane < pairs) {
+            const int4 f = s_pair[wv][lane];
+            const Item v0 = item[f.x], v1 = item[f.x + 1];
+            bool split = false, swap = false;
+            for (int a = 0; a < 3; a++) {
+                const float c0 = fromkey(v0.w[6 + a]), c1 = fromkey(v1.w[6 + a]);
+                const float lo = fromkey(min(v0.w[6 + a], v1.w[6 + a]));
+                const float ext = fromkey(max(v0.w[6 + a], v1.w[6 + a])) - lo;
+                if (split || !(ext > 0.0f)) continue;
+                const float scale = (float)kBins / ext;
+                const int b0 = bin_of(c0, lo, scale), b1 = bin_of(c1, lo, scale);
+                split = b0 != b1;
+                swap = b1 < b0;
+            }
+            DBox x0, x1;
+            for (int q = 0; q < 3; q++) {
+                x0.lo[q] = fromkey(v0.w[q]); x0.hi[q] = fromkey(v0.w[3 + q]);
+                x1.lo[q] = fromkey(v1.w[q]); x1.hi[q] = fromkey(v1.w[3 + q]);
+            }
+            const float cost = box_area(x0) * (float)(int32_t)v0.w[9] + box_area(x1) * (float)(int32_t)v1.w[9];
+            swap = swap && cost < __builtin_huge_valf();       // else the items keep their order
+            const int mid = t.b + f.x + 1;
+            TopRec rec;
+            for (int q = 0; q < 3; q++) {
+                rec.box[0][q] = swap ? x1.lo[q] : x0.lo[q];
+                rec.box[0][3 + q] = swap ? x1.hi[q] : x0.hi[q];
+                rec.box[1][q] = swap ? x0.lo[q] : x1.lo[q];
+                rec.box[1][3 + q] = swap ? x0.hi[q] : x1.hi[q];
+            }
+            rec.child[0] = (int32_t)(swap ? v1.w[10] : v0.w[10]);
+            rec.child[1] = (int32_t)(swap ? v0.w[10] : v1.w[10]);
+            rec.kind[0] = rec.kind[1] = kChildRef;
+            B.rec[mid] = rec;
+            B.level[mid - 1] = level_key(f.w);
+            if (f.z) B.rec[f.z >> 1].child[f.z & 1] = mid;
+        }
     }
-    __syncthreads();
-    if (tid < 12) out[blockIdx.x].box[tid / 6][tid % 6] = fromkey(s_box[tid / 6][tid % 6]);
-    if (tid == 0) out[blockIdx.x].mid = mid;
 }
 
-
-// Wide levels: a level of at most kWideTasks nodes (the first levels, where
-// one workgroup per node would leave most CUs idle) is split by a grid of
-// workgroups over chunks of kWideChunk items; chunk g of the level belongs to
-// the node whose chunk range holds it.  Per-node accumulators live in global
-// memory: centroid bounds, bins and child boxes are min / max of ordered float
-// keys and integer sums (independent of the order of the atomics), the split
-// is chosen by sah_choose_wave as above, and the partition places each chunk's
-// items after the left / right items of the node's earlier chunks, ranked
-// within the chunk by wave ballots: the same split, the same stable partition
-// and the same child boxes as k_top_split.
-constexpr int kWideTasks = 64;
-constexpr int kWideChunk = 1024;      // 4 items per thread
-constexpr int kWideMaxGrid = 1024;
-struct WideAcc {
-    uint32_t cb[kWideTasks][6];                 // centroid bounds (keys): lo xyz, hi xyz
-    uint32_t bin[kWideTasks][3][kBins][6];      // bin boxes (keys)
-    int32_t cnt[kWideTasks][3][kBins];          // bin triangle counts
-    int32_t axis[kWideTasks], split[kWideTasks], nleft[kWideTasks];
-    float lo[kWideTasks][3], ext[kWideTasks][3];
-    uint32_t box[kWideTasks][2][6];             // child boxes (keys)
-};
-// Chunk ranges of the level's nodes (wave 0 scans the chunk counts; ntask <=
-// 64) into s_first[0..ntask]; returns the number of chunks.
-SRT_D int wide_chunks(int ntask, const int32_t* tb, const int32_t* te, int32_t* s_first) {
-    if (threadIdx.x < 64u) {
-        const int t = threadIdx.x;
-        int v = t < ntask ? (te[t] - tb[t] + kWideChunk - 1) / kWideChunk : 0;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int u = __shfl_up(v, d);
-            if (t >= d) v += u;
-        }
-        s_first[t + 1] = v;
-        if (t == 0) s_first[0] = 0;
-    }
+// Chunks of a wide level: s_first[t] .. s_first[t + 1] are slot t's (at most 256 slots).  Returns their number.
+SRT_D int wide_chunks(int ntask, const TopTask* task, int32_t* s_first) {
+    __shared__ int32_t s_w[4];
+    const int t = threadIdx.x;
+    const int v = t < ntask ? (task[t].e - task[t].b + kWideChunk - 1) / kWideChunk : 0;
+    s_first[t + 1] = block_scan256(v, s_w);
+    if (t == 0) s_first[0] = 0;
     __syncthreads();
     return s_first[ntask];
 }
-SRT_D int wide_task(const int32_t* s_first, int g) {
-    int t = 0;
-    while (g >= s_first[t + 1]) t++;
-    return t;
+SRT_D int wide_slot_of(const int32_t* s_first, int g) {
+    int lo = 0, hi = 255;                 // the slot with s_first[slot] <= g < s_first[slot + 1]
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (g < s_first[mid + 1]) hi = mid;
+        else lo = mid + 1;
+    }
+    return lo;
 }
-__global__ void __launch_bounds__(256) k_wide_init(int ntask, WideAcc* A) {
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    const int j0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
-    for (int j = j0; j < ntask * 6; j += stride) (&A->cb[0][0])[j] = (j % 6 < 3) ? kinf : kninf;
-    for (int j = j0; j < ntask * 3 * kBins * 6; j += stride) (&A->bin[0][0][0][0])[j] = (j % 6 < 3) ? kinf : kninf;
-    for (int j = j0; j < ntask * 3 * kBins; j += stride) (&A->cnt[0][0][0])[j] = 0;
-    for (int j = j0; j < ntask * 12; j += stride) (&A->box[0][0][0])[j] = (j % 6 < 3) ? kinf : kninf;
-}
-__global__ void __launch_bounds__(256) k_wide_bounds(int ntask, const int32_t* tb, const int32_t* te, Items it, WideAcc* A) {
-    __shared__ int32_t s_first[kWideTasks + 1];
-    __shared__ uint32_t s_cb[6];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    const int total = wide_chunks(ntask, tb, te, s_first);
-    for (int g = blockIdx.x; g < total; g += gridDim.x) {
-        const int t = wide_task(s_first, g);
-        const int b = tb[t] + (g - s_first[t]) * kWideChunk, e = min(b + kWideChunk, te[t]);
-        if (tid < 6) s_cb[tid] = (tid < 3) ? kinf : kninf;
-        __syncthreads();
-        uint32_t mn[3] = {kinf, kinf, kinf}, mx[3] = {kninf, kninf, kninf};
-        for (int i = b + tid; i < e; i += 256)
-            for (int a = 0; a < 3; a++) {
-                const uint32_t k = fkey(item_c(it, a, i));
-                mn[a] = min(mn[a], k);
-                mx[a] = max(mx[a], k);
-            }
-        for (int a = 0; a < 3; a++) {
-            const uint32_t wmn = wave_min_u32(mn[a]), wmx = wave_max_u32(mx[a]);
-            if (lane == 0) {
-                atomicMin(&s_cb[a], wmn);
-                atomicMax(&s_cb[3 + a], wmx);
-            }
-        }
-        __syncthreads();
-        if (tid < 3) atomicMin(&A->cb[t][tid], s_cb[tid]);
-        else if (tid < 6) atomicMax(&A->cb[t][tid], s_cb[tid]);
-        __syncthreads();
+static_assert((1 << (kWideLevels - 1)) <= 256 && kTopWaves == 4, "a wide level's slots are scanned by one workgroup");
+__global__ void __launch_bounds__(64 * kTopWaves) k_top_wide_bins(TopBuild B, int L) {
+    __shared__ int32_t s_first[257];
+    __shared__ alignas(16) uint32_t s_bins[kAccTotal * kBlockCopies];
+    const int tid = threadIdx.x, wv = tid >> 6, g = blockIdx.x;
+    const TopTask* task = B.wide[L & 1];
+    if (g >= wide_chunks(1 << L, task, s_first)) return;
+    const int t = wide_slot_of(s_first, g);
+    const TopTask tk = task[t];
+    const int b = tk.b + (g - s_first[t]) * kWideChunk, e = min(b + kWideChunk, tk.e);
+    constexpr int kPart = kWideChunk / kTopWaves;
+    bins_clear<kBlockCopies>(s_bins, tid, 64 * kTopWaves);
+    __syncthreads();
+    const int wb = min(b + wv * kPart, e);
+    bins_add<kBlockCopies>(B.it[L & 1], wb, min(wb + kPart, e), tk.cb, s_bins);
+    __syncthreads();
+    uint32_t* out = B.acc + ((size_t)t * kWideCopies + g % kWideCopies) * kAccTotal;
+    for (int j = tid; j < kAccTotal; j += 64 * kTopWaves) {
+        const int q = j / 48, l = j % 48;
+        const uint32_t v = bins_word<kBlockCopies>(s_bins, q, l);
+        if (q == 13) B.chunk_items[(size_t)g * 48 + l] = (int32_t)v;
+        if (v == acc_empty(q)) continue;
+        if (q >= 12) atomicAdd(out + j, v);
+        else if (q % 6 < 3) atomicMin(out + j, v);
+        else atomicMax(out + j, v);
     }
 }
-__global__ void __launch_bounds__(256) k_wide_bins(int ntask, const int32_t* tb, const int32_t* te, Items it, WideAcc* A) {
-    __shared__ int32_t s_first[kWideTasks + 1];
-    __shared__ uint32_t s_bin[kSplitWaves][3][kBins][6];
-    __shared__ int32_t s_cnt[kSplitWaves][3][kBins];
-    __shared__ float s_lo[3], s_ext[3];
-    const int tid = threadIdx.x, wv = tid >> 6;
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    const int total = wide_chunks(ntask, tb, te, s_first);
-    for (int g = blockIdx.x; g < total; g += gridDim.x) {
-        const int t = wide_task(s_first, g);
-        const int b = tb[t] + (g - s_first[t]) * kWideChunk, e = min(b + kWideChunk, te[t]);
-        for (int j = tid; j < kSplitWaves * 3 * kBins * 6; j += 256) (&s_bin[0][0][0][0])[j] = ((j % 6) < 3) ? kinf : kninf;
-        for (int j = tid; j < kSplitWaves * 3 * kBins; j += 256) (&s_cnt[0][0][0])[j] = 0;
-        if (tid < 3) {
-            const float lo = fromkey(A->cb[t][tid]), hi = fromkey(A->cb[t][3 + tid]);
-            s_lo[tid] = lo;
-            s_ext[tid] = hi - lo;
-        }
-        __syncthreads();
-        for (int i = b + tid; i < e; i += 256) {
-            const DBox ib = ldbox(it.box, i);
-            const int cnt = it.count[i];
-            for (int a = 0; a < 3; a++) {
-                const float ex = s_ext[a];
-                if (!(ex > 0.0f)) continue;
-                const float scale = (float)kBins / ex;
-                const int bi = bin_of(item_c(it, a, i), s_lo[a], scale);
-                for (int q = 0; q < 3; q++) {
-                    atomicMin(&s_bin[wv][a][bi][q], fkey(ib.lo[q]));
-                    atomicMax(&s_bin[wv][a][bi][3 + q], fkey(ib.hi[q]));
-                }
-                atomicAdd(&s_cnt[wv][a][bi], cnt);
+// workgroup (one wave) t: the split of slot t, its children, and its accumulators empty again
+__global__ void __launch_bounds__(64) k_top_wide_sah(TopBuild B, int L) {
+    const int t = blockIdx.x, lane = threadIdx.x;
+    const TopTask tk = B.wide[L & 1][t];
+    const bool more = L + 1 < B.wide_levels;
+    if (more && lane < 2) {
+        TopTask* c = B.wide[(L + 1) & 1] + 2 * t + lane;
+        c->b = c->e = 0;
+    }
+    if (tk.e <= tk.b) return;
+    __syncthreads();                      // the children below replace the empty slots
+    uint32_t acc[kAccWords];
+    for (int q = 0; q < kAccWords; q++) acc[q] = acc_empty(q);
+    if (lane < 48)
+        for (int c = 0; c < kWideCopies; c++) {
+            uint32_t* p = B.acc + ((size_t)t * kWideCopies + c) * kAccTotal + lane;
+            for (int q = 0; q < kAccWords; q++) {
+                acc[q] = acc_union(q, acc[q], p[q * 48]);
+                p[q * 48] = acc_empty(q);
             }
         }
-        __syncthreads();
-        // merge the waves' bins and add the non-empty ones to the node's bins
-        for (int j = tid; j < 3 * kBins * 7; j += 256) {
-            const int w = j % 7, ab = j / 7;
-            const int a = ab / kBins, k = ab % kBins;
-            int32_t n = 0;
-            for (int q = 0; q < kSplitWaves; q++) n += s_cnt[q][a][k];
-            if (n == 0) continue;
-            if (w < 6) {
-                uint32_t v = s_bin[0][a][k][w];
-                for (int q = 1; q < kSplitWaves; q++) v = (w < 3) ? min(v, s_bin[q][a][k][w]) : max(v, s_bin[q][a][k][w]);
-                if (w < 3) atomicMin(&A->bin[t][a][k][w], v);
-                else atomicMax(&A->bin[t][a][k][w], v);
-            } else {
-                atomicAdd(&A->cnt[t][a][k], n);
-            }
+    uint32_t side[2][kAccWords];
+    const int w = sah_choose_wave(acc, tk.cb, side);
+    const Items& src = B.it[L & 1];
+    int mid = (tk.b + tk.e) / 2;
+    WideSplit s = {-1, 0, mid, 0.0f, 0.0f};
+    if (w >= 0) {
+        mid = tk.b + (int)side[0][13];
+        const int axis = w >> 4;
+        const float lo = fromkey(axis == 0 ? tk.cb[0] : (axis == 1 ? tk.cb[1] : tk.cb[2]));
+        const float ext = fromkey(axis == 0 ? tk.cb[3] : (axis == 1 ? tk.cb[4] : tk.cb[5])) - lo;
+        s = {axis, w & 15, mid, lo, (float)kBins / ext};
+    } else {
+        union_items(src, tk.b, mid, side[0]);
+        union_items(src, mid, tk.e, side[1]);
+    }
+    if (lane == 0) {
+        uint32_t sd[2][12];
+        for (int q = 0; q < 12; q++) {
+            sd[0][q] = side[0][q];
+            sd[1][q] = side[1][q];
         }
-        __syncthreads();
+        B.wsplit[t] = s;
+        top_node(B, L, tk, mid, sd, more ? 2 * t : -1);
     }
 }
-__global__ void __launch_bounds__(64) k_wide_sah(WideAcc* A) {
-    const int t = blockIdx.x;
-    float ext[3];
-    for (int a = 0; a < 3; a++) {
-        const float lo = fromkey(A->cb[t][a]), hi = fromkey(A->cb[t][3 + a]);
-        ext[a] = hi - lo;
-        if (threadIdx.x == 0) {
-            A->lo[t][a] = lo;
-            A->ext[t][a] = ext[a];
-        }
+__global__ void __launch_bounds__(64 * kTopWaves) k_top_wide_scatter(TopBuild B, int L) {
+    __shared__ int32_t s_first[257];
+    __shared__ int32_t s_left[kTopWaves], s_before[kTopWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = blockIdx.x;
+    const TopTask* task = B.wide[L & 1];
+    if (g >= wide_chunks(1 << L, task, s_first)) return;
+    const int t = wide_slot_of(s_first, g), f = s_first[t];
+    const int tb = task[t].b, b = tb + (g - f) * kWideChunk, e = min(b + kWideChunk, task[t].e);
+    const WideSplit s = B.wsplit[t];
+    const Items &src = B.it[L & 1], &dst = B.it[(L + 1) & 1];
+    if (s.axis < 0) {
+        for (int i = b + tid; i < e; i += 64 * kTopWaves) copy_item(src, i, dst, i);
+        return;
     }
-    int32_t ax, sp;
-    sah_choose_wave(A->bin[t], A->cnt[t], ext, &ax, &sp);
-    if (threadIdx.x == 0) {
-        A->axis[t] = ax;
-        A->split[t] = sp;
-    }
-}
-// left items of each chunk (a node without a split keeps its order)
-__global__ void __launch_bounds__(256) k_wide_count(int ntask, const int32_t* tb, const int32_t* te, Items it,
-                                                    const WideAcc* A, int32_t* chunk_left) {
-    __shared__ int32_t s_first[kWideTasks + 1];
-    __shared__ int32_t s_w[kSplitWaves];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int total = wide_chunks(ntask, tb, te, s_first);
-    for (int g = blockIdx.x; g < total; g += gridDim.x) {
-        const int t = wide_task(s_first, g);
-        const int axis = A->axis[t];
-        if (axis < 0) continue;          // uniform over the workgroup
-        const int b = tb[t] + (g - s_first[t]) * kWideChunk, e = min(b + kWideChunk, te[t]);
-        const float scale = (float)kBins / A->ext[t][axis], lo = A->lo[t][axis];
-        const int split = A->split[t];
-        int n = 0;
-        for (int i = b + tid; i < e; i += 256) n += (bin_of(item_c(it, axis, i), lo, scale) <= split) ? 1 : 0;
-        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
-        if (lane == 0) s_w[wv] = n;
-        __syncthreads();
-        if (tid == 0) chunk_left[g] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
-        __syncthreads();
-    }
-}
-// stable partition of each chunk into tmp: its left items after the left
-// items of the node's earlier chunks, its right items after all left items
-// and the right items of the earlier chunks
-__global__ void __launch_bounds__(256) k_wide_scatter(int ntask, const int32_t* tb, const int32_t* te, Items it, Items tmp,
-                                                      WideAcc* A, const int32_t* chunk_left) {
-    __shared__ int32_t s_first[kWideTasks + 1];
-    __shared__ int32_t s_w[2][kSplitWaves];
-    __shared__ int32_t s_sum[2][kSplitWaves];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const int total = wide_chunks(ntask, tb, te, s_first);
-    for (int g = blockIdx.x; g < total; g += gridDim.x) {
-        const int t = wide_task(s_first, g);
-        const int axis = A->axis[t];
-        if (axis < 0) continue;          // uniform over the workgroup
-        const int k = g - s_first[t];
-        const int tb0 = tb[t];
-        const int b = tb0 + k * kWideChunk, e = min(b + kWideChunk, te[t]);
-        // left items before this chunk and in the whole node
-        int before = 0, all = 0;
-        for (int q = s_first[t] + tid; q < s_first[t + 1]; q += 256) {
-            const int c = chunk_left[q];
-            all += c;
-            before += (q < g) ? c : 0;
-        }
-        for (int off = 32; off > 0; off >>= 1) {
-            before += __shfl_xor(before, off);
-            all += __shfl_xor(all, off);
-        }
-        if (lane == 0) { s_sum[0][wv] = before; s_sum[1][wv] = all; }
-        __syncthreads();
-        const int lbefore = s_sum[0][0] + s_sum[0][1] + s_sum[0][2] + s_sum[0][3];
-        const int nleft = s_sum[1][0] + s_sum[1][1] + s_sum[1][2] + s_sum[1][3];
-        if (k == 0 && tid == 0) A->nleft[t] = nleft;
-        const float scale = (float)kBins / A->ext[t][axis], lo = A->lo[t][axis];
-        const int split = A->split[t];
-        int lrun = tb0 + lbefore;                          // next left slot
-        int rrun = tb0 + nleft + (b - tb0 - lbefore);      // next right slot
-        for (int start = b; start < e; start += 256) {
-            const int i = start + tid;
-            bool has = i < e, left = false;
-            if (has) left = bin_of(item_c(it, axis, i), lo, scale) <= split;
-            const unsigned long long ml = __ballot(has && left), mr = __ballot(has && !left);
-            if (lane == 0) { s_w[0][wv] = __popcll(ml); s_w[1][wv] = __popcll(mr); }
-            __syncthreads();
-            int lb = 0, rb = 0, lt = 0, rt = 0;
-            for (int q = 0; q < kSplitWaves; q++) {
-                lb += (q < wv) ? s_w[0][q] : 0;
-                rb += (q < wv) ? s_w[1][q] : 0;
-                lt += s_w[0][q];
-                rt += s_w[1][q];
-            }
-            if (has) {
-                const int dst = left ? lrun + lb + __popcll(ml & below) : rrun + rb + __popcll(mr & below);
-                copy_item(it, i, tmp, dst);
-            }
-            lrun += lt;
-            rrun += rt;
-            __syncthreads();
-        }
-    }
-}
-// copy the partitioned chunks back and reduce the child boxes
-__global__ void __launch_bounds__(256) k_wide_boxes(int ntask, const int32_t* tb, const int32_t* te, Items it, Items tmp,
-                                                    WideAcc* A) {
-    __shared__ int32_t s_first[kWideTasks + 1];
-    __shared__ uint32_t s_box[2][6];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    const int total = wide_chunks(ntask, tb, te, s_first);
-    for (int g = blockIdx.x; g < total; g += gridDim.x) {
-        const int t = wide_task(s_first, g);
-        const int axis = A->axis[t];
-        const int b = tb[t] + (g - s_first[t]) * kWideChunk, e = min(b + kWideChunk, te[t]);
-        const int mid = axis < 0 ? (tb[t] + te[t]) / 2 : tb[t] + A->nleft[t];
-        if (tid < 12) (&s_box[0][0])[tid] = ((tid % 6) < 3) ? kinf : kninf;
-        __syncthreads();
-        uint32_t mn[2][3], mx[2][3];
-        for (int sd = 0; sd < 2; sd++)
-            for (int q = 0; q < 3; q++) { mn[sd][q] = kinf; mx[sd][q] = kninf; }
-        for (int i = b + tid; i < e; i += 256) {
-            DBox ib;
-            if (axis >= 0) {
-                ib = ldbox(tmp.box, i);
-                copy_item(tmp, i, it, i);
-            } else {
-                ib = ldbox(it.box, i);
-            }
-            const int side = (i < mid) ? 0 : 1;
-            for (int q = 0; q < 3; q++) {
-                mn[side][q] = min(mn[side][q], fkey(ib.lo[q]));
-                mx[side][q] = max(mx[side][q], fkey(ib.hi[q]));
-            }
-        }
-        for (int sd = 0; sd < 2; sd++)
-            for (int q = 0; q < 3; q++) {
-                const uint32_t wmn = wave_min_u32(mn[sd][q]), wmx = wave_max_u32(mx[sd][q]);
-                if (lane == 0) {
-                    atomicMin(&s_box[sd][q], wmn);
-                    atomicMax(&s_box[sd][3 + q], wmx);
-                }
-            }
-        __syncthreads();
-        if (tid < 12) {
-            const int sd = tid / 6, q = tid % 6;
-            if (q < 3) atomicMin(&A->box[t][sd][q], s_box[sd][q]);
-            else atomicMax(&A->box[t][sd][q], s_box[sd][q]);
-        }
-        __syncthreads();
-    }
-}
-__global__ void __launch_bounds__(64) k_wide_final(int ntask, const int32_t* tb, const int32_t* te, const WideAcc* A,
-                                                   TopSplit* out) {
-    const int t = blockIdx.x, tid = threadIdx.x;
-    if (t >= ntask) return;
-    if (tid < 12) out[t].box[tid / 6][tid % 6] = fromkey(A->box[t][tid / 6][tid % 6]);
-    if (tid == 0) out[t].mid = A->axis[t] < 0 ? (tb[t] + te[t]) / 2 : tb[t] + A->nleft[t];
-}
-
-// Levels of many small nodes: one wave per node (four per workgroup), each
-// with its own LDS bins; the same bounds, bins, split, stable partition and
-// child boxes as k_top_split, with wave reductions and ballots in place of the
-// workgroup's.  A node of any size is handled (in rounds of 64 items).
-constexpr int kWaveSplitMin = 1024;      // levels of more nodes than this use the wave form
-__global__ void __launch_bounds__(256) k_top_split_wave(int ntask, Items it, Items tmp, const int32_t* task_b,
-                                                        const int32_t* task_e, TopSplit* out) {
-    __shared__ uint32_t s_bin[kSplitWaves][3][kBins][6];
-    __shared__ int32_t s_cnt[kSplitWaves][3][kBins];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int t = blockIdx.x * kSplitWaves + wv;
-    const bool active = t < ntask;       // uniform over the wave
-    const int b = active ? task_b[t] : 0, e = active ? task_e[t] : 0;
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const uint32_t kinf = fkey(__builtin_huge_valf()), kninf = fkey(-__builtin_huge_valf());
-    for (int j = lane; j < 3 * kBins * 6; j += 64) (&s_bin[wv][0][0][0])[j] = ((j % 6) < 3) ? kinf : kninf;
-    for (int j = lane; j < 3 * kBins; j += 64) (&s_cnt[wv][0][0])[j] = 0;
-    // centroid bounds
-    float lo[3], ext[3];
-    {
-        uint32_t mn[3] = {kinf, kinf, kinf}, mx[3] = {kninf, kninf, kninf};
-        for (int i = b + lane; i < e; i += 64)
-            for (int a = 0; a < 3; a++) {
-                const uint32_t k = fkey(item_c(it, a, i));
-                mn[a] = min(mn[a], k);
-                mx[a] = max(mx[a], k);
-            }
-        for (int a = 0; a < 3; a++) {
-            lo[a] = fromkey(wave_min_u32(mn[a]));
-            ext[a] = fromkey(wave_max_u32(mx[a])) - lo[a];
-        }
+    // left items of the node's chunks before this one, and of the waves' parts of it
+    int32_t before = 0;
+    for (int j = tid; j < (g - f) * 16; j += 64 * kTopWaves)
+        if ((j & 15) <= s.split) before += B.chunk_items[(size_t)(f + (j >> 4)) * 48 + 16 * s.axis + (j & 15)];
+    for (int d = 32; d > 0; d >>= 1) before += __shfl_xor(before, d);
+    constexpr int kPart = kWideChunk / kTopWaves;
+    const int wb = min(b + wv * kPart, e), we = min(wb + kPart, e);
+    int32_t left = 0;
+    for (int i = wb + lane; i < we; i += 64) left += bin_of(item_c(src, s.axis, i), s.lo, s.scale) <= s.split ? 1 : 0;
+    for (int d = 32; d > 0; d >>= 1) left += __shfl_xor(left, d);
+    if (lane == 0) {
+        s_left[wv] = left;
+        s_before[wv] = before;
     }
     __syncthreads();
-    for (int i = b + lane; i < e; i += 64) {
-        const DBox ib = ldbox(it.box, i);
-        const int cnt = it.count[i];
-        for (int a = 0; a < 3; a++) {
-            if (!(ext[a] > 0.0f)) continue;
-            const float scale = (float)kBins / ext[a];
-            const int bi = bin_of(item_c(it, a, i), lo[a], scale);
-            for (int q = 0; q < 3; q++) {
-                atomicMin(&s_bin[wv][a][bi][q], fkey(ib.lo[q]));
-                atomicMax(&s_bin[wv][a][bi][3 + q], fkey(ib.hi[q]));
-            }
-            atomicAdd(&s_cnt[wv][a][bi], cnt);
-        }
-    }
-    __syncthreads();
-    int32_t axis = -1, split = -1;
-    if (active) sah_choose_wave(s_bin[wv], s_cnt[wv], ext, &axis, &split);
-    int mid = (b + e) / 2;
-    if (axis >= 0) {
-        const float scale = (float)kBins / ext[axis], l0 = lo[axis];
-        int nleft = 0;
-        for (int start = b; start < e; start += 64) {
-            const int i = start + lane;
-            const bool left = i < e && bin_of(item_c(it, axis, i), l0, scale) <= split;
-            nleft += __popcll(__ballot(left));
-        }
-        int lrun = b, rrun = b + nleft;
-        for (int start = b; start < e; start += 64) {
-            const int i = start + lane;
-            const bool has = i < e;
-            const bool left = has && bin_of(item_c(it, axis, i), l0, scale) <= split;
-            const unsigned long long ml = __ballot(left), mr = __ballot(has && !left);
-            if (has) copy_item(it, i, tmp, left ? lrun + __popcll(ml & below) : rrun + __popcll(mr & below));
-            lrun += __popcll(ml);
-            rrun += __popcll(mr);
-        }
-        mid = b + nleft;
-    }
-    __syncthreads();      // the partition's global writes are visible to the wave's other lanes
-    uint32_t mn[2][3], mx[2][3];
-    for (int sd = 0; sd < 2; sd++)
-        for (int q = 0; q < 3; q++) { mn[sd][q] = kinf; mx[sd][q] = kninf; }
-    for (int i = b + lane; i < e; i += 64) {
-        DBox ib;
-        if (axis >= 0) {
-            ib = ldbox(tmp.box, i);
-            copy_item(tmp, i, it, i);
-        } else {
-            ib = ldbox(it.box, i);
-        }
-        const int side = (i < mid) ? 0 : 1;
-        for (int q = 0; q < 3; q++) {
-            mn[side][q] = min(mn[side][q], fkey(ib.lo[q]));
-            mx[side][q] = max(mx[side][q], fkey(ib.hi[q]));
-        }
-    }
-    float bx[12];
-    for (int sd = 0; sd < 2; sd++)
-        for (int q = 0; q < 3; q++) {
-            bx[sd * 6 + q] = fromkey(wave_min_u32(mn[sd][q]));
-            bx[sd * 6 + 3 + q] = fromkey(wave_max_u32(mx[sd][q]));
-        }
-    if (active && lane < 12) {
-        float v = bx[0];
-        for (int j = 1; j < 12; j++) v = (lane == j) ? bx[j] : v;
-        out[t].box[lane / 6][lane % 6] = v;
-    }
-    if (active && lane == 0) out[t].mid = mid;
+    int l = 0;
+    for (int w = 0; w < kTopWaves; w++) l += s_before[w] + (w < wv ? s_left[w] : 0);
+    partition_items(src, dst, wb, we, s.axis, s.lo, s.scale, s.split, tb + l, s.mid + (wb - tb) - l);
 }
 
-// Numbering of a level's inner children as an exclusive scan over the nodes:
-// k_link_count gives each node its number of inner children (child ranges of
-// more than one item), the scan their first number, k_link_write the children
-// (breadth-first numbering, left before right, as k_top_link), k_link_finish
-// the next level's size and the next free node id.
-__global__ void __launch_bounds__(256) k_link_count(int ntask, const int32_t* task_b, const int32_t* task_e,
-                                                    const TopSplit* sp, int32_t* inner) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntask) return;
-    const int b = task_b[t], e = task_e[t], mid = sp[t].mid;
-    inner[t] = (mid - b > 1 ? 1 : 0) + (e - mid > 1 ? 1 : 0);
+// empty lists, counters and accumulators (slots: middle slots; words: of the wide accumulators)
+__global__ void __launch_bounds__(256) k_top_clear(TopBuild B, int slots, int words) {
+    const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+    for (int i = i0; i < 2 * slots; i += stride) {
+        TopTask* t = B.mid[i >= slots ? 1 : 0] + (i >= slots ? i - slots : i);
+        t->b = t->e = 0;
+    }
+    for (int i = i0; i < kRegions * 64; i += stride) B.nsmall[i] = 0;
+    for (int i = i0; i < kLevels; i += stride) B.any[i] = 0;
+    for (int i = i0; i < 6; i += stride) B.cb[i] = acc_empty(i);
+    for (int i = i0; i < words; i += stride) B.acc[i] = acc_empty(i / 48 % kAccWords);
 }
-__global__ void __launch_bounds__(256) k_link_write(int ntask, const int32_t* task_b, const int32_t* task_e,
-                                                    const int32_t* task_node, const TopSplit* sp, const int32_t* item_ref,
-                                                    const int32_t* first, BvhNode* nodes, int32_t* next_b, int32_t* next_e,
-                                                    int32_t* next_node, const int32_t* next_id) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntask) return;
-    const int b = task_b[t], e = task_e[t], mid = sp[t].mid;
-    const int rb[2] = {b, mid}, re[2] = {mid, e};
-    const int32_t id0 = *next_id;
-    int q = first[t];
-    BvhNode* nd = nodes + task_node[t];
+// centroid bounds of all items
+__global__ void __launch_bounds__(256) k_top_bounds(TopBuild B) {
+    __shared__ uint32_t s_cb[4][6];
+    uint32_t v[6];
+    for (int q = 0; q < 6; q++) v[q] = acc_empty(q);
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < B.m; i += gridDim.x * 256)
+        for (int a = 0; a < 3; a++) {
+            const uint32_t c = fkey(item_c(B.it[0], a, i));
+            v[a] = min(v[a], c);
+            v[3 + a] = max(v[3 + a], c);
+        }
+    for (int q = 0; q < 6; q++) {
+        for (int d = 32; d > 0; d >>= 1) v[q] = acc_union(q, v[q], (uint32_t)__shfl_xor((int)v[q], d));
+        if ((threadIdx.x & 63) == 0) s_cb[threadIdx.x >> 6][q] = v[q];
+    }
+    __syncthreads();
+    const int q = threadIdx.x;
+    if (q < 6) {
+        uint32_t x = s_cb[0][q];
+        for (int w = 1; w < 4; w++) x = acc_union(q, x, s_cb[w][q]);
+        if (q < 3) atomicMin(B.cb + q, x);
+        else atomicMax(B.cb + q, x);
+    }
+}
+__global__ void k_top_root(TopBuild B) {
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    TopTask t;
+    t.b = 0; t.e = B.m; t.up = 0;
+    for (int q = 0; q < 6; q++) t.cb[q] = B.cb[q];
+    if (B.wide_levels > 0) {
+        B.wide[0][0] = t;
+    } else if (B.m > kSmallItems) {
+        B.mid[0][mid_slot(0)] = t;
+    } else {
+        B.small[0] = {0, B.m, 0, 0};
+        B.nsmall[0] = 1;
+    }
+}
+// node r: the r-th boundary in (level, boundary) order
+__global__ void __launch_bounds__(256) k_top_write(TopBuild B, const uint32_t* ids, const int32_t* number, BvhNode* nodes) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= B.m - 1) return;
+    const TopRec rec = B.rec[ids[r] + 1];
     for (int side = 0; side < 2; side++) {
         DBox bx;
-        for (int k = 0; k < 3; k++) { bx.lo[k] = sp[t].box[side][k]; bx.hi[k] = sp[t].box[side][3 + k]; }
-        int32_t ref;
-        if (re[side] - rb[side] == 1) {
-            ref = item_ref[rb[side]];
-        } else {
-            ref = id0 + q;
-            next_b[q] = rb[side]; next_e[q] = re[side]; next_node[q] = ref;
-            q++;
-        }
-        set_child(nd, side, bx, ref);
-    }
-}
-__global__ void k_link_finish(int ntask, const int32_t* inner, const int32_t* first, int32_t* next_id, int32_t* next_count) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const int32_t n = first[ntask - 1] + inner[ntask - 1];
-    *next_count = n;
-    *next_id += n;
-}
-
-// Numbers the inner children of one level (one workgroup; `next_id` holds the
-// next free top-level node id) and writes the parents' children.
-__global__ void __launch_bounds__(kTopThreads) k_top_link(int ntask, const int32_t* task_b, const int32_t* task_e,
-                                                          const int32_t* task_node, const TopSplit* sp, const int32_t* item_ref,
-                                                          BvhNode* nodes, int32_t* next_b, int32_t* next_e,
-                                                          int32_t* next_node, int32_t* next_id, int32_t* next_count) {
-    __shared__ int32_t s_scan[kTopThreads];
-    __shared__ int32_t s_base, s_id;
-    const int tid = threadIdx.x;
-    if (tid == 0) { s_base = 0; s_id = *next_id; }
-    __syncthreads();
-    for (int start = 0; start < ntask; start += kTopThreads) {
-        const int t = start + tid;
-        int rb[2] = {0, 0}, re[2] = {0, 0}, inner = 0;
-        if (t < ntask) {
-            const int b = task_b[t], e = task_e[t], mid = sp[t].mid;
-            rb[0] = b; re[0] = mid; rb[1] = mid; re[1] = e;
-            inner = (re[0] - rb[0] > 1 ? 1 : 0) + (re[1] - rb[1] > 1 ? 1 : 0);
-        }
-        s_scan[tid] = inner;
-        __syncthreads();
-        for (int off = 1; off < kTopThreads; off <<= 1) {
-            int v = (tid >= off) ? s_scan[tid - off] : 0;
-            __syncthreads();
-            s_scan[tid] += v;
-            __syncthreads();
-        }
-        if (t < ntask) {
-            int q = s_base + s_scan[tid] - inner;
-            BvhNode* nd = nodes + task_node[t];
-            for (int side = 0; side < 2; side++) {
-                DBox bx;
-                for (int k = 0; k < 3; k++) { bx.lo[k] = sp[t].box[side][k]; bx.hi[k] = sp[t].box[side][3 + k]; }
-                int32_t ref;
-                if (re[side] - rb[side] == 1) {
-                    ref = item_ref[rb[side]];
-                } else {
-                    ref = s_id + q;
-                    next_b[q] = rb[side]; next_e[q] = re[side]; next_node[q] = ref;
-                    q++;
-                }
-                set_child(nd, side, bx, ref);
-            }
-        }
-        __syncthreads();
-        if (tid == 0) s_base += s_scan[kTopThreads - 1];
-        __syncthreads();
-    }
-    if (tid == 0) {
-        *next_count = s_base;
-        *next_id = s_id + s_base;
+        for (int k = 0; k < 3; k++) { bx.lo[k] = rec.box[side][k]; bx.hi[k] = rec.box[side][3 + k]; }
+        const int32_t c = rec.child[side], kind = rec.kind[side];
+        int32_t ref = c;
+        if (kind == kChildNode) ref = number[c - 1];
+        else if (kind >= kChildItem) ref = kind == kChildItem ? B.it[0].ref[c] : B.it[1].ref[c];
+        set_child(nodes + r, side, bx, ref);
     }
 }
 
@@ -1594,8 +1602,10 @@ struct Tmp {
     }
 };
 inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)std::max<int64_t>(1, (n + b - 1) / b); }
-// node ids of `n` keyed nodes in level order, and the levels' first positions on the host (kLevels + 1)
-int order_levels(srt_ctx* c, Tmp& tmp, int n, const uint8_t* key, uint32_t* ids, std::vector<int32_t>& first) {
+// node ids of `n` keyed nodes in level order; `number` (or null) the nodes' positions, `first` (or null) the levels'
+// first positions on the host (kLevels + 1), for which it waits
+int order_levels(srt_ctx* c, Tmp& tmp, int n, const uint8_t* key, uint32_t* ids, int32_t* number,
+                 std::vector<int32_t>* first) {
     const int pieces = (int)nblk(n, kLevelPiece);
     int32_t* hist = tmp.get<int32_t>((size_t)kLevels * pieces);
     int32_t* size = tmp.get<int32_t>(kLevels);
@@ -1604,9 +1614,10 @@ int order_levels(srt_ctx* c, Tmp& tmp, int n, const uint8_t* key, uint32_t* ids,
     hipStream_t st = c->stream;
     k_level_hist<<<pieces, 256, 0, st>>>(n, key, pieces, hist);
     k_level_scan<<<kLevels, 256, 0, st>>>(pieces, hist, size);
-    k_level_rank<<<pieces, 256, 0, st>>>(n, key, pieces, hist, size, ids, dfirst);
-    first.resize(kLevels + 1);
-    if (int r = hip_check(c, hipMemcpyAsync(first.data(), dfirst, 4 * first.size(), hipMemcpyDeviceToHost, st), "copy"))
+    k_level_rank<<<pieces, 256, 0, st>>>(n, key, pieces, hist, size, ids, number, dfirst);
+    if (!first) return SRT_OK;
+    first->resize(kLevels + 1);
+    if (int r = hip_check(c, hipMemcpyAsync(first->data(), dfirst, 4 * first->size(), hipMemcpyDeviceToHost, st), "copy"))
         return r;
     return hip_check(c, hipStreamSynchronize(st), "level order");
 }
@@ -1674,7 +1685,7 @@ int bvh_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
         if (tmp.failed) return set_err(c, SRT_E_OOM, "depth scratch");
         k_radix_depth<<<nblk(m), 256, 0, st>>>(m, par_int, dkey);
         std::vector<int32_t> df;
-        if (int r = order_levels(c, tmp, m, dkey, dids, df)) return r;
+        if (int r = order_levels(c, tmp, m, dkey, dids, nullptr, &df)) return r;
         int dmax = 0;
         while (dmax + 1 < kLevels && df[dmax + 1] < m) dmax++;
         if (dmax >= kLevelNone - 1) return set_err(c, SRT_E_LIMIT, "radix tree depth %d exceeds %d", dmax, kLevelNone - 2);
@@ -1729,72 +1740,64 @@ int bvh_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
 
     int32_t root;
     if (m > 1) {
-        Items it, it2;
-        auto mk_items = [&](Items& x) {
+        TopBuild B;
+        B.m = m;
+        B.wide_levels = 0;
+        while (B.wide_levels < kWideLevels && (m >> B.wide_levels) > kWideMin) B.wide_levels++;
+        for (Items& x : B.it) {
             x.box.lox = tmp.get<float>(m); x.box.loy = tmp.get<float>(m); x.box.loz = tmp.get<float>(m);
             x.box.hix = tmp.get<float>(m); x.box.hiy = tmp.get<float>(m); x.box.hiz = tmp.get<float>(m);
             x.cx = tmp.get<float>(m); x.cy = tmp.get<float>(m); x.cz = tmp.get<float>(m);
             x.count = tmp.get<int32_t>(m); x.ref = tmp.get<int32_t>(m);
-        };
-        mk_items(it);
-        mk_items(it2);
-        int32_t* lb[2] = {tmp.get<int32_t>(m), tmp.get<int32_t>(m)};
-        int32_t* le[2] = {tmp.get<int32_t>(m), tmp.get<int32_t>(m)};
-        int32_t* ln[2] = {tmp.get<int32_t>(m), tmp.get<int32_t>(m)};
-        TopSplit* sp = tmp.get<TopSplit>(m);
-        WideAcc* wacc = tmp.get<WideAcc>(1);
-        int32_t* link_inner = tmp.get<int32_t>(m);
-        int32_t* link_first = tmp.get<int32_t>(m);
-        size_t link_bytes = 0;
-        (void)hipcub::DeviceScan::ExclusiveSum(nullptr, link_bytes, link_inner, link_first, m, st);
-        void* link_tmp = tmp.get<char>(link_bytes);
-        int32_t* chunk_left = tmp.get<int32_t>((size_t)m / kWideChunk + kWideTasks + 1);
-        int32_t* ctr = tmp.get<int32_t>(2);     // next free node id, next level size
-        if (tmp.failed || !ctr || !link_tmp) return set_err(c, SRT_E_OOM, "top-level scratch");
-        k_items<<<nblk(m), 256, 0, st>>>(m, clusters, order, tb, K, kfirst, top, it);
-        // level 0: the root (node 0) over all items; ids 1.. follow breadth-first
-        k_fill_i32<<<1, 64, 0, st>>>(lb[0], 1, 0);
-        k_fill_i32<<<1, 64, 0, st>>>(le[0], 1, m);
-        k_fill_i32<<<1, 64, 0, st>>>(ln[0], 1, 0);
-        k_fill_i32<<<1, 64, 0, st>>>(ctr, 1, 1);
-        int ntask = 1, cur = 0;
-        while (ntask > 0) {
-            if (ntask <= kWideTasks) {
-                // chunks of the level: at most m / kWideChunk + one partial chunk per node
-                const int grid = std::min(kWideMaxGrid, m / kWideChunk + ntask);
-                k_wide_init<<<8, 256, 0, st>>>(ntask, wacc);
-                k_wide_bounds<<<grid, 256, 0, st>>>(ntask, lb[cur], le[cur], it, wacc);
-                k_wide_bins<<<grid, 256, 0, st>>>(ntask, lb[cur], le[cur], it, wacc);
-                k_wide_sah<<<ntask, 64, 0, st>>>(wacc);
-                k_wide_count<<<grid, 256, 0, st>>>(ntask, lb[cur], le[cur], it, wacc, chunk_left);
-                k_wide_scatter<<<grid, 256, 0, st>>>(ntask, lb[cur], le[cur], it, it2, wacc, chunk_left);
-                k_wide_boxes<<<grid, 256, 0, st>>>(ntask, lb[cur], le[cur], it, it2, wacc);
-                k_wide_final<<<ntask, 64, 0, st>>>(ntask, lb[cur], le[cur], wacc, sp);
-            } else if (ntask <= kWaveSplitMin) {
-                k_top_split<<<ntask, kSplitThreads, 0, st>>>(it, it2, lb[cur], le[cur], sp);
-            } else {
-                k_top_split_wave<<<(ntask + kSplitWaves - 1) / kSplitWaves, 256, 0, st>>>(ntask, it, it2, lb[cur], le[cur],
-                                                                                           sp);
-            }
-            if (ntask <= kTopThreads) {
-                k_top_link<<<1, kTopThreads, 0, st>>>(ntask, lb[cur], le[cur], ln[cur], sp, it.ref, nodes, lb[cur ^ 1],
-                                                      le[cur ^ 1], ln[cur ^ 1], ctr, ctr + 1);
-            } else {
-                k_link_count<<<nblk(ntask), 256, 0, st>>>(ntask, lb[cur], le[cur], sp, link_inner);
-                if (int r = hip_check(c, hipcub::DeviceScan::ExclusiveSum(link_tmp, link_bytes, link_inner, link_first, ntask, st),
-                                      "link scan"))
-                    return r;
-                k_link_write<<<nblk(ntask), 256, 0, st>>>(ntask, lb[cur], le[cur], ln[cur], sp, it.ref, link_first, nodes,
-                                                          lb[cur ^ 1], le[cur ^ 1], ln[cur ^ 1], ctr);
-                k_link_finish<<<1, 64, 0, st>>>(ntask, link_inner, link_first, ctr, ctr + 1);
-            }
-            int32_t next = 0;
-            if (int r = hip_check(c, hipMemcpyAsync(&next, ctr + 1, 4, hipMemcpyDeviceToHost, st), "top level")) return r;
-            if (int r = hip_check(c, hipStreamSynchronize(st), "top level")) return r;
-            if (next > m) return set_err(c, SRT_E_LIMIT, "top-level build overflow");
-            ntask = next;
-            cur ^= 1;
         }
+        const int slots = mid_slots(m), wide_slots = 1 << std::max(B.wide_levels - 1, 0);
+        const int acc_words = B.wide_levels > 0 ? wide_slots * kWideCopies * kAccTotal : 0;
+        B.rec = tmp.get<TopRec>(m);
+        B.level = tmp.get<uint8_t>(m);
+        for (int k = 0; k < 2; k++) {
+            B.wide[k] = tmp.get<TopTask>(wide_slots);
+            B.mid[k] = tmp.get<TopTask>(slots);
+        }
+        B.small = tmp.get<SmallTask>((size_t)region_base(m, kRegions));
+        B.nsmall = tmp.get<int32_t>(kRegions * 64);
+        B.any = tmp.get<int32_t>(kLevels);
+        B.cb = tmp.get<uint32_t>(6);
+        B.acc = tmp.get<uint32_t>(acc_words);
+        B.chunk_items = tmp.get<int32_t>(((size_t)m / kWideChunk + wide_slots) * 48);
+        B.wsplit = tmp.get<WideSplit>(wide_slots);
+        uint32_t* ids = tmp.get<uint32_t>(m);
+        int32_t* number = tmp.get<int32_t>(m);
+        if (tmp.failed) return set_err(c, SRT_E_OOM, "top-level scratch");
+        k_items<<<nblk(m), 256, 0, st>>>(m, clusters, order, tb, K, kfirst, top, B.it[0]);
+        k_top_clear<<<std::min(nblk(std::max(2 * slots, acc_words)), 1024u), 256, 0, st>>>(B, slots, acc_words);
+        k_top_bounds<<<std::min(nblk(m), 128u), 256, 0, st>>>(B);
+        k_top_root<<<1, 64, 0, st>>>(B);
+        int L = 0;
+        for (; L < B.wide_levels; L++) {
+            // every chunk but a node's last one is full
+            const int chunks = m / kWideChunk + (1 << L);
+            k_top_wide_bins<<<chunks, 64 * kTopWaves, 0, st>>>(B, L);
+            k_top_wide_sah<<<1 << L, 64, 0, st>>>(B, L);
+            k_top_wide_scatter<<<chunks, 64 * kTopWaves, 0, st>>>(B, L);
+        }
+        // The middle levels of a tree half as deep again as a balanced one are
+        // queued at once, then four at a time until a level has no middle node:
+        // an empty one costs up to 13 us, a wait 45 us (the 1M-triangle field has
+        // 23 levels above its small nodes, a balanced tree would have 14).
+        int balanced = 0;
+        while ((m >> balanced) > kSmallItems) balanced++;
+        for (int to = 3 * balanced / 2 + 2; balanced > 0; to += 4) {
+            if (to >= kLevelNone) return set_err(c, SRT_E_LIMIT, "BVH depth exceeds the traversal limit %d", kMaxDepth);
+            for (; L < to; L++)
+                k_top_mid<<<nblk(slots, kMidSlots), 64 * kTopWaves, 0, st>>>(B, L, slots);
+            int32_t more = 0;
+            if (int r = hip_check(c, hipMemcpyAsync(&more, B.any + L, 4, hipMemcpyDeviceToHost, st), "top level")) return r;
+            if (int r = hip_check(c, hipStreamSynchronize(st), "top level")) return r;
+            if (!more) break;
+        }
+        k_top_small<<<kRegions * kRegionBlocks, 64 * kTopWaves, 0, st>>>(B);
+        if (int r = order_levels(c, tmp, top, B.level, ids, number, nullptr)) return r;
+        k_top_write<<<nblk(top), 256, 0, st>>>(B, ids, number, nodes);
         k_fill_i32<<<nblk(top), 256, 0, st>>>(valid, top, 1);
         root = 0;
     } else if (n == 1) {
@@ -1818,7 +1821,7 @@ int bvh_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
         if (tmp.failed) return set_err(c, SRT_E_OOM, "level scratch");
         k_node_level<<<nblk(num_nodes), 256, 0, st>>>(num_nodes, valid, parent, lkey);
         std::vector<int32_t> hf;
-        if (int r = order_levels(c, tmp, num_nodes, lkey, (uint32_t*)s->level_nodes.p, hf)) return r;
+        if (int r = order_levels(c, tmp, num_nodes, lkey, (uint32_t*)s->level_nodes.p, nullptr, &hf)) return r;
         while (depth < kLevelNone && hf[depth] < hf[kLevelNone]) depth++;
         if (depth > kMaxDepth)
             return set_err(c, SRT_E_LIMIT, "BVH depth %d exceeds the traversal limit %d", depth, kMaxDepth);

@@ -76,6 +76,43 @@ def test_leaf_sizes(ctx, leaf):
     _compare(ctx, _soup(3000, seed=4), max_leaf=leaf, cluster_size=64)
 
 
+def _points(c, size=0.01):
+    """Small triangles around the given centres."""
+    c = np.asarray(c, np.float64)
+    v = c[:, None, :] + size * np.array([[-1, -1, 0], [1, -1, 0], [0, 2, 0]])
+    n = len(c)
+    return scenes.SceneData(positions=v.reshape(-1, 3).astype(np.float32),
+                            indices=np.arange(3 * n, dtype=np.uint32).reshape(n, 3),
+                            mesh_first=np.array([0, n], np.int32), mesh_material=np.array([0], np.int32),
+                            materials=np.asarray([scenes.material()], scenes.MAT_DTYPE))
+
+
+# one triangle per cluster: pairs, one wave's subtrees (21 items), nodes of one
+# wave and of four (256), with and without wide levels (1024, 512 per chunk)
+@pytest.mark.parametrize("n", [2, 3, 20, 21, 22, 23, 45, 255, 256, 257, 258, 1023, 1024, 1025, 1537, 2048, 2050, 9001])
+def test_top_level_node_sizes(ctx, n):
+    info = _compare(ctx, _soup(n, seed=100 + n), max_leaf=1, cluster_size=1)
+    assert info["clusters"] == n
+
+
+@pytest.mark.parametrize("n", [2, 5, 21, 22, 257, 1025, 3000])
+@pytest.mark.parametrize("kind", ["one_point", "line", "two_points", "skewed"])
+def test_top_level_degenerate_items(ctx, kind, n):
+    """Items that no boundary separates (one centroid: halves in order), a
+    single axis with an extent, many items in two places, and distances that
+    shrink by a constant factor (deep, unbalanced trees)."""
+    i = np.arange(n, dtype=np.float64)
+    if kind == "one_point":
+        c = np.zeros((n, 3))
+    elif kind == "line":
+        c = np.stack([0 * i, i, 0 * i], 1)
+    elif kind == "two_points":
+        c = np.stack([(i % 2) * 5, 0 * i, (i % 2) * -3], 1)
+    else:
+        c = np.stack([4.0 ** -(i % 40), np.sin(i) * 1e-3, 2.0 ** -(i % 70)], 1)
+    _compare(ctx, _points(c), max_leaf=1, cluster_size=1)
+
+
 def test_cluster_size_below_leaf_size_is_raised(ctx):
     info = _compare(ctx, _soup(2000, seed=11), max_leaf=8, cluster_size=2)
     assert info["cluster_size"] == 8
