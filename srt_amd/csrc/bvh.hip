@@ -10,16 +10,16 @@
 //   1. triangle boxes, box centroids, centroid bounds (two-level reduction)
 //   2. 63-bit Morton codes of centroids, stable radix sort of (code, id)
 //   3. Karras (HPG 2012) binary radix tree, index tie-break for equal codes
-//   4. bottom-up pass, one launch per radix-tree depth (deepest first, nodes
-//      sorted by depth): boxes, primitive counts, SAH costs, collapse-to-leaf
+//   4. bottom-up pass by radix-tree depth (deepest first, nodes ordered by
+//      depth, runs of small levels in one launch): boxes, primitive counts, SAH costs, collapse-to-leaf
 //      decisions (leaves of <= max_leaf triangles)
 //   5. frontier of the highest subtrees with <= T primitives ("clusters")
-//   6. top of the tree rebuilt with a 16-bin SAH sweep over the clusters, in one
-//      workgroup, breadth-first node numbering
+//   6. top of the tree rebuilt with a 16-bin SAH sweep over the clusters, by
+//      levels, breadth-first node numbering at the end
 //   7. emit 64-byte nodes (two child boxes per node) and the triangles in
 //      Morton order (48 bytes each, primitive and mesh id in the w lanes)
-// Refit keeps the topology and recomputes child boxes bottom-up, one launch per
-// tree level.  Kernel boundaries order the levels: per-node device-scope fences
+// Refit keeps the topology and recomputes child boxes bottom-up by levels.
+// Kernel boundaries (barriers in a run of small levels) order them: per-node device-scope fences
 // (an L2 write-back and invalidate each on gfx950) made the arrival-counter
 // form of these passes several times slower.
 #include "srt_internal.h"
@@ -1592,7 +1592,7 @@ namespace {
 // device chunks.  The chunks go back to the context when the build ends and
 // the next build takes them again (the smallest kept chunk that fits), so a
 // rebuild of the same scene calls neither hipMalloc nor hipFree: each hipFree
-// of a chunk cost about 0.25 ms of host time, a third of a 1M-triangle
+// of a chunk cost about 0.25 ms of host time, 18 chunks for a 1M-triangle
 // rebuild.  Kernels of a build still queued when its chunks go back are
 // ordered before the next build's by the context's stream.
 struct Tmp {
@@ -1688,7 +1688,7 @@ int bvh_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
     hipStream_t st = c->stream;
     // default: clusters of at most 4 triangles under the binned-SAH top (at
     // most 2^18 clusters): 3.5 % faster traversal than 64 on the 1M-triangle
-    // field, for a build of about 0.1 us per triangle
+    // field, for a build of about 3 ns per triangle
     // a cluster holds at least a leaf's triangles: a collapsed (leaf) subtree
     // never spans the cluster frontier
     const int T = std::max(max_leaf, cluster_size > 0 ? cluster_size : std::max(kAutoClusterMin, n / kAutoClusterDiv));
@@ -1735,7 +1735,7 @@ int bvh_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
     k_fill_i32<<<nblk(n), 256, 0, st>>>(par_int, n, -1);
     if (n > 1) {
         k_karras<<<nblk(n - 1), 256, 0, st>>>(keys2, n, kl, kr, kfirst, par_int, par_leaf);
-        // bottom-up by depth: the n - 1 radix-tree nodes ordered by depth, then one launch per depth
+        // bottom-up by depth: the n - 1 radix-tree nodes ordered by depth
         const int m = n - 1;
         uint8_t* dkey = tmp.get<uint8_t>(m);
         uint32_t* dids = tmp.get<uint32_t>(m);
