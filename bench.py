@@ -155,7 +155,8 @@ def pmc_summary(fetch_dir, write_dir, copy_fetch_dir, copy_write_dir):
              "gpurun_out/pmc_copy_FETCH_SIZE gpurun_out/pmc_copy_WRITE_SIZE", "",
              "Each rocprofv3 run: cd /tmp && export TMPDIR=/tmp, bench.py by its path in the repository.",
              "The frame runs hold one counting pass (k_trace<true, true>/k_shadow<true, true>, not counted here; its k_shade",
-             "dispatches are) and one frame; trace is k_trace_cam (first bounce) and k_trace (later bounces);",
+             "dispatches are) and one frame; trace is k_trace_cam (first bounce) and k_trace (later bounces, until k_paths",
+             "finishes the last 2^20 paths);",
              "FETCH_SIZE/WRITE_SIZE are the L2-to-fabric bytes (MALL or HBM).", "",
              f"Calibration: copy kernel of {COPY_ELEMS * 4} B read + {COPY_ELEMS * 4} B written: "
              f"FETCH_SIZE {cf:.1f} KiB, WRITE_SIZE {cw:.1f} KiB per dispatch -> factors fetch {ff:.4f}, "
@@ -199,7 +200,7 @@ def valu_summary(d):
              "    python3 bench.py --valu-summary gpurun_out/pmc_valu", "",
              "The rocprofv3 run: cd /tmp && export TMPDIR=/tmp, bench.py by its path in the repository; the counting",
              "pass's k_trace<true, true>/k_shadow<true, true> are not counted here (its k_shade dispatches are); trace",
-             "is k_trace_cam (first bounce) and k_trace (later bounces).",
+             "is k_trace_cam (first bounce) and k_trace (later bounces, until k_paths finishes the last 2^20 paths).",
              f"busy = 4 SQ_ACTIVE_INST_VALU / ({MI355X_SIMDS} SIMDs x GRBM_GUI_ACTIVE / {MI355X_XCDS}), summed over the "
              "kernel's dispatches; lanes = SQ_THREAD_CYCLES_VALU / (64 SQ_ACTIVE_INST_VALU); wait = SQ_WAIT_ANY / "
              "SQ_WAVE_CYCLES.", "",
@@ -296,8 +297,8 @@ def kstats_summary(d, mode="frame"):
                  "--warmup 1",
                  "    python3 bench.py --kstats-summary gpurun_out/prof_skin --kstats-mode skin", "",
                  "The run builds the BVH once, then renders 1 warmup frame and 60 timed frames; every frame",
-                 "skins the tube (k_skin), refits the binary tree level by level (k_refit_level) and the 4-wide",
-                 "tree (k_refit4), then renders (k_trace_cam / k_trace, k_shade, k_shadow, k_finalize).", "",
+                 "skins the tube (k_skin), refits the binary tree level by level (k_refit_level, k_refit_run) and the 4-wide",
+                 "tree (k_refit4), then renders (k_trace_cam / k_trace, k_shade, k_shadow, k_paths, k_finalize).", "",
                  "| kernel | calls | total ms | average us | share |", "|---|---|---|---|---|"]
         out_file = SKIN_KSTATS_FILE
     elif mode == "passes":
@@ -330,10 +331,9 @@ def kstats_summary(d, mode="frame"):
                  "    python3 bench.py --kstats-summary gpurun_out/prof_ks", "",
                  "The run renders 6 frames: the untimed counting pass (k_trace_cam<true, true>, k_trace<true, true>,",
                  "k_shadow<true, true>), 1 warmup, 2 timed frames and 2 frames copied to host memory; the first bounce's",
-                 "closest hits run in k_trace_cam (camera rays computed from the slot), later ones in k_trace; the BVH",
-                 "build runs twice (cold, then a rebuild): the",
-                 "top-level SAH levels (k_wide_* for levels of <= 64 nodes, k_top_split, k_top_split_wave for levels of",
-                 "> 1024 nodes, k_top_link / k_link_*), k_bottom_up_level, sorts, 4-wide collapse.", "",
+                 "closest hits run in k_trace_cam (camera rays computed from the slot), later ones in k_trace until at most",
+                 "2^20 paths live, which k_paths finishes; the BVH build runs twice (cold, then a rebuild): top-level SAH",
+                 "(k_top_*), k_bottom_up_level / _run, the Morton sort, 4-wide collapse (k_c4_*).", "",
                  "| kernel | calls | total ms | average us | share |", "|---|---|---|---|---|"]
         out_file = KSTATS_FILE
     for n, c, t, a in rows[:16]:
