@@ -2524,8 +2524,8 @@ static int wait_live(srt_ctx* c, int64_t* n) {
     }
 }
 
-// Runs one chunk: segments (in slot order) of one scene share the path queues.
-int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, TrainOut* train) {
+// The stages of a chunk: segments (in slot order) of one scene share the path queues.
+static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, TrainOut* train) {
     if (nseg <= 0 || nseg > kMaxSegments) return set_err(c, SRT_E_LIMIT, "bad segment count %d", nseg);
     int64_t n = 0;
     int max_depth = 0, mlp_mode = 0;
@@ -2722,6 +2722,15 @@ int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, Train
     if (mlp_mode == 2 && train && train->count < train->cap)
         train->count = std::min<int64_t>(train->cap, train->count + __atomic_load_n(c->live + 1, __ATOMIC_SEQ_CST));
     return SRT_OK;
+}
+
+// Runs one chunk.  A chunk that fails part-way leaves kernels queued that still
+// write c->live, the queues and the caller's film: they end before the error is
+// returned, or the next chunk could take the old chunk's live count for its own.
+int run_chunk(srt_ctx* c, SceneRec* s, const Segment* segs_host, int nseg, TrainOut* train) {
+    const int r = chunk_stages(c, s, segs_host, nseg, train);
+    if (r) (void)hipStreamSynchronize(c->stream);
+    return r;
 }
 
 int render_wavefront(srt_ctx* c, SceneRec* s, const DevCamera& cam, const DevParams& p, float* film_dev, TrainOut* train) {

@@ -166,3 +166,38 @@ def test_hooks_equal_in_whole_path_kernel_and_queue_stages(ctx):
     assert out[0][:2] == out[1][:2] and out[0][1] > 1000
     assert np.array_equal(out[0][2], out[1][2])
     assert np.array_equal(out[0][3], out[1][3])
+
+
+def test_failed_training_frame_leaves_the_next_frame_alone():
+    """A training frame whose last allocation (the scan's scratch, after its
+    bounces are queued) exceeds the budget returns an error while millions of
+    its paths are still in flight; the context's next frame, which waits for
+    live-path counts of its own, is complete."""
+    from srt_amd import abi, scenes
+    s = scenes.cornell()
+    u, t = data(1 << 12, 1)
+
+    def frame(budget):
+        c = abi.Context(0, budget)
+        c.set_option("keep_build_scratch", 0)
+        h = c.upload(s)
+        c.build_bvh(h)
+        c.mlp_create(seed=3, lr=1e-3)
+        c.mlp_train_step(u, t)        # the training buffers: the scan's scratch is then the frame's last allocation
+        try:
+            c.mlp_train_frame(h, s.camera, 4000, 4000, 1, 3, 4, seed=9, max_samples=1 << 12, steps=1)
+            failed, used = False, c.hbm_used()
+        except abi.SrtError as e:
+            assert e.code == -4 and "budget" in str(e)
+            failed, used = True, None
+        img = c.render(h, s.camera, 1300, 1000, 1, 4, 4, 1, 1, 2)
+        counts = c.last_counts()
+        c.close()
+        return failed, used, img, counts
+
+    failed, used, ref, n = frame(0)
+    assert not failed and n[0] > 1300 * 1000
+    failed, _, img, m = frame(used - 1)
+    assert failed
+    assert m == n
+    assert np.array_equal(img, ref)
