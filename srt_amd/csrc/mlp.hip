@@ -659,6 +659,7 @@ static int refresh_copies(srt_ctx* c, MlpState* m) {
 
 static int ensure_train(srt_ctx* c, MlpState* m, int64_t n) {
     if (m->cap >= n) return SRT_OK;
+    m->cap = 0;                     // (nothing is held should an allocation fail)
     DevBuf* bs[] = {&m->wpart, &m->bpart, &m->loss_part, &m->tgt_buf};
     for (DevBuf* b : bs) dev_free(c, *b);
     // blocks of any step of at most n samples: ceil(n' / train_chunk(n')) <= max(256, ceil(n / 1024))
@@ -674,6 +675,7 @@ static int ensure_train(srt_ctx* c, MlpState* m, int64_t n) {
 
 static int ensure_in(srt_ctx* c, MlpState* m, int64_t n) {
     if (m->infer_cap >= n) return SRT_OK;
+    m->infer_cap = 0;
     dev_free(c, m->in_buf);
     dev_free(c, m->out_buf);
     int r = dev_alloc(c, m->in_buf, (size_t)n * 36);

@@ -793,6 +793,7 @@ int srt_mlp_train_frame(srt_ctx* c, srt_scene h, const srt_camera* cam, const sr
     if (p->samples_per_pixel <= 0 || p->max_depth < 3) return set_err(c, SRT_E_INVALID, "training paths need max_depth >= 3");
     if (int r = ensure_bvh(c, s)) return r;
     if (c->train_cap < max_samples) {
+        c->train_cap = 0;
         dev_free(c, c->train_in9);
         dev_free(c, c->train_t);
         if (int r = dev_alloc(c, c->train_in9, (size_t)max_samples * 36)) return r;

@@ -2479,6 +2479,7 @@ __global__ void __launch_bounds__(256) k_scatter_train(int n, const uint32_t* fl
 // per-slot buffers of the MLP hooks (allocated on first use, sized to the pool)
 static int ensure_mlp_bufs(srt_ctx* c, int64_t slots) {
     if (c->mlp_pool_cap >= slots) return SRT_OK;
+    c->mlp_pool_cap = 0;
     for (auto& b : c->mlpbuf) dev_free(c, b);
     const size_t n = (size_t)slots;
     const size_t qn = (size_t)kParts * part_cap((uint32_t)slots);   // partitioned appends (>= n)
@@ -2740,6 +2741,7 @@ int render_wavefront(srt_ctx* c, SceneRec* s, const DevCamera& cam, const DevPar
     if (pool > total) pool = total;
     if (pool > 0x7fffffff) pool = 0x7fffffff;
     if (c->film_pixels < wh) {
+        c->film_pixels = 0;
         dev_free(c, c->film_acc);
         if (dev_alloc(c, c->film_acc, (size_t)wh * 3 * sizeof(float))) return SRT_E_OOM;
         c->film_pixels = wh;

@@ -201,3 +201,53 @@ def test_failed_training_frame_leaves_the_next_frame_alone():
     assert failed
     assert m == n
     assert np.array_equal(img, ref)
+
+
+@pytest.mark.parametrize("refused", ["film", "samples", "hooks", "infer", "train"])
+def test_smaller_calls_work_after_a_refused_allocation(refused):
+    """A call whose buffers do not fit the budget frees the smaller ones it
+    would have replaced; the next smaller call allocates its own again."""
+    from srt_amd import abi, scenes
+    s = scenes.cornell()
+    small, large = data(1000, 4), data(1 << 22, 4)
+
+    def session(budget):
+        c = abi.Context(0, budget)
+        c.set_option("keep_build_scratch", 0)
+        c.set_option("path_pool", 3000)
+        h = c.upload(s)
+        c.build_bvh(h)
+        c.mlp_create(seed=3, lr=1e-3)
+        if refused == "hooks":
+            c.set_option("path_pool", 1 << 20)
+            c.render(h, s.camera, 1000, 1000, 1, 5, 4, 1, 1, 2)       # the path pool of the larger frame
+
+        def call(big):
+            if refused == "film":         # several chunks: the sums of the earlier ones are kept
+                return c.render(h, s.camera, *((2048, 2048, 1) if big else (64, 64, 2)), 5, 4, 1, 1, 2)
+            if refused == "samples":
+                return c.mlp_train_frame(h, s.camera, 64, 64, 1, 5, 4, seed=9, max_samples=1 << (22 if big else 12), steps=1)
+            if refused == "hooks":
+                return c.render(h, s.camera, *((1000, 1000) if big else (64, 48)), 1, 5, 4, 1, 1, 2, mlp_mode=1)
+            if refused == "infer":
+                return c.mlp_infer((large if big else small)[0])
+            return c.mlp_train_step(*(large if big else small), apply=False)
+
+        first = call(False)
+        if not budget:
+            used = c.hbm_used()
+            c.close()
+            return used
+        with pytest.raises(abi.SrtError) as e:
+            call(True)
+        assert e.value.code == -4
+        again = call(False)
+        c.close()
+        return first, again
+
+    # beyond the small calls' memory: the tree build's scratch, and the larger image's output film (64 MB)
+    first, again = session(session(0) + (65 << 20))
+    if refused == "samples":
+        assert first[1] == again[1] > 0       # (the weights moved on between them)
+    else:
+        assert np.array_equal(first, again)
