@@ -1727,7 +1727,8 @@ int bvh_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
     int32_t* tri_mesh = (int32_t*)s->tri_mesh.p;
     if (tmp.failed || !cen || !K.collapse) return set_err(c, SRT_E_OOM, "BVH build scratch exceeds the HBM budget");
 
-    // final outputs
+    // final outputs: the scene is without a tree until all of them are written
+    s->has_bvh = false;
     if (dev_realloc(c, s->order, (size_t)n * 4) || dev_realloc(c, s->tris, (size_t)n * 48)) return SRT_E_OOM;
     uint32_t* order = (uint32_t*)s->order.p;
 

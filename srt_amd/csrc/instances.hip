@@ -379,6 +379,7 @@ int inst_build(srt_ctx* c, SceneRec* s, int max_leaf, int cluster_size) {
                                         hipMemcpyHostToDevice, st), "top-level nodes");
     std::vector<int32_t> inst_root(s->ninst);
     for (int i = 0; i < s->ninst; i++) inst_root[i] = mesh_root[s->h_inst_mesh[i]];
+    s->has_bvh = false;               // until the arrays below have replaced the scene's
     dev_free(c, s->inst_root);
     if (!r) r = dev_alloc(c, s->inst_root, 4 * (size_t)s->ninst);
     if (!r) r = hip_check(c, hipMemcpyAsync(s->inst_root.p, inst_root.data(), 4 * (size_t)s->ninst, hipMemcpyHostToDevice, st),

@@ -188,3 +188,46 @@ def test_refit_identity_and_skin(ctx):
         assert np.array_equal(tris.view(np.uint32), tr.view(np.uint32))
         assert np.array_equal(nodes, nr)
     ctx.release(h)
+
+
+def test_refused_rebuild_leaves_no_half_built_tree():
+    """A rebuild that the memory budget refuses part-way leaves the scene with
+    its old tree or with none (the next render builds the default one): over a
+    sweep of budgets every later frame is one of the two trees' or SRT_E_OOM."""
+    from srt_amd import abi
+    s = scenes.tube()
+
+    def session(budget, rebuild):
+        c = abi.Context(0, budget)
+        c.set_option("keep_build_scratch", 0)
+        h = c.upload(s)
+        img = None
+        try:
+            c.build_bvh(h, cluster_size=0 if rebuild is None else 64)
+            c.render(h, s.camera, 64, 36, 1, 3, 4, 1, 1, 2)
+        except abi.SrtError:
+            c.close()
+            return "first", None
+        state, used = "built", c.hbm_used()
+        if rebuild:
+            try:
+                c.build_bvh(h, max_leaf=1, cluster_size=1)
+            except abi.SrtError as e:
+                assert e.code == -4
+                state = "refused"
+        try:
+            img = c.render(h, s.camera, 64, 36, 1, 3, 4, 1, 1, 2)
+        except abi.SrtError as e:
+            assert e.code == -4 and state == "refused"
+        c.close()
+        return state, img if budget else (img, used)
+
+    default = session(0, None)[1][0]
+    old, used = session(0, False)[1]
+    states = []
+    for mb in range(30, 160, 2):
+        state, img = session(used + (mb << 20), True)
+        states.append(state)
+        if state == "refused" and img is not None:
+            assert np.array_equal(img, old) or np.array_equal(img, default), mb
+    assert states.count("refused") >= 5 and states[-1] == "built"
