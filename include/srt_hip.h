@@ -124,7 +124,10 @@ const char* srt_last_error(const srt_ctx* ctx);
  * that makes the wave test them, 1..64; 0, the default: per-ray traversal; the
  * results are identical; packets gain 1 % of the closest-hit time on a scene
  * that fills the frame with deep traversals and lose 10 % where camera rays
- * visit few nodes), "keep_build_scratch" (1, the
+ * visit few nodes), "whole_paths" (a chunk's paths are finished in one launch
+ * that holds each in registers once at most this many live, 0..2^31 - 1, default
+ * 2^20; 0: bounce by bounce to the end; the results are identical),
+ * "keep_build_scratch" (1, the
  * default: the device scratch of a BVH build, and of a denoise pass up to 512 MiB,
  * stays allocated for the next one and counts in srt_hbm_used; it is freed when
  * an allocation would exceed the budget or fail; 0: freed now and at the end of

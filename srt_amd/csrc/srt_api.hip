@@ -286,6 +286,12 @@ int srt_set_option(srt_ctx* c, const char* key, int64_t value) {
         c->trace_packet = (int32_t)value;
         return SRT_OK;
     }
+    if (!strcmp(key, "whole_paths")) {
+        if (value < 0 || value > kMaxPathPool)
+            return set_err(c, SRT_E_INVALID, "whole_paths must be in [0, %lld]", (long long)kMaxPathPool);
+        c->whole_paths = value;
+        return SRT_OK;
+    }
     if (!strcmp(key, "keep_build_scratch")) {
         if (value != 0 && value != 1) return set_err(c, SRT_E_INVALID, "keep_build_scratch must be 0 or 1");
         c->keep_build_scratch = value == 1;

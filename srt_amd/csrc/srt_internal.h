@@ -65,6 +65,14 @@ struct TraceCfg {
                          // testing postponed leaves once this many lanes hold one
     int32_t deal;        // first bounce: the slots are dealt to the pieces (CamView)
 };
+// Live paths at which chunk_stages finishes a chunk's paths with k_paths (4-wide
+// trees; visit counts come from the queue stages).  Measured with the switch
+// at 0 / 2^20 / 2^21 / 2^22 live paths: 1M-triangle frame 1280x720x1 depth 16
+// 2.89 / 1.61 / 1.63 / 1.62 ms, instanced 1280x720x8 8.12 / 7.14 / 7.11 / 7.62,
+// tube 1280x720x16 4.01 / 3.32 / 3.21 / 3.28, Cornell 256x256x16 0.476 / 0.404 /
+// 0.403 / 0.407, 256x256x64 with the MLP 0.740 / 0.717 / 0.770 / 0.817,
+// 512x512x16 (4.2M paths, all of them at once) 0.87 against 1.04.
+constexpr int64_t kWholePaths = 1 << 20;
 
 // ---------------------------------------------------------------------------
 // device view of one resident scene
@@ -331,6 +339,7 @@ struct srt_ctx {
     uint32_t* live = nullptr;
     unsigned long long* host_totals = nullptr;
     std::map<std::pair<const void*, size_t>, int> occupancy;   // resident workgroups per CU by kernel and LDS bytes
+    int64_t whole_paths = srt::kWholePaths;   // live paths finished in one launch (0: never)
     int32_t trace_inner_exit = 18;        // stragglers resume after the leaf step
     int32_t trace_packet = 0;             // > 0: camera rays traversed as 64-ray packets (0: per ray)
     int64_t max_wide_nodes = srt::kMaxNodes4;   // 4-wide trees above this many nodes are traversed in binary form

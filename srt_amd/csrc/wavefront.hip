@@ -1505,7 +1505,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(DevScene S, ShadowQueue 
 // is done goes on with its own next ray, so a launch lasts as long as its
 // slowest path.  The price is registers (156 VGPRs, 3 waves per SIMD, against 6
 // of the traversal kernels), which loses once there are rays enough to fill the
-// queue stages: run_chunk switches to it at kWholePathMax live paths.
+// queue stages: chunk_stages switches to it at kWholePaths live paths.
 // A wave traces until `refill` of its lanes wait for shading or a new path (or
 // none is tracing), then shades those together; a lane starts its path's next
 // ray right after the shadow ray, without waiting for the others.  The shadow
@@ -2507,14 +2507,6 @@ static int ensure_mlp_bufs(srt_ctx* c, int64_t slots) {
     return SRT_OK;
 }
 
-// Live paths at which run_chunk finishes a chunk's paths with k_paths (4-wide
-// trees; visit counts come from the queue stages).  Measured with the switch
-// at 0 / 2^20 / 2^21 / 2^22 live paths: 1M-triangle frame 1280x720x1 depth 16
-// 2.89 / 1.61 / 1.63 / 1.62 ms, instanced 1280x720x8 8.12 / 7.14 / 7.11 / 7.62,
-// tube 1280x720x16 4.01 / 3.32 / 3.21 / 3.28, Cornell 256x256x16 0.476 / 0.404 /
-// 0.403 / 0.407, 256x256x64 with the MLP 0.740 / 0.717 / 0.770 / 0.817,
-// 512x512x16 (4.2M paths, all of them at once) 0.87 against 1.04.
-constexpr int64_t kWholePathMax = 1 << 20;
 constexpr int64_t kPathSpread = 32;      // workgroups per 128 paths that k_paths may use
 
 // Waits for the size of the next bounce's queue (report_live), which arrives
@@ -2569,7 +2561,7 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     if (int r = ensure_gstack(c, s, (int64_t)std::max(tgrid, wgrid) * kTraceBlock)) return r;
     TraceCfg tcfg = trace_cfg(c, s);
     for (int k = 0; k < nseg; k++) tcfg.deal |= n < (int64_t)kParts * segs_host[k].wh ? 1 : 0;
-    const int64_t whole = tcfg.wide && !c->count_visits ? kWholePathMax : 0;
+    const int64_t whole = tcfg.wide && !c->count_visits ? c->whole_paths : 0;
     int64_t npaths = n;                   // live paths of the bounce
     uint32_t* live = c->live;
     TraceCfg scfg = tcfg;

@@ -251,3 +251,57 @@ def test_smaller_calls_work_after_a_refused_allocation(refused):
         assert first[1] == again[1] > 0       # (the weights moved on between them)
     else:
         assert np.array_equal(first, again)
+
+
+@pytest.mark.parametrize("form", ["after 1", "after 2", "whole"])
+@pytest.mark.parametrize("name,W,H,spp", [("cornell", 77, 53, 4), ("spheres", 160, 90, 3)])
+def test_hooks_across_the_switch_to_whole_paths(ctx, name, W, H, spp, form):
+    """Training and query frames whose paths go over to the whole-path kernel
+    after the first bounce (records, snapshots and queries are made there), after
+    the second (they were made by the queue stages) or start in it: the bits of
+    the queue stages alone."""
+    from srt_amd import scenes
+    from test_gpu_render import _limits
+    s = getattr(scenes, name)()
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    out = []
+    try:
+        train, query = (_limits(ctx, h, s.camera, W, H, spp, 5, 1, seed) for seed in (9, 2))
+        for f in ("never", form):
+            ctx.mlp_create(seed=3, lr=1e-3)
+            ctx.set_option("whole_paths", train[f])
+            loss, n = ctx.mlp_train_frame(h, s.camera, W, H, spp, 5, 4, seed=9, max_samples=1 << 14, steps=3)
+            params = ctx.mlp_params()
+            ctx.set_option("whole_paths", query[f])
+            out.append((loss, n, params, ctx.render(h, s.camera, W, H, spp, 5, 4, 1, 1, 2, mlp_mode=1)))
+    finally:
+        ctx.set_option("whole_paths", 1 << 20)
+        ctx.release(h)
+    assert out[0][:2] == out[1][:2] and out[0][1] > 1000
+    assert np.array_equal(out[0][2], out[1][2])
+    assert np.array_equal(out[0][3], out[1][3])
+
+
+@pytest.mark.parametrize("whole", [0, 100, 1 << 20])
+def test_training_frame_without_a_hit(ctx, whole):
+    """No camera ray hits: no path lives after the first bounce, which ends the
+    queue stages, and no sample is recorded."""
+    from srt_amd import scenes
+    s = scenes.spheres()
+    away = dict(s.camera)
+    pos, target = np.asarray(away["position"], float), np.asarray(away["target"], float)
+    away["target"] = tuple(2 * pos - target)
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    try:
+        ctx.set_option("whole_paths", whole)
+        ctx.mlp_create(seed=3, lr=1e-3)
+        p = ctx.mlp_params()
+        loss, n = ctx.mlp_train_frame(h, away, 64, 36, 2, 5, 4, seed=9, max_samples=1 << 12, steps=2)
+        assert (loss, n) == (0.0, 0)
+        assert ctx.last_counts() == (64 * 36 * 2, 0)
+        assert np.array_equal(ctx.mlp_params(), p)
+    finally:
+        ctx.set_option("whole_paths", 1 << 20)
+        ctx.release(h)

@@ -283,3 +283,47 @@ def test_dealt_slots_cover_every_path(ctx, W, H, spp):
         osc = O.Scene(s)
         ref, _ = O.render(osc, s.camera, W, H, spp, 3, 4, 1, 1, 13, bvh=O.Bvh(osc))
         assert _rel(a[:, :3], ref[:, :3]).max() <= TOL
+
+
+def _limits(ctx, h, cam, W, H, spp, depth, nee, seed):
+    """Values of whole_paths: never, switch after the first bounce, switch after
+    the second, whole from the start (the paths live at a bounce are the
+    segments that one more bounce adds)."""
+    ctx.set_option("whole_paths", 0)
+    seg = []
+    for d in (1, 2, 3):
+        ctx.render(h, cam, W, H, spp, min(d, depth), 4, nee, nee, seed)
+        seg.append(ctx.last_counts()[0])
+    live1, live2 = seg[1] - seg[0], seg[2] - seg[1]
+    assert seg[0] == W * H * spp > live1 > live2 > 0
+    return {"never": 0, "after 1": live1, "after 2": live2, "whole": 1 << 20}
+
+
+@pytest.mark.parametrize("form", ["never", "after 1", "after 2", "whole"])
+@pytest.mark.parametrize("name,W,H,spp,depth,nee", [("cornell", 97, 61, 5, 8, 1), ("cornell", 64, 64, 8, 5, 0),
+                                                    ("spheres", 192, 108, 2, 8, 1), ("tube", 128, 72, 2, 6, 1),
+                                                    ("cornell_instanced", 67, 45, 4, 5, 1)])
+def test_every_path_form_matches_oracle(ctx, name, W, H, spp, depth, nee, form):
+    """The queue stages alone, each switch from them to the whole-path kernel
+    and that kernel alone (option whole_paths) give the oracle's image and ray
+    counts, with and without light sampling."""
+    s = getattr(scenes, name)()
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    try:
+        ctx.set_option("whole_paths", _limits(ctx, h, s.camera, W, H, spp, depth, nee, 6)[form])
+        img = ctx.render(h, s.camera, W, H, spp, depth, 4, nee, nee, 6)
+        counts = ctx.last_counts()
+    finally:
+        ctx.set_option("whole_paths", 1 << 20)
+        ctx.release(h)
+    osc = O.Scene(s)
+    ref, _ = O.render(osc, s.camera, W, H, spp, depth, 4, nee, nee, 6, bvh=O.Bvh(osc))
+    assert _rel(img[:, :3], ref[:, :3]).max() <= TOL
+    assert counts == tuple(O.last_counts())
+
+
+def test_whole_paths_range(ctx):
+    for v in (-1, 1 << 31):
+        with pytest.raises(Exception):
+            ctx.set_option("whole_paths", v)

@@ -209,3 +209,21 @@ def test_each_scene_queries_its_own_mlp(served):
         ctx.release(h2)
     assert ctx.lib.srt_hbm_used(ctx.h) < used          # the scene and its MLP are freed
     assert np.array_equal(ctx.render(hc, cb.camera, 32, 24, 4, 5, 4, 1, 1, 16, mlp_mode=1), shared)
+
+
+@pytest.mark.parametrize("whole", [0, 15000])
+def test_mix_equals_alone_in_queue_stages(served, whole):
+    """A chunk of several requests run bounce by bounce (whole_paths 0), or
+    until its first bounces have left 15000 of its 40000 paths, gives each
+    request's own image."""
+    ctx, reqs, alone = served
+    ctx.set_option("whole_paths", whole)
+    ctx.serve_start(0)
+    try:
+        for k, (t, img) in enumerate(_submit_all(ctx, reqs)):
+            assert ctx.wait(t)["status"] == 2
+            assert np.array_equal(img, alone[k]), (k, whole)
+    finally:
+        ctx.serve_stop()
+        ctx.forget_tickets()
+        ctx.set_option("whole_paths", 1 << 20)
