@@ -125,8 +125,10 @@ const char* srt_last_error(const srt_ctx* ctx);
  * results are identical; packets gain 1 % of the closest-hit time on a scene
  * that fills the frame with deep traversals and lose 10 % where camera rays
  * visit few nodes), "whole_paths" (a chunk's paths are finished in one launch
- * that holds each in registers once at most this many live, 0..2^31 - 1, default
- * 2^20; 0: bounce by bounce to the end; the results are identical),
+ * that holds each in registers once at most this many live (after the first
+ * bounce at most 2^17 (k + 2) with k bounces left, and 2^20),
+ * 0..2^31 - 1, default 2^20; 0: bounce by bounce to the end; the results are
+ * identical),
  * "keep_build_scratch" (1, the
  * default: the device scratch of a BVH build, and of a denoise pass up to 512 MiB,
  * stays allocated for the next one and counts in srt_hbm_used; it is freed when

@@ -65,14 +65,24 @@ struct TraceCfg {
                          // testing postponed leaves once this many lanes hold one
     int32_t deal;        // first bounce: the slots are dealt to the pieces (CamView)
 };
-// Live paths at which chunk_stages finishes a chunk's paths with k_paths (4-wide
-// trees; visit counts come from the queue stages).  Measured with the switch
-// at 0 / 2^20 / 2^21 / 2^22 live paths: 1M-triangle frame 1280x720x1 depth 16
-// 2.89 / 1.61 / 1.63 / 1.62 ms, instanced 1280x720x8 8.12 / 7.14 / 7.11 / 7.62,
-// tube 1280x720x16 4.01 / 3.32 / 3.21 / 3.28, Cornell 256x256x16 0.476 / 0.404 /
-// 0.403 / 0.407, 256x256x64 with the MLP 0.740 / 0.717 / 0.770 / 0.817,
-// 512x512x16 (4.2M paths, all of them at once) 0.87 against 1.04.
+// Live paths up to which chunk_stages finishes a chunk's paths with k_paths
+// (4-wide trees; visit counts come from the queue stages): kWholePaths (option
+// "whole_paths").  Times in ms at 0 (queue stages alone) / 2^18 / 2^19 / 2^20 /
+// 2^21 live paths: 1M triangles 1280x720x1 depth 16 2.84 / 1.88 / 1.68 / 1.53 /
+// 1.52, 1280x720x2 depth 8 3.07 / 2.26 / 2.26 / 2.08 / 2.18, instanced
+// 1280x720x8 8.01 / 7.28 / 7.03 / 7.04 / 7.03, tube 1280x720x16 3.66 / 3.25 /
+// 2.95 / 2.97 / 2.95, Cornell depth 5 256x256x16 0.440 / 0.398 / 0.404 / 0.397 /
+// 0.396, 256x256x64 with the MLP 0.692 / 0.691 / 0.690 / 0.689 / 0.757.
 constexpr int64_t kWholePaths = 1 << 20;
+// The same once bounces have run as stages and `left` remain.  What k_paths then
+// saves is the tail of each remaining launch (its slowest ray); what it costs,
+// at half the waves of the traversal kernels, grows with the live paths.  With
+// few bounces left the cost wins earlier.  Limits whatever the number left of 0 /
+// 2^18 / 2^19 / 3 x 2^18 / 2^20: Cornell depth 5 512x512x16 0.91 / 0.91 / 0.93 / 0.96 /
+// 0.97, 256x256x48 0.78 / 0.78 / 0.80 / 0.81 / 0.82; 1M triangles 1280x720x2 depth 3,
+// half a million paths with two bounces left, 1.71 as stages and 1.65 whole.
+// With the line below 0.90, 0.81 and 1.69, and the others above as at 2^20.
+inline int64_t whole_path_limit(int left) { return std::min(kWholePaths, (int64_t)(left + 2) << 17); }
 
 // ---------------------------------------------------------------------------
 // device view of one resident scene

@@ -1505,7 +1505,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(DevScene S, ShadowQueue 
 // is done goes on with its own next ray, so a launch lasts as long as its
 // slowest path.  The price is registers (156 VGPRs, 3 waves per SIMD, against 6
 // of the traversal kernels), which loses once there are rays enough to fill the
-// queue stages: chunk_stages switches to it at kWholePaths live paths.
+// queue stages: chunk_stages switches to it at kWholePaths live paths or fewer.
 // A wave traces until `refill` of its lanes wait for shading or a new path (or
 // none is tracing), then shades those together; a lane starts its path's next
 // ray right after the shadow ray, without waiting for the others.  The shadow
@@ -2561,7 +2561,10 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     if (int r = ensure_gstack(c, s, (int64_t)std::max(tgrid, wgrid) * kTraceBlock)) return r;
     TraceCfg tcfg = trace_cfg(c, s);
     for (int k = 0; k < nseg; k++) tcfg.deal |= n < (int64_t)kParts * segs_host[k].wh ? 1 : 0;
-    const int64_t whole = tcfg.wide && !c->count_visits ? c->whole_paths : 0;
+    const int64_t whole_max = tcfg.wide && !c->count_visits ? c->whole_paths : 0;
+    auto whole = [&](int depth) {
+        return depth == 0 ? whole_max : std::min(whole_max, whole_path_limit(max_depth - depth));
+    };
     int64_t npaths = n;                   // live paths of the bounce
     uint32_t* live = c->live;
     TraceCfg scfg = tcfg;
@@ -2617,14 +2620,14 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     if (max_depth == 0)                   // no shade stage sets the radiance
         for (float* L : {Lr, Lg, Lb}) k_zero<<<nblk, 256, 0, st>>>(L, (size_t)n);
     const int packet0 = c->count_visits ? 0 : trace_packet_ok(c, s, tcfg);     // camera rays as packets
-    if (mlp_mode == 2 && (n > whole || packet0))                               // (whole paths clear their own)
+    if (mlp_mode == 2 && (n > whole(0) || packet0))                               // (whole paths clear their own)
         k_zero<<<nblk, 256, 0, st>>>((float*)mio.rec_valid, (size_t)n);
     for (int depth = 0; depth < max_depth && npaths > 0; depth++) {
         int qi = depth & 1;
         const bool cam = depth == 0;
         const bool cnt = c->count_visits;
         const int packet = cam ? packet0 : 0;
-        if (npaths <= whole && !packet) {      // the rest of every path in one launch
+        if (npaths <= whole(depth) && !packet) {      // the rest of every path in one launch
             prof_begin(c, "paths", &ev);
             float* snap = mlp_mode == 2 && depth <= 1 ? (float*)c->mlpbuf[7].p : nullptr;
             if (inst) {
