@@ -122,16 +122,19 @@ SRT_D void clear_parts(uint32_t* first) {
 }
 // Partition of this workgroup in a partitioned queue, and its index among the
 // partition's workgroups (grid: a multiple of kParts).  Consecutive workgroups
-// run on the 8 XCDs in turn: where the grid allows, each partition gets
-// workgroups of every XCD (kXcds consecutive ones), so that a partition with more
-// work than the others is not left to one XCD.  With partition = workgroup
-// mod kParts, the lower half of an image whose upper half is sky (alternate
-// pieces at 16 samples) kept four XCDs busy and four idle.
+// run on the 8 XCDs in turn, so a partition's appends come from one XCD and meet
+// in its L2.
+SRT_D uint32_t my_part() { return blockIdx.x % (uint32_t)kParts; }
+SRT_D uint32_t my_index() { return blockIdx.x / (uint32_t)kParts; }
+// The piece of a k_paths workgroup: where the grid allows, each piece gets
+// workgroups of every XCD (kXcds consecutive ones), since its few long paths
+// should not share a chiplet.  Cornell 64x64x4 takes 175 us, 178 with my_part; the
+// queue stages lose by it, their partitions being written from every XCD:
+// Cornell 512x512x30 depth 3 1.15 ms, 1.12 with my_part, 256x256x64 with the MLP
+// 0.693 and 0.675, tube 1280x720x16 2.88 and 2.85.
 constexpr uint32_t kXcds = 8;
-SRT_D bool xcd_spread() { return gridDim.x % (kXcds * (unsigned)kParts) == 0u; }
-SRT_D uint32_t my_part() { return (xcd_spread() ? blockIdx.x / kXcds : blockIdx.x) % (uint32_t)kParts; }
-SRT_D uint32_t my_index() {
-    return xcd_spread() ? blockIdx.x / (kXcds * (unsigned)kParts) * kXcds + blockIdx.x % kXcds : blockIdx.x / (unsigned)kParts;
+SRT_D uint32_t spread_part() {
+    return (gridDim.x % (kXcds * (unsigned)kParts) == 0u ? blockIdx.x / kXcds : blockIdx.x) % (uint32_t)kParts;
 }
 
 // One ray's traversal state, kept in registers while its lane walks the BVH.
@@ -542,8 +545,9 @@ struct QueueView {
 };
 // Workgroup prologue, run by all its threads: the prefix sums of the kParts
 // size counters at counts[cnt] into lds[0..kParts], and this workgroup's piece
-// [lo, hi) of the concatenation (piece blockIdx mod kParts of kParts equal ones).
-SRT_D QueueView queue_piece(const uint32_t* counts, int cnt, uint32_t cap, uint32_t* lds, uint32_t& lo, uint32_t& hi) {
+// [lo, hi) of the concatenation (piece `piece` of kParts equal ones).
+SRT_D QueueView queue_piece(const uint32_t* counts, int cnt, uint32_t cap, uint32_t* lds, uint32_t& lo, uint32_t& hi,
+                            uint32_t piece = my_part()) {
     if (threadIdx.x < 64u) {
         uint32_t v = threadIdx.x < (unsigned)kParts ? counts[cnt + threadIdx.x * kCntLine] : 0u;
         for (int d = 1; d < 64; d <<= 1) {
@@ -555,7 +559,6 @@ SRT_D QueueView queue_piece(const uint32_t* counts, int cnt, uint32_t cap, uint3
     }
     __syncthreads();
     const uint32_t total = lds[kParts];
-    const uint32_t piece = my_part();
     lo = (uint32_t)((uint64_t)total * piece / kParts);
     hi = (uint32_t)((uint64_t)total * (piece + 1u) / kParts);
     QueueView v{lds, cap, 0u};
@@ -632,8 +635,9 @@ struct Feeder {
 // over a partitioned queue's concatenation (or the first bounce's slots), the
 // counters at counts[cnt]
 template <class View>
-SRT_D Feeder<View> queue_feeder(const View& view, const uint32_t* prefix, uint32_t* counts, int cnt) {
-    return Feeder<View>(view, counts + cnt, prefix[kParts], (uint32_t)kParts, my_part());
+SRT_D Feeder<View> queue_feeder(const View& view, const uint32_t* prefix, uint32_t* counts, int cnt,
+                                uint32_t piece = my_part()) {
+    return Feeder<View>(view, counts + cnt, prefix[kParts], (uint32_t)kParts, piece);
 }
 // over a dense array [0, n): min(kParts, grid size) pieces
 SRT_D Feeder<IdentityEntry> dense_feeder(uint32_t n, uint32_t* fetch) {
@@ -1547,12 +1551,12 @@ __global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segm
                                                       float* Lb, int32_t* gstack, MlpIO mio, float* snap, TraceCfg cfg) {
     __shared__ uint32_t prefix[kParts + 1];
     uint32_t lo, hi;
-    const QueueView view = queue_piece(counts, cnt_q(qi), cap, prefix, lo, hi);
-    const uint32_t part = my_part();
+    const uint32_t part = spread_part();
+    const QueueView view = queue_piece(counts, cnt_q(qi), cap, prefix, lo, hi, part);
     std::conditional_t<CAM, CamView, QueueView> pview;
     if constexpr (CAM) pview = cam_view(prefix[kParts], cfg.deal);
     else pview = view;
-    auto feed = queue_feeder(pview, prefix, counts, CNT_FETCH_T);
+    auto feed = queue_feeder(pview, prefix, counts, CNT_FETCH_T, part);
     const TravStack k = make_stack<INST>(gstack, cfg);
     const f3 env = mk(S.env[0], S.env[1], S.env[2]);
     const int lane = __lane_id();
