@@ -261,10 +261,11 @@ def test_whole_path_kernel_equals_queue_stages(ctx, name, W, H, spp, depth):
     assert out[0][1] == out[1][1]
 
 
-@pytest.mark.parametrize("W,H,spp", [(8, 8, 1), (61, 37, 1), (160, 57, 1), (311, 170, 5), (640, 411, 2), (97, 61, 40)])
+@pytest.mark.parametrize("W,H,spp", [(8, 8, 1), (61, 37, 1), (160, 57, 1), (203, 101, 2), (301, 109, 4), (311, 170, 5),
+                                      (640, 411, 2), (97, 61, 40)])
 def test_dealt_slots_cover_every_path(ctx, W, H, spp):
     """Chunks of fewer than 32 sample planes deal their slots to the queue's
-    pieces in runs of 1, 64 or 512: every path is traced once whatever the
+    pieces in runs of 1, 64 (from 2^15 paths) or 256 (from 2^17): every path is traced once whatever the
     remainder (queue stages by visit counting), and the image is the whole-path
     kernel's and, for small frames, the oracle's."""
     s = scenes.cornell()
