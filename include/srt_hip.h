@@ -104,37 +104,30 @@ typedef struct srt_bvh_opts {
 int srt_create(int device, size_t hbm_budget_bytes, srt_ctx** out);
 void srt_destroy(srt_ctx* ctx);
 const char* srt_last_error(const srt_ctx* ctx);
-/* tunables: "path_pool" (path slots per chunk, default 2^27), "profile" (0/1 per-kernel HIP events),
- * "count_visits" (0/1 count BVH node visits and triangle tests), "hbm_budget"
- * (bytes; at least srt_hbm_used), "trace_stack_lds" (traversal stack entries per
- * lane in LDS, 4..64, default 16), "trace_refill" / "shadow_refill" (finished
- * lanes that make a traversal wave fetch new rays, 1..64, defaults 40 / 32),
- * "trace_blocks_per_cu"
- * (0: as many as fit), "trace_bvh_width" (4: traverse the 4-wide tree collapsed
- * from the binary one, default; 2: the binary tree; results are identical),
- * "trace_inner_exit" (a traversal wave leaves its inner-node loop once at most
- * this many lanes still search for a leaf, 0..63, default 18), "max_wide_nodes"
- * (a BVH built while this is set keeps its 4-wide form only up to this many
- * 4-wide nodes, else it is traversed in binary form with the same results;
- * 0..16777215, the default: 4-wide nodes are addressed with 32-bit byte
- * offsets), "serve_age" (serving order, below: the weight of the time a request
- * has waited, per mille, 0..1000, default 250), "trace_packet" (camera rays of a
- * flat scene with a 4-wide tree are traversed as 64-ray packets, one node
- * sequence per wave; the value is the number of lanes holding postponed leaves
- * that makes the wave test them, 1..64; 0, the default: per-ray traversal; the
- * results are identical; packets gain 1 % of the closest-hit time on a scene
- * that fills the frame with deep traversals and lose 10 % where camera rays
- * visit few nodes), "whole_paths" (a chunk's paths are finished in one launch
- * that holds each in registers once at most this many live (after the first
- * bounce at most 2^17 (k + 2) with k bounces left, and 2^20),
- * 0..2^31 - 1, default 2^20; 0: bounce by bounce to the end; the results are
- * identical),
- * "keep_build_scratch" (1, the
- * default: the device scratch of a BVH build, and of a denoise pass up to 512 MiB,
- * stays allocated for the next one and counts in srt_hbm_used; it is freed when
- * an allocation would exceed the budget or fail; 0: freed now and at the end of
- * every build and pass).  Limits: 2^28 - 1 triangles per scene; "path_pool" and the pool
- * of srt_serve_start in [64, 2^31 - 1]. */
+/* tunables: "path_pool" (path slots per chunk, default 2^27), "profile" (0/1 per-kernel HIP
+ * events), "count_visits" (0/1 count BVH node visits and triangle tests), "hbm_budget" (bytes; at
+ * least srt_hbm_used), "trace_stack_lds" (traversal stack entries per lane in LDS, 4..64, default
+ * 16), "trace_refill" / "shadow_refill" (finished lanes that make a traversal wave fetch new rays,
+ * 1..64, defaults 40 / 32), "trace_blocks_per_cu" (0, the default: as many as fit, at most 12
+ * outside packet traversal), "trace_bvh_width" (4: traverse the 4-wide tree collapsed from the
+ * binary one, default; 2: the binary tree; results are identical), "trace_inner_exit" (a traversal
+ * wave leaves its inner-node loop once at most this many lanes still search for a leaf, 0..63,
+ * default 18), "max_wide_nodes" (a BVH built while this is set keeps its 4-wide form only up to
+ * this many 4-wide nodes, else it is traversed in binary form with the same results; 0..16777215,
+ * the default: 4-wide nodes are addressed with 32-bit byte offsets), "serve_age" (serving order,
+ * below: the weight of the time a request has waited, per mille, 0..1000, default 250),
+ * "trace_packet" (camera rays of a flat scene with a 4-wide tree are traversed as 64-ray packets,
+ * one node sequence per wave; the value is the number of lanes holding postponed leaves that makes
+ * the wave test them, 1..64; 0, the default: per-ray traversal; the results are identical; a frame
+ * that deep traversals fill takes the same time, one whose camera rays visit few nodes 4 to 7 %
+ * more), "whole_paths" (a chunk's paths are finished in one launch that holds each in registers
+ * once at most this many live (after the first bounce at most 2^17 (k + 2) with k bounces left,
+ * and 2^20), 0..2^31 - 1, default 2^20; 0: bounce by bounce to the end; the results are
+ * identical), "keep_build_scratch" (1, the default: the device scratch of a BVH build, and of a
+ * denoise pass up to 512 MiB, stays allocated for the next one and counts in srt_hbm_used; it is
+ * freed when an allocation would exceed the budget or fail; 0: freed now and at the end of every
+ * build and pass).  Limits: 2^28 - 1 triangles per scene; "path_pool" and the pool of
+ * srt_serve_start in [64, 2^31 - 1]. */
 int srt_set_option(srt_ctx* ctx, const char* key, int64_t value);
 size_t srt_hbm_used(const srt_ctx* ctx);
 

@@ -2382,11 +2382,11 @@ static size_t trace_lds_bytes(const TraceCfg& cfg, bool inst = false) {
 
 // Persistent traversal grid: as many workgroups as are resident at once
 // (occupancy of the traversal kernel with its LDS stack), at most 6 waves per
-// SIMD, capped by the work.  A seventh wave (a kernel of 72 VGPRs or fewer)
-// costs more in the caches than it hides: 37.6 against 35.9 ms of closest
-// hits on the 1M-triangle frame.
-constexpr int kTraceBlocksPerCu = 6 * 4 * 64 / kTraceBlock;
-static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr) {
+// SIMD for per-ray traversal, capped by the work.  A seventh wave (a kernel of
+// 72 VGPRs or fewer) costs more in the caches than it hides: 37.6 against 35.9 ms
+// of closest hits on the 1M-triangle frame.
+constexpr int kTraceBlocksPerCu = 6 * 4 * 64 / kTraceBlock, kAnyBlocksPerCu = 64;
+static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr, int most = kTraceBlocksPerCu) {
     const TraceCfg cfg = trace_cfg(c, nullptr);
     int per_cu = c->trace_blocks_per_cu;
     if (per_cu <= 0) {
@@ -2396,7 +2396,7 @@ static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr) {
             (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kTraceBlock, trace_lds_bytes(cfg)) != hipSuccess ||
              nb <= 0))
             nb = 8;
-        per_cu = std::min(nb, kTraceBlocksPerCu);
+        per_cu = std::min(nb, most);
     }
     int64_t want = (n + kTraceBlock - 1) / kTraceBlock;
     int64_t cap = (int64_t)num_cus(c) * per_cu;
@@ -2557,7 +2557,7 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     const MlpBind bind(c, s->handle);       // mode 1 queries the scene's MLP (else the context's own)
     if (int r = ensure_pool(c, n)) return r;
     const int tgrid = part_grid(trace_grid(c, n));
-    const int pgrid = part_grid(trace_grid(c, n, reinterpret_cast<const void*>(k_trace_packet)));
+    const int pgrid = part_grid(trace_grid(c, n, reinterpret_cast<const void*>(k_trace_packet), kAnyBlocksPerCu));
     const uint32_t cap = part_cap((uint32_t)n);
     const bool inst = s->ninst > 0;
     // few paths are spread over more waves (k_paths' quota): the lanes of a wave
