@@ -133,8 +133,10 @@ SRT_D uint32_t my_index() { return blockIdx.x / (uint32_t)kParts; }
 // Cornell 512x512x30 depth 3 1.15 ms, 1.12 with my_part, 256x256x64 with the MLP
 // 0.693 and 0.675, tube 1280x720x16 2.88 and 2.85.
 constexpr uint32_t kXcds = 8;
-SRT_D uint32_t spread_part() {
-    return (gridDim.x % (kXcds * (unsigned)kParts) == 0u ? blockIdx.x / kXcds : blockIdx.x) % (uint32_t)kParts;
+SRT_D bool spread_xcds() { return gridDim.x % (kXcds * (unsigned)kParts) == 0u; }
+SRT_D uint32_t spread_part() { return (spread_xcds() ? blockIdx.x / kXcds : blockIdx.x) % (uint32_t)kParts; }
+SRT_D uint32_t spread_index() {
+    return spread_xcds() ? blockIdx.x / (kXcds * (unsigned)kParts) * kXcds + blockIdx.x % kXcds : my_index();
 }
 
 // One ray's traversal state, kept in registers while its lane walks the BVH.
@@ -1552,7 +1554,8 @@ struct PathSink {      // shade_path's results for a path held in registers
 template <bool CAM, bool INST>
 __global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segment* segs, int nseg, PathQueue q, int depth0,
                                                       int qi, uint32_t cap, uint32_t* counts, float* Lr, float* Lg,
-                                                      float* Lb, int32_t* gstack, MlpIO mio, float* snap, TraceCfg cfg) {
+                                                      float* Lb, int32_t* gstack, uint32_t gstack_lanes, MlpIO mio,
+                                                      float* snap, TraceCfg cfg) {
     __shared__ uint32_t prefix[kParts + 1];
     uint32_t lo, hi;
     const uint32_t part = spread_part();
@@ -1561,14 +1564,21 @@ __global__ void __launch_bounds__(kTraceBlock, 3) k_paths(DevScene S, const Segm
     if constexpr (CAM) pview = cam_view(prefix[kParts], cfg.deal);
     else pview = view;
     auto feed = queue_feeder(pview, prefix, counts, CNT_FETCH_T, part);
-    const TravStack k = make_stack<INST>(gstack, cfg);
+    TravStack k = make_stack<INST>(gstack, cfg);
     const f3 env = mk(S.env[0], S.env[1], S.env[2]);
     const int lane = __lane_id();
-    // a launch with fewer paths than resident lanes spreads them over its waves
-    const uint32_t waves = gridDim.x / (unsigned)kParts * (kTraceBlock / 64);
-    const uint32_t quota = min(64u, max(1u, (hi - lo + waves - 1u) / waves));
+    // A launch with fewer paths than resident lanes spreads them over its waves.
+    // Its lanes in use then share the stack memory of gstack_lanes lanes (at least
+    // 64 per piece), with fewer waves where it is short of that.
+    const uint32_t piece_max = max(1u, (prefix[kParts] + (uint32_t)kParts - 1u) / (uint32_t)kParts);
+    const uint32_t all_waves = gridDim.x / (unsigned)kParts * (kTraceBlock / 64);
+    const uint32_t quota = __builtin_amdgcn_readfirstlane(min(64u, (piece_max + all_waves - 1u) / all_waves));
+    const uint32_t waves = min(all_waves, gstack_lanes / ((uint32_t)kParts * quota));
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(spread_index() * (kTraceBlock / 64) + (threadIdx.x >> 6));
+    k.gst = gstack + (size_t)(part * waves + wave) * quota + lane;
+    k.gstride = (size_t)kParts * waves * quota;
     const int refill = max(1, (int)(cfg.refill * quota / 64u)), inner_exit = (int)(k.inner_exit * quota / 64u);
-    bool exhausted = (uint32_t)lane >= quota;
+    bool exhausted = (uint32_t)lane >= quota || wave >= waves;
     uint32_t nseg_traced = 0, nshadow = 0, nv = 0;
     // the path
     uint32_t slot = 0, flags = 0;
@@ -2566,7 +2576,8 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     // less; Cornell 64x64x4 0.196 -> 0.171
     const int wgrid = part_grid(trace_grid(c, n * kPathSpread, inst ? reinterpret_cast<const void*>(k_paths<true, true>)
                                                                     : reinterpret_cast<const void*>(k_paths<true, false>)));
-    if (int r = ensure_gstack(c, s, (int64_t)std::max(tgrid, wgrid) * kTraceBlock)) return r;
+    const uint32_t glanes = (uint32_t)tgrid * kTraceBlock;
+    if (int r = ensure_gstack(c, s, glanes)) return r;
     TraceCfg tcfg = trace_cfg(c, s);
     for (int k = 0; k < nseg; k++) tcfg.deal |= n < (int64_t)kParts * segs_host[k].wh ? 1 : 0;
     const int64_t whole_max = tcfg.wide && !c->count_visits ? c->whole_paths : 0;
@@ -2639,11 +2650,11 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
             prof_begin(c, "paths", &ev);
             float* snap = mlp_mode == 2 && depth <= 1 ? (float*)c->mlpbuf[7].p : nullptr;
             if (inst) {
-                if (cam) k_paths<true, true><<<wgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
-                else k_paths<false, true><<<wgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
+                if (cam) k_paths<true, true><<<wgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, glanes, mio, snap, tcfg);
+                else k_paths<false, true><<<wgrid, kTraceBlock, ilds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, glanes, mio, snap, tcfg);
             } else {
-                if (cam) k_paths<true, false><<<wgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
-                else k_paths<false, false><<<wgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, mio, snap, tcfg);
+                if (cam) k_paths<true, false><<<wgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, glanes, mio, snap, tcfg);
+                else k_paths<false, false><<<wgrid, kTraceBlock, tlds, st>>>(S, segs, nseg, Q[qi], depth, qi, cap, counts, Lr, Lg, Lb, gst, glanes, mio, snap, tcfg);
             }
             prof_end(c, "paths", ev, 0);
             if (depth <= 1 && mlp_mode == 1) {

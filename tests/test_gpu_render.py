@@ -328,3 +328,28 @@ def test_whole_paths_range(ctx):
     for v in (-1, 1 << 31):
         with pytest.raises(Exception):
             ctx.set_option("whole_paths", v)
+
+
+@pytest.mark.parametrize("W,H,spp", [(1, 1, 1), (5, 3, 1), (64, 36, 1), (64, 64, 1), (97, 61, 2), (160, 90, 9)])
+def test_whole_paths_in_the_stacks_of_the_queue_stages(W, H, spp):
+    """The whole-path kernel spreads a small frame's paths over many waves, whose
+    lanes share the traversal stacks that the queue stages need for the frame:
+    the same image in no more memory (4 stack entries in LDS, the rest there)."""
+    from srt_amd import abi
+    s = scenes.spheres()
+
+    def frame(whole):
+        c = abi.Context(0)
+        c.set_option("trace_stack_lds", 4)
+        c.set_option("whole_paths", whole)
+        h = c.upload(s)
+        c.build_bvh(h)
+        img = c.render(h, s.camera, W, H, spp, 6, 4, 1, 1, 3)
+        used = c.hbm_used()
+        c.close()
+        return img, used
+
+    ref, stages = frame(0)
+    img, used = frame(1 << 20)
+    assert np.array_equal(img, ref)
+    assert used == stages
