@@ -896,18 +896,23 @@ int srt_denoise(srt_ctx* c, float* rgba, int32_t W, int32_t H, int32_t on_device
     if (n > (1ll << 28)) return set_err(c, SRT_E_LIMIT, "resolution too large");
     DevBuf tmp, tp;
     int r = on_device ? SRT_OK : post_buffer(c, rgba, n, tp);
-    // three images of scratch where they fit, else the two that are needed; the
-    // scratch of the last call serves when it is large enough
+    // three images of scratch where the budget has room for the third as it is
+    // (it is not worth the kept memory of other calls), else the two that are
+    // needed; the scratch of the last call serves when it is large enough
     {
         std::lock_guard<std::mutex> g(c->scratch_mu);
         std::swap(tmp, c->post_scratch);
     }
-    int images = 3;
-    if (tmp.bytes < (size_t)n * 48) dev_free(c, tmp);
-    if (!r && !tmp.p && dev_alloc(c, tmp, (size_t)n * 48)) {
-        (void)hipGetLastError();
-        images = 2;
-        r = dev_alloc(c, tmp, (size_t)n * 32);
+    const size_t two = (size_t)n * 32, three = (size_t)n * 48;
+    int images = tmp.bytes >= three || c->used - tmp.bytes + three <= c->budget ? 3 : 2;
+    if (tmp.bytes < (images == 3 ? three : two)) dev_free(c, tmp);
+    if (!r && !tmp.p) {
+        r = dev_alloc(c, tmp, images == 3 ? three : two);
+        if (r && images == 3) {                     // the device has less than the budget
+            (void)hipGetLastError();
+            images = 2;
+            r = dev_alloc(c, tmp, two);
+        }
     }
     if (!r) r = denoise_dev(c, on_device ? rgba : (float*)tp.p, (float*)tmp.p, images, W, H);
     if (!r && !on_device) r = hip_check(c, hipMemcpy(rgba, tp.p, (size_t)n * 16, hipMemcpyDeviceToHost), "download");

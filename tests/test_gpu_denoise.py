@@ -94,3 +94,29 @@ def test_row_groups_and_scratch_sizes(ctx, W, H, short):
             ctx.set_option("keep_build_scratch", 1)
     assert np.array_equal(np.isnan(out), np.isnan(ref))
     assert np.array_equal(np.nan_to_num(out), np.nan_to_num(ref))
+
+
+def test_optional_image_does_not_evict_kept_scratch():
+    """The third scratch image only saves time: where the budget has no room for
+    it beside a build's kept scratch, the pass takes two images and the scratch
+    stays; where it has, or where even two need the scratch's room, as before."""
+    from srt_amd import abi
+    W, H = 512, 300
+    rng = np.random.default_rng(5)
+    a = rng.uniform(0.0, 2.0, size=(W * H, 4)).astype(np.float32)
+    ref = O.denoise(a, W, H)
+    s = scenes.cornell()
+    for images, held in ((2.5, 2), (3, 3), (1, 2)):
+        c = abi.Context(0)
+        c.build_bvh(c.upload(s))                    # leaves its scratch, two chunks of 16 MiB
+        ptr = c.device_alloc(a.nbytes)
+        c.upload_bytes(ptr, a)
+        used = c.hbm_used()
+        c.set_option("hbm_budget", used + int(images * a.nbytes))
+        c.denoise_device(ptr, W, H)
+        out = np.zeros_like(a)
+        c.download_bytes(out, ptr)
+        kept = 32 << 20 if images == 1 else 0       # released for the two images
+        assert c.hbm_used() == used - kept + held * a.nbytes, images
+        c.close()
+        assert np.array_equal(out, ref)
