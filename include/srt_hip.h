@@ -106,7 +106,7 @@ void srt_destroy(srt_ctx* ctx);
 const char* srt_last_error(const srt_ctx* ctx);
 /* tunables: "path_pool" (path slots per chunk, default 2^27), "profile" (0/1 per-kernel HIP
  * events), "count_visits" (0/1 count BVH node visits and triangle tests), "hbm_budget" (bytes; at
- * least srt_hbm_used), "trace_stack_lds" (traversal stack entries per lane in LDS, 4..64, default
+ * least srt_hbm_used without kept scratch, which is freed for it), "trace_stack_lds" (traversal stack entries per lane in LDS, 4..64, default
  * 16), "trace_refill" / "shadow_refill" (finished lanes that make a traversal wave fetch new rays,
  * 1..64, defaults 40 / 32), "trace_blocks_per_cu" (0, the default: as many as fit, at most 12
  * outside packet traversal), "trace_bvh_width" (4: traverse the 4-wide tree collapsed from the

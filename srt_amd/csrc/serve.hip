@@ -92,7 +92,8 @@ static void dispatcher(srt_ctx* c) {
                 Request* q = S->pending.front();
                 size_t need = request_bytes(q->req);
                 if (c->used.load() + need > c->budget) {
-                    if (S->active.empty() && release_build_scratch(c)) continue;   // kept BVH-build chunks first
+                    // the kept scratch of builds and denoise passes first (neither runs while serving)
+                    if (release_build_scratch(c)) continue;
                     if (S->active.empty()) {          // nothing will ever free memory for it
                         S->pending.pop_front();
                         set_err(c, SRT_E_OOM, "request %llu needs %zu bytes beyond the HBM budget",

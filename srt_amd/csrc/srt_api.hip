@@ -299,6 +299,7 @@ int srt_set_option(srt_ctx* c, const char* key, int64_t value) {
         return SRT_OK;
     }
     if (!strcmp(key, "hbm_budget")) {
+        if (value > 0 && (size_t)value < c->used.load()) release_build_scratch(c);
         if (value <= 0 || (size_t)value < c->used.load())
             return set_err(c, SRT_E_INVALID, "hbm_budget must be positive and cover the %zu bytes in use", c->used.load());
         c->budget = (size_t)value;

@@ -227,3 +227,37 @@ def test_mix_equals_alone_in_queue_stages(served, whole):
         ctx.serve_stop()
         ctx.forget_tickets()
         ctx.set_option("whole_paths", 1 << 20)
+
+
+def test_kept_scratch_gives_way_to_admission():
+    """The kept scratch of a build (32 MiB) and of a denoise pass is released for
+    a request that does not fit beside it while another one runs, and for a
+    budget below what is held with it."""
+    ctx = abi.Context(0)
+    s = scenes.cornell()
+    h = ctx.upload(s)
+    ctx.build_bvh(h)
+    ctx.set_option("path_pool", 1 << 20)
+    ctx.render(h, s.camera, 1280, 720, 2, 5, 4, 1, 1, 1)          # the path pool of a serving chunk
+    ctx.denoise(np.ones((1280 * 720, 4), np.float32), 1280, 720)
+    need, used = 28 * 1280 * 720, ctx.hbm_used()
+    ctx.set_option("hbm_budget", used + need + (1 << 20))
+    ctx.serve_start(1 << 20)
+    try:
+        large, _ = ctx.submit(h, s.camera, 1280, 720, 256, 5, 4, 1, 1, 1)
+        small, _ = ctx.submit(h, s.camera, 400, 300, 1, 5, 4, 1, 1, 2)      # 3.4 MB
+        a, b = ctx.wait(large), ctx.wait(small)
+    finally:
+        ctx.serve_stop()
+        ctx.forget_tickets()
+    assert a["status"] == b["status"] == 2
+    assert a["chunks"] > 100 and b["admit_ms"] < a["done_ms"]
+    ctx.set_option("hbm_budget", 64 << 30)
+    bare = ctx.hbm_used()
+    ctx.build_bvh(h)
+    assert ctx.hbm_used() == bare + (32 << 20)
+    ctx.set_option("hbm_budget", bare)
+    assert ctx.hbm_used() == bare
+    with pytest.raises(abi.SrtError):
+        ctx.set_option("hbm_budget", bare - 1)
+    ctx.close()
