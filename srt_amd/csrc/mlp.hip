@@ -689,7 +689,7 @@ static int ensure_in(srt_ctx* c, MlpState* m, int64_t n) {
 static int infer_grid(srt_ctx* c, int64_t n) {
     int64_t tiles = (n + T_TILE - 1) / T_TILE;
     int64_t blocks = (tiles + MLP_BLOCK / 64 - 1) / (MLP_BLOCK / 64);
-    int64_t cap = (int64_t)num_cus(c) * 2;
+    int64_t cap = (int64_t)c->cus * 2;
     return (int)std::max<int64_t>(1, std::min(blocks, cap));
 }
 

@@ -177,6 +177,8 @@ int srt_create(int device, size_t hbm_budget_bytes, srt_ctx** out) {
     if (hipSetDevice(device) != hipSuccess) return SRT_E_HIP;
     srt_ctx* c = new srt_ctx();
     c->device = device;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) c->cus = cus;
     size_t free_b = 0, total_b = 0;
     (void)hipMemGetInfo(&free_b, &total_b);
     c->budget = hbm_budget_bytes ? hbm_budget_bytes : (size_t)(free_b * 0.9);

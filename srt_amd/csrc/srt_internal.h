@@ -320,7 +320,7 @@ struct KernelStat {
 }  // namespace srt
 
 struct srt_ctx {
-    int device = 0;
+    int device = 0, cus = 256;            // the device and its CUs
     size_t budget = 0;
     std::atomic<size_t> used{0};          // the serving thread allocates films too
     hipStream_t stream = nullptr;
@@ -385,7 +385,6 @@ struct srt_ctx {
     } while (0)
 
 namespace srt {
-int num_cus(srt_ctx* c);
 // allocation helpers (budget-checked)
 int dev_alloc(srt_ctx* c, DevBuf& b, size_t bytes);
 void dev_free(srt_ctx* c, DevBuf& b);

@@ -2349,16 +2349,6 @@ __global__ void __launch_bounds__(256) k_atrous(const float4* in, const float4* 
 // ---------------------------------------------------------------------------
 // host drivers
 // ---------------------------------------------------------------------------
-int num_cus(srt_ctx* c) {
-    static int cached = -1;
-    if (cached < 0) {
-        hipDeviceProp_t prop;
-        if (hipGetDeviceProperties(&prop, c->device) != hipSuccess) return 256;
-        cached = prop.multiProcessorCount;
-    }
-    return cached;
-}
-
 // The 4-wide tree is traversed when the context asks for it and the scene
 // has one (a tree beyond 32-bit node offsets keeps only its binary form).
 static bool use_wide(const srt_ctx* c, const SceneRec* s) {
@@ -2409,7 +2399,7 @@ static int trace_grid(srt_ctx* c, int64_t n, const void* kernel = nullptr, int m
         per_cu = std::min(nb, most);
     }
     int64_t want = (n + kTraceBlock - 1) / kTraceBlock;
-    int64_t cap = (int64_t)num_cus(c) * per_cu;
+    int64_t cap = (int64_t)c->cus * per_cu;
     if (want > cap) want = cap;
     if (want < 1) want = 1;
     return (int)want;
@@ -2629,7 +2619,7 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     }
     float* Lr = (float*)c->Lbuf[0].p; float* Lg = (float*)c->Lbuf[1].p; float* Lb = (float*)c->Lbuf[2].p;
     int32_t* gst = (int32_t*)c->gstack.p;
-    const int shade_grid = part_grid(std::min<int64_t>((n + 255) / 256, (int64_t)num_cus(c) * 8));
+    const int shade_grid = part_grid(std::min<int64_t>((n + 255) / 256, (int64_t)c->cus * 8));
     const int nblk = (int)((n + 255) / 256);
     hipEvent_t ev;
     // the first bounce's queue is the slots (its trace and shade stages compute
@@ -2896,7 +2886,7 @@ int render_light(srt_ctx* c, SceneRec* s, const DevCamera& cam, int spp, int max
     for (int64_t p0 = 0; p0 < total; p0 += pool) {
         const int n = (int)std::min<int64_t>(pool, total - p0);
         P.path_begin = p0;
-        const int shade_grid = part_grid(std::min<int64_t>((n + 255) / 256, (int64_t)num_cus(c) * 8));
+        const int shade_grid = part_grid(std::min<int64_t>((n + 255) / 256, (int64_t)c->cus * 8));
         const uint32_t cap = part_cap((uint32_t)n);
         k_lt_raygen<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(S, P, Q[0], n, cap, counts);
         for (int depth = 0; depth < max_depth; depth++) {
