@@ -65,11 +65,6 @@ static double now_ms(ServeState* S) {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - S->t0).count();
 }
 
-__global__ void k_zero_f(float* p, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
-}
-
 static size_t request_bytes(const srt_request& r) { return (size_t)r.width * r.height * (12 + 16); }
 
 static void finish(ServeState* S, Request* q, int32_t status) {
@@ -114,8 +109,6 @@ static void dispatcher(srt_ctx* c) {
                     S->done_cv.notify_all();
                     continue;
                 }
-                size_t n3 = (size_t)q->req.width * q->req.height * 3;
-                k_zero_f<<<(unsigned)((n3 + 255) / 256), 256, 0, c->stream>>>((float*)q->acc.p, n3);
                 q->status = 1;
                 q->t_admit = now_ms(S);
                 S->active.push_back(q);

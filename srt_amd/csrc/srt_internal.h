@@ -164,7 +164,7 @@ struct Segment {
     int32_t max_depth, rr_depth, use_nee, use_mis, mlp_mode;
     int32_t last;            // the request's final paths: write film_out
     DevCamera cam;
-    float* film_acc;         // 3 floats per pixel, zeroed before the first chunk
+    float* film_acc;         // 3 floats per pixel: the sums of the request's earlier chunks
     float4* film_out;
 };
 constexpr int kMaxSegments = 255;

@@ -486,11 +486,6 @@ SRT_D bool trav_leaf(const DevScene& S, TravState& st, uint32_t& nt) {
     return false;
 }
 
-// As trav_pend with the kind of ray known per lane (any: the first hit ends
-// the traversal, as trav_leaf<true>).
-template <bool INST>
-SRT_D bool trav_pend_any(const DevScene& S, TravState& st, const TravStack& k, bool any);
-
 // The postponed item of a lane: a triangle leaf (trav_leaf), or, in an
 // instanced scene, an instance to enter: the lane's current world-space
 // entry (if any) and kInstReturn are pushed, and the ray continues at the
@@ -515,6 +510,8 @@ SRT_D bool trav_pend(const DevScene& S, TravState& st, const TravStack& k, uint3
     return trav_leaf<ANY, COUNT, INST>(S, st, nt);
 }
 
+// As trav_pend with the kind of ray known per lane (any: the first hit ends
+// the traversal, as trav_leaf<true>).
 template <bool INST>
 SRT_D bool trav_pend_any(const DevScene& S, TravState& st, const TravStack& k, bool any) {
     uint32_t nt = 0;
@@ -2232,7 +2229,8 @@ __global__ void __launch_bounds__(256) k_denoise_guide(const float4* in, float4*
     g[i] = make_float4(pt_logf(1.0f + c.x), pt_logf(1.0f + c.y), pt_logf(1.0f + c.z), 0.0f);
 }
 
-// exp(x) for x <= 0 or NaN: pt_expf's operations without its branches (the
+// exp(x) for x <= 0 or NaN: pt_expf's operations (reduction by k ln 2 in two
+// parts, Taylor polynomial of degree 8) without its branches (the
 // range ends become selects; k >= -150, so one of pt_expf's two exponent
 // folds remains), which lets the taps' chains overlap.
 SRT_D float exp_neg(float x) {
