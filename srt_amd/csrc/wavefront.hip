@@ -574,16 +574,19 @@ struct IdentityEntry {
 // share holding run 32 r + (p + a mixed turn of r) mod 32 of every round r (the
 // turns keep a piece from meeting the same image columns in every round when
 // the width is a power of two: without them Cornell 256x256x16 took 0.56 ms
-// instead of 0.40).  What does not fill a round keeps its place.  Runs of 256
-// slots (4 tiles) keep neighbouring tiles together in this and the next queues;
-// frames too small for 16 runs a piece take shorter ones.
+// instead of 0.40).  What does not fill a round keeps its place.  Runs of 512
+// slots (8 tiles) keep neighbouring tiles together in this and the next queues;
+// frames that k_paths takes whole keep no queues and do best with 256, frames too
+// small for 16 such runs a piece with less.
 // In us, in slot order / dealt in runs of 64, 256, 512, 2048, 2^15: tube 1280x720x16
 // 3186 / 2933 2888 2872 2887 3246, 1M triangles 1280x720x1 1574 / 1499 1501 1514
 // 1566 1592, MLP training frame 256x256x8 624 / 571 573 587 582 626, Cornell 512x512x8
 // 618 / 574 578 580 596 608, 1900x1000x8 1809 / 1758 1702 1720 1732 1715.  A frame
 // whose two halves cost the same has no need of it at 16 samples, where a piece is
 // half a plane: Cornell 256x256x16 371 / 388 389 397 398 373, 512x512x16 872 / 889 880
-// 880 904 919.  Chunks of 32 sample planes or more, whose pieces are whole planes,
+// 880 904 919.  256 against 512 above 2^20 paths, with the MLP: Cornell 700x500x6 349 / 342,
+// 700x500x5 317 / 308, 500x400x12 396 / 403; below: Cornell 1000x1000x1 354 / 360,
+// 512x512x3 304 / 315, tube 640x360x4 678 / 695.  Chunks of 32 sample planes or more, whose pieces are whole planes,
 // would lose their order for nothing: 1920x1080x64 59.3 ms, 60.9 in runs of 512.
 struct CamView {
     uint32_t per, shift;      // runs per piece
@@ -599,7 +602,8 @@ struct CamView {
 SRT_D CamView cam_view(uint32_t n, int deal) {
     n = __builtin_amdgcn_readfirstlane(n);
     CamView v;
-    v.shift = n >= (uint32_t)kParts * 16u * 256u ? 8u : (n >= (uint32_t)kParts * 16u * 64u ? 6u : 0u);
+    v.shift = n > (uint32_t)kWholePaths ? 9u
+                                        : (n >= (uint32_t)kParts * 16u * 512u ? 8u : (n >= (uint32_t)kParts * 16u * 64u ? 6u : 0u));
     v.per = deal ? (n >> v.shift) / (uint32_t)kParts : 0u;
     return v;
 }

@@ -262,10 +262,11 @@ def test_whole_path_kernel_equals_queue_stages(ctx, name, W, H, spp, depth):
 
 
 @pytest.mark.parametrize("W,H,spp", [(8, 8, 1), (61, 37, 1), (160, 57, 1), (203, 101, 2), (301, 109, 4), (311, 170, 5),
-                                      (640, 411, 2), (97, 61, 40)])
+                                      (640, 411, 2), (641, 411, 4), (97, 61, 40)])
 def test_dealt_slots_cover_every_path(ctx, W, H, spp):
     """Chunks of fewer than 32 sample planes deal their slots to the queue's
-    pieces in runs of 1, 64 (from 2^15 paths) or 256 (from 2^17): every path is traced once whatever the
+    pieces in runs of 1, 64 (from 2^15 paths), 256 (from 2^18) or 512 (above
+    2^20): every path is traced once whatever the
     remainder (queue stages by visit counting), and the image is the whole-path
     kernel's and, for small frames, the oracle's."""
     s = scenes.cornell()
