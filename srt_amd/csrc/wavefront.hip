@@ -2574,7 +2574,8 @@ static int chunk_stages(srt_ctx* c, SceneRec* s, const Segment* segs_host, int n
     for (int k = 0; k < nseg; k++) tcfg.deal |= n < (int64_t)kParts * segs_host[k].wh ? 1 : 0;
     const int64_t whole_max = tcfg.wide && !c->count_visits ? c->whole_paths : 0;
     auto whole = [&](int depth) {
-        return depth == 0 ? whole_max : std::min(whole_max, whole_path_limit(max_depth - depth));
+        // (mode 1: the paths end at vertex 2, one launch instead of that bounce's three)
+        return depth == 0 || mlp_mode == 1 ? whole_max : std::min(whole_max, whole_path_limit(max_depth - depth));
     };
     int64_t npaths = n;                   // live paths of the bounce
     uint32_t* live = c->live;
