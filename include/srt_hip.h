@@ -122,7 +122,7 @@ const char* srt_last_error(const srt_ctx* ctx);
  * that deep traversals fill takes the same time, one whose camera rays visit few nodes 4 to 7 %
  * more), "whole_paths" (a chunk's paths are finished in one launch that holds each in registers
  * once at most this many live (after the first bounce at most 2^17 (k + 2) with k bounces left,
- * and 2^20), 0..2^31 - 1, default 2^20; 0: bounce by bounce to the end; the results are
+ * and 2^20, unless the paths end in MLP queries), 0..2^31 - 1, default 2^20; 0: bounce by bounce to the end; the results are
  * identical), "keep_build_scratch" (1, the default: the device scratch of a BVH build, and of a
  * denoise pass up to 512 MiB, stays allocated for the next one and counts in srt_hbm_used; it is
  * freed when an allocation would exceed the budget or fail; 0: freed now and at the end of every
